@@ -144,35 +144,46 @@ __device__ __forceinline__ void restrict_at(const Grid &gc, const Grid &gf, int 
 // phi_f += P phi_c for face component A in dimension D (stag_prolongation_2d/3d,
 // stag_mg_solver.f90:1370-1633): bilinear in the transverse directions,
 // linear along A.  The component is a template argument so every index is static.
-// The prolongation arithmetic of one fine point c of component A
-// (stag_prolongation_2d/3d, stag_mg_solver.f90:1370-1633): at(sa, s1, s2) is
-// the coarse value at Q + sa along A, + s1 along the first transverse
-// direction and + s2 along the second (s1, s2 in {0, o1 / o2}).
+// The prolongation arithmetic of one fine point (stag_prolongation_2d/3d,
+// stag_mg_solver.f90:1370-1633): at(sa, s1, s2) is the coarse value at the
+// point's coarse cell, shifted up along the component's direction (sa) and to
+// the nearer side across it (s1, s2); even: the point lies on a coarse face.
+template <typename T, int D, typename F>
+__device__ __forceinline__ T prolong_sum(T v, bool even, F &&at) {
+  if (D == 2) {
+    if (even) {
+      v = v + (T)0.75 * at(false, false, false) + (T)0.25 * at(false, true, false);
+    } else {
+      v = v + (T)0.375 * at(false, false, false) + (T)0.125 * at(false, true, false) +
+          (T)0.375 * at(true, false, false) + (T)0.125 * at(true, true, false);
+    }
+  } else {
+    const T nine16 = (T)0.5625, three16 = (T)0.1875, one16 = (T)0.0625;
+    const T nine32 = (T)0.28125, three32 = (T)0.09375, one32 = (T)0.03125;
+    if (even) {
+      v = v + nine16 * at(false, false, false) + three16 * at(false, true, false) +
+          three16 * at(false, false, true) + one16 * at(false, true, true);
+    } else {
+      v = v + nine32 * at(false, false, false) + three32 * at(false, true, false) +
+          three32 * at(false, false, true) + one32 * at(false, true, true) + nine32 * at(true, false, false) +
+          three32 * at(true, true, false) + three32 * at(true, false, true) + one32 * at(true, true, true);
+    }
+  }
+  return v;
+}
+
+// The same for point c of component A: at(sa, s1, s2) is the coarse value at
+// Q + sa along A, + s1 along the first transverse direction and + s2 along
+// the second (s1, s2 in {0, o1 / o2}).
 template <typename T, int D, int A, typename F>
 __device__ __forceinline__ T prolong_combine(const int c[3], T v, F &&at) {
   constexpr int T1 = (D == 2) ? 1 - A : (A == 0 ? 1 : 0);
   constexpr int T2 = (D == 2) ? -1 : (A == 2 ? 1 : 2);
   const int o1 = (c[T1] & 1) ? 1 : -1;
   const int o2 = (T2 >= 0 && (c[T2 >= 0 ? T2 : 0] & 1)) ? 1 : -1;
-  const bool even = (c[A] & 1) == 0;
-  if (D == 2) {
-    if (even) {
-      v = v + (T)0.75 * at(0, 0, 0) + (T)0.25 * at(0, o1, 0);
-    } else {
-      v = v + (T)0.375 * at(0, 0, 0) + (T)0.125 * at(0, o1, 0) + (T)0.375 * at(1, 0, 0) +
-          (T)0.125 * at(1, o1, 0);
-    }
-  } else {
-    const T nine16 = (T)0.5625, three16 = (T)0.1875, one16 = (T)0.0625;
-    const T nine32 = (T)0.28125, three32 = (T)0.09375, one32 = (T)0.03125;
-    if (even) {
-      v = v + nine16 * at(0, 0, 0) + three16 * at(0, o1, 0) + three16 * at(0, 0, o2) + one16 * at(0, o1, o2);
-    } else {
-      v = v + nine32 * at(0, 0, 0) + three32 * at(0, o1, 0) + three32 * at(0, 0, o2) + one32 * at(0, o1, o2) +
-          nine32 * at(1, 0, 0) + three32 * at(1, o1, 0) + three32 * at(1, 0, o2) + one32 * at(1, o1, o2);
-    }
-  }
-  return v;
+  return prolong_sum<T, D>(v, (c[A] & 1) == 0, [&](bool sa, bool s1, bool s2) -> T {
+    return at(sa ? 1 : 0, s1 ? o1 : 0, s2 ? o2 : 0);
+  });
 }
 
 template <typename T, int D, int A>
