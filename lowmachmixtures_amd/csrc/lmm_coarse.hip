@@ -60,7 +60,7 @@ __device__ void blk_stag_smooth_d(const SLevelDesc<T> &L, int visc, T omega, int
       const int a = (color - 1) / 2, par = (color + 1) % 2;
       if (a < alo || a >= ahi) continue;  // uniform over the workgroup
       for (long t = threadIdx.x; t < half; t += CTPB)
-        gs_colour_at<T>(L.g, visc, a, par, omega, dxsqinv, L.phi, L.K, L.rhs.c[a], t);
+        gs_colour_at<T>(L.g, DIM, visc, a, par, omega, dxsqinv, L.phi, L.K, L.rhs.c[a], t);
       __syncthreads();
     }
   }
@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(CTPB) k_stag_coarse_vcycle(SCoarseArgs<T> A) {
     blk_stag_smooth<T>(L, A.visc, A.omega, A.nd, alo, ahi);
     const T dxsqinv = (T)(1.0 / (L.g.dx * L.g.dx));
     for (int a = alo; a < ahi; a++)
-      for (long t = threadIdx.x; t < L.g.N; t += CTPB) residual_at<T>(L.g, A.visc, dxsqinv, L.phi, L.rhs, L.res, L.K, a, t);
+      for (long t = threadIdx.x; t < L.g.N; t += CTPB) residual_at<T>(L.g, dim, A.visc, dxsqinv, L.phi, L.rhs, L.res, L.K, a, t);
     __syncthreads();
     const SLevelDesc<T> &Cn = A.L[n + 1];
     for (int a = alo; a < ahi; a++)

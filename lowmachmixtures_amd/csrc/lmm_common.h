@@ -108,15 +108,28 @@ __device__ __forceinline__ long at_sh(const Grid &g, const Pt &p, int d1, int s1
   return at3(g, p, sh[0], sh[1], sh[2]);
 }
 
+// Calls f with the component, dimension and viscosity type as constants
+// (f(Const<A>)): with them the neighbour offsets and pointer tables of
+// stag_point fold away; with run-time values they are indexed in memory.
+template <int V>
+struct Const {
+  static constexpr int value = V;
+};
+template <int DIM, typename F>
+__device__ __forceinline__ void with_component(int a, F &&f) {
+  if (a == 0) f(Const<0>());
+  else if (a == 1 || DIM == 2) f(Const<1>());
+  else f(Const<DIM == 2 ? 1 : 2>());
+}
+
 // Staggered operator at one face point of component a, written term by term
 // in the order of stag_applyop_2d/3d (stag_applyop.f90:204-1067); fac is the
 // diagonal of stag_mg_update_2d/3d (stag_mg_solver.f90:1769-2463) in its own
 // order.  Lout = (theta*alpha - L)phi at the point.
 template <typename T>
-__device__ __forceinline__ void stag_point(int visc, const Grid &g, int a, const Pt &P,
+__device__ __forceinline__ void stag_point(int visc, int dim, const Grid &g, int a, const Pt &P,
                                            const T *const phi[3], const StagCoef<T> &K,
                                            T dxsqinv, T &Lout, T &fac) {
-  const int dim = g.dim;
   int t1, t2 = -1;
   if (dim == 2) {
     t1 = 1 - a;

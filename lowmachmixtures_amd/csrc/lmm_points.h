@@ -58,21 +58,21 @@ __device__ __forceinline__ void decode_half(const Grid &g, long t, int par, int 
 // colour read only points of other colours, so the in-place update equals
 // the reference's two passes (stag_mg_solver.f90:373-382).
 template <typename T>
-__device__ __forceinline__ void gs_colour_at(const Grid &g, int visc, int a, int par, T omega, T dxsqinv,
+__device__ __forceinline__ void gs_colour_at(const Grid &g, int dim, int visc, int a, int par, T omega, T dxsqinv,
                                              const Ptr3<T> &ph, const StagCoef<T> &K, const T *rhs, long t) {
   int i, j, k;
   decode_half(g, t, par, i, j, k);
   Pt P = make_pt(g, i, j, k);
   const T *phr[3] = {ph.c[0], ph.c[1], ph.c[2]};
   T L, fac;
-  stag_point<T>(visc, g, a, P, phr, K, dxsqinv, L, fac);
+  stag_point<T>(visc, dim, g, a, P, phr, K, dxsqinv, L, fac);
   long p = i + g.s[1] * j + g.s[2] * k;
   ph.c[a][p] = ph.c[a][p] + gs_div(omega * (rhs[p] - L), fac);
 }
 
 // res = rhs - L phi at point t of component a (stag_mg_solver.f90:404-416: -(Lphi - rhs))
 template <typename T>
-__device__ __forceinline__ void residual_at(const Grid &g, int visc, T dxsqinv, const Ptr3<T> &ph,
+__device__ __forceinline__ void residual_at(const Grid &g, int dim, int visc, T dxsqinv, const Ptr3<T> &ph,
                                             const Ptr3<T> &rh, const Ptr3<T> &res, const StagCoef<T> &K, int a,
                                             long t) {
   int i, j, k;
@@ -80,7 +80,7 @@ __device__ __forceinline__ void residual_at(const Grid &g, int visc, T dxsqinv, 
   Pt P = make_pt(g, i, j, k);
   const T *phr[3] = {ph.c[0], ph.c[1], ph.c[2]};
   T L, fac;
-  stag_point<T>(visc, g, a, P, phr, K, dxsqinv, L, fac);
+  stag_point<T>(visc, dim, g, a, P, phr, K, dxsqinv, L, fac);
   long p = i + g.s[1] * j + g.s[2] * k;
   res.c[a][p] = rh.c[a][p] - L;
 }
