@@ -214,12 +214,12 @@ void launch_stokes_dot(hipStream_t s, const Grid &g, const double *a, const doub
 // Finalize: op 0 -> out[0] = (s0 + s1 (+ s2)) + pnw2*s3
 //           op 1 -> out[0] = sqrt(sqrt(su)^2 + (pnw*sqrt(s3))^2), out[1] = sqrt(su), out[2] = pnw*sqrt(s3)
 //           op 2 -> out[0..3] = raw segment sums
-//           op 3 -> out[0] = s3 / total_volume (pressure mean)
-//           op 4 -> out[d] = face-sum_d / total_volume (velocity means)
-void launch_finalize(hipStream_t s, const Grid &g, const double *partial, double *out, int op,
-                     double pnw);
+// host (may be null): pinned host memory that receives the same values
+void launch_finalize(hipStream_t s, const Grid &g, const double *partial, double *out, int op, double pnw,
+                     double *host = nullptr);
 void launch_face_maxabs(hipStream_t s, const Grid &g, const double *const r[3], double *partial);
-void launch_finalize_max(hipStream_t s, const double *partial, double *out);
+// host[0..2] = the three maxima of launch_face_maxabs on g (pinned host memory)
+void launch_finalize_max(hipStream_t s, const Grid &g, const double *partial, double *host);
 template <typename T>
 void launch_sum_faces_weighted(hipStream_t s, const Grid &g, T *const u[3], double *partial);
 
@@ -227,6 +227,7 @@ void launch_sum_faces_weighted(hipStream_t s, const Grid &g, T *const u[3], doub
 void launch_bmax_neg(hipStream_t s, double *tmp, const double *b, long n);       // tmp = -(tmp - b)
 void launch_div_by(hipStream_t s, double *v, const double *src, long n, const double *scal);  // v = src / *scal
 void launch_axmy(hipStream_t s, double *w, const double *v, long n, const double *scal);     // w = w - v * *scal
+// x += sum_k y_k V_k; y: host values, at most 32
 void launch_update_sol(hipStream_t s, double *x, double *const V[], const double *y, int i, long n);
 // w -= h[0]*v, then the Stokes dot of the new w with vn (vn = nullptr: with
 // itself) into partial, bit-identical to launch_axmy + launch_stokes_dot
@@ -237,13 +238,13 @@ void launch_div_by_f32(hipStream_t s, double *v, float *v32, const double *src, 
 // values v0 .. v0+count-1 of the counter-based Gaussian stream (seed, step)
 // into out (lmm_rng.hip)
 void launch_fill_normal_philox(hipStream_t s, double *out, long count, long v0, uint64_t seed, uint64_t step);
-// x += sum_k y_k Z_k, Z in FP32 (at most 32 vectors)
+// x += sum_k y_k Z_k, Z in FP32 (at most 32 vectors); y: host values
 void launch_update_sol_z32(hipStream_t s, double *x, float *const Z[], const double *y, int i, long n);
 // Classical Gram-Schmidt passes of the flexible GMRES (1..CGS_MAXV basis
 // vectors per pass).  launch_cgs_dots: segment sums of <w, V_k> into
 // partial[blk*CGS_STRIDE + 4k + seg]; launch_cgs_finalize: d_k = <w, V_k>
 // (Stokes product, box-face weights, pressure weighted by pnw^2) and
-// c_k = sig2[k]*d_k; launch_cgs_update: vn = src - sum_k c_k V_k, its FP32
+// c_k = sig2[k]*d_k (d_k also into pinned host memory); launch_cgs_update: vn = src - sum_k c_k V_k, its FP32
 // copy (v32 may be null) and the segment sums of <vn, vn> for
 // launch_finalize.  Every level extent must be even (cell pairs).
 constexpr int CGS_MAXV = 8;
@@ -251,7 +252,7 @@ constexpr int CGS_STRIDE = 4 * CGS_MAXV;
 void launch_cgs_dots(hipStream_t s, const Grid &g, const double *w, const double *const V[], int nv,
                      double *partial);
 void launch_cgs_finalize(hipStream_t s, const Grid &g, const double *partial, int nv, const double *sig2,
-                         double pnw, double *d_out, double *c_out);
+                         double pnw, double *d_out, double *c_out, double *host);
 void launch_cgs_update(hipStream_t s, const Grid &g, const double *src, const double *const V[], int nv,
                        const double *c, double *vn, float *v32, double *partial);
 // r = b - A x in one pass (FP64, 3D visc_type -1 / 1); false when not available
@@ -261,10 +262,15 @@ bool launch_apply_matrix_resid(hipStream_t s, const Grid &g, int visc, double *c
 // FP64 A x of an FP32 x (3D visc_type -1 / 1); false when not available
 bool launch_apply_matrix_x32(hipStream_t s, const Grid &g, int visc, float *const x_u[3], const float *x_p,
                              double *const b_u[3], double *b_p, const StagCoef<double> &K);
+// Means subtracted: x_c -= (sum over b < nparts of src[b*stride + c]) / cells
+// for c < nc, and x -= its mean from k_precon_final's nsrc partial sums (work:
+// RED_BLOCKS doubles).
 template <typename T>
-void launch_sub_scalar(hipStream_t s, T *x, long n, const double *scal);
+void launch_sub_means(hipStream_t s, const Grid &g, T *const x[3], int nc, const double *src, int nparts, int stride);
 template <typename T>
-void launch_sub_scalar3(hipStream_t s, const Grid &g, T *const u[3], const double *scal);
+void launch_sub_cell_mean(hipStream_t s, const Grid &g, T *x, const double *src, int nsrc, double *work);
+// workgroups (and partial rows) of the reductions over the cells of g
+inline int red_blocks(const Grid &g) { return g.N < 256L * RED_BLOCKS ? (int)((g.N + 255) / 256) : RED_BLOCKS; }
 
 // ---- inertial time step (lmm_inertial.hip) ----
 struct AdvArgs {

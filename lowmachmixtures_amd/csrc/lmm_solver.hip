@@ -25,10 +25,6 @@
 
 using namespace lmm;
 
-namespace lmm {
-void launch_fold_cells(hipStream_t s, const double *src, int nsrc, double *partial);
-}
-
 // ---------------------------------------------------------------------------
 // context and fields
 // ---------------------------------------------------------------------------
@@ -575,8 +571,7 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
 static void resid_inf(lmm_ctx *c, SLevel<double> &L, double *const phi[3], double *const rhs[3], double out[3]) {
   launch_stag_residual<double>(c->stream, L.g, c->prm.visc_type, phi, rhs, L.res, L.K());
   launch_face_maxabs(c->stream, L.g, L.res, c->partial);
-  launch_finalize_max(c->stream, c->partial, c->scal + 4000);
-  hipMemcpyAsync(c->hscal, c->scal + 4000, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  launch_finalize_max(c->stream, L.g, c->partial, c->hscal);
   hipStreamSynchronize(c->stream);
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
 }
@@ -584,8 +579,7 @@ static void resid_inf(lmm_ctx *c, SLevel<double> &L, double *const phi[3], doubl
 // max |rhs| per component on level 0 (FP64), synchronises
 static void rhs_inf(lmm_ctx *c, SLevel<double> &L, double *const rhs[3], double out[3]) {
   launch_face_maxabs(c->stream, L.g, rhs, c->partial);
-  launch_finalize_max(c->stream, c->partial, c->scal + 4000);
-  hipMemcpyAsync(c->hscal, c->scal + 4000, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  launch_finalize_max(c->stream, L.g, c->partial, c->hscal);
   hipStreamSynchronize(c->stream);
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
 }
@@ -740,8 +734,7 @@ static double cell_inf(lmm_ctx *c, const Grid &g, const double *a) {
   g1.dim = 1;  // the face reduction over one array
   const double *r[3] = {a, nullptr, nullptr};
   launch_face_maxabs(c->stream, g1, r, c->partial);
-  launch_finalize_max(c->stream, c->partial, c->scal + 4030);
-  hipMemcpyAsync(c->hscal, c->scal + 4030, sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  launch_finalize_max(c->stream, g1, c->partial, c->hscal);
   hipStreamSynchronize(c->stream);
   return c->hscal[0];
 }
@@ -982,15 +975,11 @@ static void apply_precon_t(lmm_ctx *c, std::vector<SLevel<T>> &S, std::vector<CL
   int nb = (int)((g.N + 255) / 256);
   launch_precon_final<T>(s, g, c->prm.visc_type, xu, xp, phi, mac_rhs, ainv, beta, gamma, theta_alpha,
                          c->partial2);
-  launch_fold_cells(s, c->partial2, nb, c->partial);
-  launch_finalize(s, g, c->partial, c->scal + 4010, 3, 1.0);
-  // the pressure mean (and velocity means when theta_alpha = 0) are
-  // accumulated and subtracted in FP64 also for FP32 fields
-  launch_sub_scalar<T>(s, xp, g.N, c->scal + 4010);
+  // the pressure mean (and velocity means when theta_alpha = 0)
+  launch_sub_cell_mean<T>(s, g, xp, c->partial2, nb, c->partial);
   if (theta_alpha == 0.0) {
     launch_sum_faces_weighted<T>(s, g, xu, c->partial);
-    launch_finalize(s, g, c->partial, c->scal + 4020, 4, 1.0);
-    launch_sub_scalar3<T>(s, g, xu, c->scal + 4020);
+    launch_sub_means<T>(s, g, xu, dim, c->partial, red_blocks(g), 4);
   }
 }
 
@@ -1000,11 +989,16 @@ static void precon64(lmm_ctx *c, const SV &b, const SV &x, double theta_alpha) {
 
 // ------------------------- reductions to host ----------------------------
 
-// dot / norm of Stokes vectors; result in device slot, optional host copy
+// The pinned host mirror of a device scalar slot: the reductions write both,
+// so the host reads a result after a stream synchronisation without a copy
+// (fetch).
+static double *mirror(lmm_ctx *c, const double *slot) { return c->hscal + (slot - c->scal); }
+
+// dot / norm of Stokes vectors; result in a device slot and its host mirror
 static void stokes_dot_dev(lmm_ctx *c, const double *a, const double *b, double *slot, int op) {
   ProfScope ps(c, "krylov", (double)c->g.N * 8.0 * 2 * (c->g.dim + 1));
   launch_stokes_dot(c->stream, c->g, a, b, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, slot, op, c->prm.p_norm_weight);
+  launch_finalize(c->stream, c->g, c->partial, slot, op, c->prm.p_norm_weight, mirror(c, slot));
 }
 
 // Modified Gram-Schmidt of w against V_0..V_{i-1} (gmres.f90:338-358): the
@@ -1030,14 +1024,15 @@ static void mgs(lmm_ctx *c, const VF &Vk, int i, double *H, double *nrm) {
     const bool last = (k == i);
     ProfScope ps(c, "krylov", (double)L * 8.0 * (last ? 3 : 4));
     launch_axmy_dot(s, c->g, c->w, Vk(k - 1), H + k - 1, last ? nullptr : Vk(k), c->partial);
-    launch_finalize(s, c->g, c->partial, last ? nrm : H + k, last ? 1 : 0, c->prm.p_norm_weight);
+    double *slot = last ? nrm : H + k;
+    launch_finalize(s, c->g, c->partial, slot, last ? 1 : 0, c->prm.p_norm_weight, mirror(c, slot));
   }
 }
 
+// n results from device slot dev on, from their host mirror
 static void fetch(lmm_ctx *c, const double *dev, int n, double *host) {
-  hipMemcpyAsync(c->hscal, dev, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream);
   hipStreamSynchronize(c->stream);
-  memcpy(host, c->hscal, sizeof(double) * n);
+  memcpy(host, mirror(c, dev), sizeof(double) * n);
 }
 
 // ------------------------- GMRES host scalars (gmres.f90:517-605) --------
@@ -1207,11 +1202,11 @@ static int gmres_ref(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
       apply_matrix_dev(c, vi, tmp);
       precon64(c, tmp, w, theta_alpha);
       // H(1..i, i), then H(i+1,i) = |w|
+      // (|w| goes to its entry of the column; its two parts land in entries
+      // that nothing has written yet, below it or in the next column)
       double *col = dH + (long)(m + 1) * (i - 1);
-      double *sl = c->scal + 3100;
-      mgs(c, Vk, i, col, sl);
-      hipMemcpyAsync(col + i, sl, sizeof(double), hipMemcpyDeviceToDevice, s);
-      launch_div_by(s, Vk(i), c->w, L, sl);
+      mgs(c, Vk, i, col, col + i);
+      launch_div_by(s, Vk(i), c->w, L, col + i);
       fetch(c, dH + (long)(m + 1) * (i - 1), i + 1, &hs.h(1, i));
       if (hs.h(i + 1, i) == 0.0) {
         brk = true;
@@ -1231,12 +1226,9 @@ static int gmres_ref(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
       return set_err(c, LMM_ERR_BREAKDOWN, "gmres: error in orthogonalization");
     }
     hs.solve(i_copy - 1);
-    memcpy(c->hscal, hs.y.data(), sizeof(double) * i_copy);
-    hipMemcpyAsync(c->scal + 3200, c->hscal, sizeof(double) * i_copy, hipMemcpyHostToDevice, s);
     std::vector<double *> vl(i_copy);
     for (int k = 0; k < i_copy; k++) vl[k] = Vk(k);
-    launch_update_sol(s, c->x, vl.data(), c->scal + 3200, i_copy, L);
-    hipStreamSynchronize(s);  // hscal reused
+    launch_update_sol(s, c->x, vl.data(), hs.y.data(), i_copy, L);
   }
   info->total_iter = total_iter;
   info->outer_iter = iter;
@@ -1326,7 +1318,8 @@ static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, 
     for (int k = 0; k < nv; k++) vl[k] = Vk(k0 + k);
     ProfScope ps(c, "krylov", (double)L * 8.0 * (nv + 1));
     launch_cgs_dots(s, g, c->w, vl, nv, c->partial_cgs);
-    launch_cgs_finalize(s, g, c->partial_cgs, nv, sig2.data() + k0, c->prm.p_norm_weight, dslot + k0, cslot + k0);
+    launch_cgs_finalize(s, g, c->partial_cgs, nv, sig2.data() + k0, c->prm.p_norm_weight, dslot + k0, cslot + k0,
+                        mirror(c, dslot + k0));
   }
   for (int k0 = 0; k0 < i; k0 += CGS_MAXV) {
     const int nv = std::min(CGS_MAXV, i - k0);
@@ -1336,7 +1329,7 @@ static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, 
     ProfScope ps(c, "krylov", (double)L * (8.0 * (nv + 2) + (last ? 4.0 : 0.0)));
     launch_cgs_update(s, g, (k0 == 0) ? c->w : Vk(i), vl, nv, cslot + k0, Vk(i), last ? c->b32 : nullptr, c->partial);
   }
-  launch_finalize(s, g, c->partial, nslot, 1, c->prm.p_norm_weight);
+  launch_finalize(s, g, c->partial, nslot, 1, c->prm.p_norm_weight, mirror(c, nslot));
   double hb[3 * 32 + 3];
   fetch(c, dslot, 83, hb);
   for (int k = 0; k < i; k++) hs.h(k + 1, i) = sig[i - 1] * sig[k] * hb[k];
@@ -1409,10 +1402,8 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
           cgs_step(c, Vk, i, sig, hs);  // writes V(i) and its FP32 copy
           b32_fresh = true;
         } else {
-          double *col = dH + (long)(m + 1) * (i - 1);
-          double *sl = c->scal + 3100;
+          double *col = dH + (long)(m + 1) * (i - 1), *sl = col + i;
           mgs(c, Vk, i, col, sl);
-          hipMemcpyAsync(col + i, sl, sizeof(double), hipMemcpyDeviceToDevice, s);
           if (c->fused_krylov) launch_div_by_f32(s, Vk(i), c->b32, c->w, L, sl);
           else launch_div_by(s, Vk(i), c->w, L, sl);
           b32_fresh = c->fused_krylov;
@@ -1437,21 +1428,18 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
     hs.solve(used - 1);
     // x += sum_k y_k z_k with z_k = sig_k Z_k  (Z in FP32, accumulation in FP64)
     for (int k = 0; k < used; k++) hs.y[k] *= sig[k];
-    memcpy(c->hscal, hs.y.data(), sizeof(double) * used);
-    hipMemcpyAsync(c->scal + 3200, c->hscal, sizeof(double) * used, hipMemcpyHostToDevice, s);
     if (c->z32_direct) {
       std::vector<float *> zl(used);
       for (int k = 0; k < used; k++) zl[k] = Zk(k);
       ProfScope ps(c, "krylov", (double)L * (16.0 + 4.0 * used));
-      launch_update_sol_z32(s, c->x, zl.data(), c->scal + 3200, used, L);
+      launch_update_sol_z32(s, c->x, zl.data(), hs.y.data(), used, L);
     } else {
       for (int k = 0; k < used; k++) {
         launch_convert<double, float>(s, c->r, Zk(k), L);
         double *one = c->r;
-        launch_update_sol(s, c->x, &one, c->scal + 3200 + k, 1, L);
+        launch_update_sol(s, c->x, &one, hs.y.data() + k, 1, L);
       }
     }
-    hipStreamSynchronize(s);
   }
   info->total_iter = total_iter;
   info->outer_iter = iter;
@@ -1642,7 +1630,7 @@ int lmm_ctx_create(int dim, const int n_cells[3], double dx, const lmm_params *p
   c->partial_cgs = dalloc<double>(c->stream, (long)RED_BLOCKS * CGS_STRIDE);
   c->partial2 = dalloc<double>(c->stream, (N + 255) / 256 + 1);
   c->scal = dalloc<double>(c->stream, 8192);
-  if (hipHostMalloc((void **)&c->hscal, 8192 * sizeof(double), hipHostMallocDefault) != hipSuccess) c->hscal = nullptr;
+  if (hipHostMalloc((void **)&c->hscal, 8192 * sizeof(double), hipHostMallocCoherent) != hipSuccess) c->hscal = nullptr;
   for (int d = 0; d < dim; d++) {
     c->ainv[d] = dalloc<double>(c->stream, N);
   }
@@ -2285,7 +2273,7 @@ int lmm_stag_inner_prod(lmm_ctx *c, lmm_field *const m1[3], lmm_field *const m2[
   launch_fill<double>(c->stream, c->r + dim * N, N, 0.0);
   launch_fill<double>(c->stream, c->w + dim * N, N, 0.0);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0);
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
   double h[4];
   fetch(c, c->scal + 4100, 4, h);
   for (int d = 0; d < 3; d++) prod_val[d] = d < dim ? h[d] : 0.0;
@@ -2301,7 +2289,7 @@ int lmm_cc_inner_prod(lmm_ctx *c, lmm_field *m1, lmm_field *m2, double *prod_val
   hipMemcpyAsync(c->r + dim * N, m1->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   hipMemcpyAsync(c->w + dim * N, m2->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0);
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
   double h[4];
   fetch(c, c->scal + 4100, 4, h);
   *prod_val = h[3];
@@ -3869,7 +3857,7 @@ int lmm_cnn_error_reduction(lmm_cnn *nn, lmm_field *const alpha_fc[3], lmm_field
   lmm_cnn *saved = c->cnn;
   c->cnn = nn;
   double sp = 0.0, sl = 0.0;
-  double *slot = c->scal + 4300;
+  double *slot = mirror(c, c->scal + 4300);  // the sums go straight to the host mirror
   // |phi* - z| / |phi*| over velocity and pressure (both mean-free in pressure)
   auto err2 = [&](double *out) {
     for (int d = 0; d < 3; d++) launch_sub_f32(s, du[d], ps.u[d], z.u[d], N);
@@ -3883,7 +3871,7 @@ int lmm_cnn_error_reduction(lmm_cnn *nn, lmm_field *const alpha_fc[3], lmm_field
     learned_stage(c, b.u, b.p, z.u, z.p);
     err2(slot + 4);
     double h[6];
-    fetch(c, slot, 6, h);
+    fetch(c, c->scal + 4300, 6, h);
     const double n0 = h[0] + h[1];
     sp += std::sqrt((h[2] + h[3]) / n0);
     sl += std::sqrt((h[4] + h[5]) / n0);
