@@ -26,6 +26,9 @@ struct Tuning {
   int rb_target = 768;  // workgroups the z-slab choice aims for (FP32; FP64 twice)
   int am_dz = 32;       // z depth of the operator's brick order (0: row order)
   int rb_prefetch = 0;  // FP32 fused sweep: load the next plane's coefficients one step ahead
+  // 3D levels up to this many cells sweep in bricks, and every one whose
+  // extents the marching tiles do not divide; 0: none do; -1: the measured rule
+  long rb_brick = -1;
   int rb_pairs = 2;     // FP32 three-component sweep: point pairs per thread (2: 64 x 16 tiles)
   int prolong_tiled = 1;  // 3D staggered prolongation from coarse values staged in LDS
   int coarse_split = 1;   // coarse staggered V-cycle: one workgroup per component (visc_type -1 / 1)

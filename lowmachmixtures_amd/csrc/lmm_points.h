@@ -279,6 +279,8 @@ __device__ __forceinline__ void cc_prolong_add_at(const Grid &gf, const Grid &gc
 }
 
 __device__ __forceinline__ int wrapc(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+// the same for an index any distance above the range (tiles wider than it)
+__device__ __forceinline__ int wrap_any(int i, int n) { return i < 0 ? i + n : (i >= n ? i % n : i); }
 
 // Two consecutive elements a[p], a[p+1] with one vector load (p even, so the
 // pair is aligned to its size).
@@ -311,8 +313,8 @@ __device__ __forceinline__ void st2(T *a, long p, T x0, T x1) {
 // its six neighbours in the same array (update), with the kernel's scalar
 // arguments in Args.
 
-// Component A of the staggered operator, visc_type -1, 1, 2 or 3.  The
-// terms are those of stag_applyop_3d (off-diagonal sum) and
+// Component A of the staggered operator, every visc_type (-2 and -3 by load
+// and update only).  The terms are those of stag_applyop_3d (off-diagonal sum) and
 // stag_mg_update_3d, in their order.  visc_type 2 and 3 couple the
 // components: the point reads the other two components (e1, e2 then hold
 // the arrays of t1 and t2, in the state the colour order gives them: already
@@ -320,14 +322,18 @@ __device__ __forceinline__ void st2(T *a, long p, T x0, T x1) {
 // beta[0], gamma[0] (the tile corner).
 template <typename T, int A, int VISC>
 struct StagRB {
+  static constexpr bool BRICK_ONLY = VISC < -1;  // the plane-marching forms are not built for it
+  static constexpr bool CROSS = VISC >= 2;
   struct Args {
     T omega, dxsqinv;
     const T *rhs, *alpha, *beta, *e1, *e2;
-    const T *gamma;  // visc_type 3
+    const T *gamma;    // visc_type 3, -3
+    const T *o1, *o2;  // visc_type -2, -3: the components of t1 and t2
   };
   struct Coef {
     T av, rhs, B0, B1, E10, E11, E20, E21;
-    T G[8];  // visc_type 2: the eight cross-term values; 3: their sum in G[0]
+    T G[8];  // |visc_type| 2, -3: the eight cross-term values; 3: their sum in G[0]
+    T G0, Gm;  // visc_type -3
   };
   // the array pointers in a fixed order, and back (the kernels receive them
   // as separate __restrict__ parameters)
@@ -353,7 +359,7 @@ struct StagRB {
     const long p = i + sy * j + sz * k;
     c.av = a.alpha[p];
     c.rhs = a.rhs[p];
-    if (VISC == -1) {
+    if (VISC < 0) {
       // along a = A; t1, t2 = the other two directions in increasing order
       const int im = (A == 0) ? wrapc(i - 1, g.n[0]) : i;
       const int jm = (A == 1) ? wrapc(j - 1, g.n[1]) : j;
@@ -367,6 +373,25 @@ struct StagRB {
       c.E11 = a.e1[p1];
       c.E20 = a.e2[p];
       c.E21 = a.e2[p2];
+      if (VISC < -1) {
+        // the cross terms at +t1, the point, -A +t1, -A, and the same for t2
+        const long pm = im + sy * jm + sz * km;
+        const int ip = wrapc(i + 1, g.n[0]), jp = wrapc(j + 1, g.n[1]), kp = wrapc(k + 1, g.n[2]);
+        const long q1 = (A == 0) ? im + sy * jp + sz * k : (A == 1 ? ip + sy * jm + sz * k : ip + sy * j + sz * km);
+        const long q2 = (A == 0) ? im + sy * j + sz * kp : (A == 1 ? i + sy * jm + sz * kp : i + sy * jp + sz * km);
+        c.G[0] = a.o1[p1];
+        c.G[1] = a.o1[p];
+        c.G[2] = a.o1[q1];
+        c.G[3] = a.o1[pm];
+        c.G[4] = a.o2[p2];
+        c.G[5] = a.o2[p];
+        c.G[6] = a.o2[q2];
+        c.G[7] = a.o2[pm];
+        if (VISC == -3) {
+          c.G0 = a.gamma[p];
+          c.Gm = a.gamma[pm];
+        }
+      }
     } else if (VISC >= 2) {
       c.B0 = a.beta[0];
       c.B1 = (VISC == 3) ? a.gamma[0] : (T)0;
@@ -417,7 +442,7 @@ struct StagRB {
   // vector load per array where the two points' values are adjacent.
   static __device__ __forceinline__ void load_pair(const Grid &g, int i, int j, int k, const Args &a, Coef &c0,
                                                    Coef &c1) {
-    if (VISC >= 2) {
+    if (VISC >= 2 || VISC < -1) {
       c0 = load(g, i, j, k, a);
       c1 = load(g, i + 1, j, k, a);
       return;
@@ -530,8 +555,25 @@ struct StagRB {
       const T F1m = (A == 0) ? ym : xm;
       const T F2p = (A == 2) ? yp : zp;
       const T F2m = (A == 2) ? ym : zm;
-      T dg = c.B0 + c.B1 + c.E10 + c.E11 + c.E20 + c.E21;
-      T off = Fa * c.B0 + Fma * c.B1 + F1p * c.E11 + F1m * c.E10 + F2p * c.E21 + F2m * c.E20;
+      const T fourthirds = (T)(4.0 / 3.0), twothirds = (T)(2.0 / 3.0);
+      T dg, off;
+      if (VISC == -1) {
+        dg = c.B0 + c.B1 + c.E10 + c.E11 + c.E20 + c.E21;
+        off = Fa * c.B0 + Fma * c.B1 + F1p * c.E11 + F1m * c.E10 + F2p * c.E21 + F2m * c.E20;
+      } else if (VISC == -2) {
+        dg = (T)2.0 * c.B0 + (T)2.0 * c.B1 + c.E10 + c.E11 + c.E20 + c.E21;
+        off = (T)2.0 * Fa * c.B0 + (T)2.0 * Fma * c.B1 + F1p * c.E11 + F1m * c.E10 + F2p * c.E21 + F2m * c.E20 +
+              c.G[0] * c.E11 - c.G[1] * c.E10 - c.G[2] * c.E11 + c.G[3] * c.E10 + c.G[4] * c.E21 - c.G[5] * c.E20 -
+              c.G[6] * c.E21 + c.G[7] * c.E20;
+      } else {
+        dg = fourthirds * c.B0 + c.G0 + fourthirds * c.B1 + c.Gm + c.E10 + c.E11 + c.E20 + c.E21;
+        off = Fa * (fourthirds * c.B0 + c.G0) + Fma * (fourthirds * c.B1 + c.Gm) + F1p * c.E11 + F1m * c.E10 +
+              F2p * c.E21 + F2m * c.E20 + c.G[0] * (c.E11 - twothirds * c.B0 + c.G0) -
+              c.G[1] * (c.E10 - twothirds * c.B0 + c.G0) - c.G[2] * (c.E11 - twothirds * c.B1 + c.Gm) +
+              c.G[3] * (c.E10 - twothirds * c.B1 + c.Gm) + c.G[4] * (c.E21 - twothirds * c.B0 + c.G0) -
+              c.G[5] * (c.E20 - twothirds * c.B0 + c.G0) - c.G[6] * (c.E21 - twothirds * c.B1 + c.Gm) +
+              c.G[7] * (c.E20 - twothirds * c.B1 + c.Gm);
+      }
       T fac = c.av + dg * dxsqinv;
       T L = F * fac - off * dxsqinv;
       return F + gs_div(omega * (c.rhs - L), fac);
@@ -543,6 +585,7 @@ struct StagRB {
 // arithmetic of cc_apply / the red-black update of lmm_points.h.
 template <typename T>
 struct CCRB {
+  static constexpr bool BRICK_ONLY = false, CROSS = false;
   struct Args {
     T inv;
     const T *rhs, *ax, *ay, *az;

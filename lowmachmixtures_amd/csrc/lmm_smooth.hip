@@ -46,6 +46,7 @@ constexpr int FX2 = 32, FY2 = 16;       // narrow tile of the three-component sw
 const char kFusedName[] = "k_rb_fused";
 const char kBlockName[] = "k_rb_block";
 const char kMarchName[] = "k_rb_march2";
+const char kBrickName[] = "k_rb_brick";
 const char kMarch3Name[] = "k_rb_march2x3";
 const char kResidRestrictName[] = "k_resid_restrict";
 
@@ -518,42 +519,208 @@ __global__ void __launch_bounds__(256) k_rb_block(Grid g, int nbx, int nby, int 
   }
 }
 
-// tx: the march's tile width (64, or 32 with 32 x 16 tiles)
+// Brick form of the same sweep for small levels and for extents that the
+// plane-marching tiles do not divide: a workgroup owns a 32 x KY x 4 brick,
+// KY / 4 x-pairs a thread.  Everything the brick reads from memory -- the old
+// field with a 2-point halo, the coefficients of the thread's pair and of its
+// red points of the 1-point ring -- is loaded at once, then the red and the
+// black points are updated in LDS.  A launch therefore waits for memory once,
+// where the marching form waits three times before its first plane and once
+// per plane, which is all the time of a level that fills the GPU only once.
+// The ring is computed again by the neighbours (1.7 updates per point at KY =
+// 4, 1.5 at 8), so the marching form, which streams, wins on large levels
+// (brick_level has both sides).
+// Bricks may hang over the box: points beyond it are loaded from their
+// periodic images and not stored.
+constexpr int KX = 32, KZ = 4;
+constexpr int KLX = KX + 4, KLZ = KZ + 4;
+constexpr int KRX = KX + 2, KRZ = KZ + 2;
+
+template <typename T, typename P, int KY>
+__device__ __forceinline__ void brick_tile(const Grid &g, int nbx, int nby, int b, const T *__restrict__ pin,
+                                           T *__restrict__ pout, const typename P::Args &args,
+                                           T (*sp)[KY + 4][KLX]) {
+  using Coef = typename P::Coef;
+  constexpr int KLY = KY + 4, KRY = KY + 2, NP = KX / 2 * KY * KZ / 256;  // pairs a thread
+  // red points of the ring: two end planes, two end rows of the inner planes,
+  // one end point of each inner row
+  constexpr int KRING = 2 * KRY * (KRX / 2) + 2 * KZ * (KRX / 2) + KZ * KY;
+  constexpr int KNR = (KRING + 255) / 256;
+  const int bx = b % nbx, by = (b / nbx) % nby, bz = b / (nbx * nby);
+  const int i0 = bx * KX, j0 = by * KY, k0 = bz * KZ;
+  const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
+  const long sy = g.s[1], sz = g.s[2];
+  const int tid = threadIdx.x;
+  constexpr int NPT = KLX * KLY * KLZ, NLD = (NPT + 255) / 256;
+  T old[NLD];
+#pragma unroll
+  for (int n = 0; n < NLD; n++) {
+    const int q = (NPT % 256 == 0 || tid + 256 * n < NPT) ? tid + 256 * n : NPT - 1;
+    const int x = q % KLX, y = (q / KLX) % KLY, z = q / (KLX * KLY);
+    // a null input stands for a field of zeros (the first sweep from a zero guess)
+    old[n] = pin ? pin[wrap_any(i0 - 2 + x, nx) + sy * wrap_any(j0 - 2 + y, ny) + sz * wrap_any(k0 - 2 + z, nz)] : (T)0;
+  }
+  const int m = tid % (KX / 2), i = i0 + 2 * m;
+  auto row = [&](int n) { return ((tid + 256 * n) / (KX / 2)) % KY; };
+  auto plane = [&](int n) { return (tid + 256 * n) / (KX / 2 * KY); };
+  Coef c0[NP], c1[NP], cr[KNR];
+#pragma unroll
+  for (int n = 0; n < NP; n++)
+    P::load_pair(g, wrap_any(i, nx), wrap_any(j0 + row(n), ny), wrap_any(k0 + plane(n), nz), args, c0[n], c1[n]);
+  int ring[KNR];
+#pragma unroll
+  for (int n = 0; n < KNR; n++) {
+    const int h = tid + 256 * n;
+    int rz, ry, rx;
+    if (h < 2 * KRY * (KRX / 2)) {
+      rz = (h < KRY * (KRX / 2)) ? 0 : KRZ - 1;
+      const int hh = h % (KRY * (KRX / 2));
+      ry = hh / (KRX / 2);
+      rx = 2 * (hh % (KRX / 2));
+    } else if (h < 2 * KRY * (KRX / 2) + 2 * KZ * (KRX / 2)) {
+      const int hh = h - 2 * KRY * (KRX / 2);
+      rz = 1 + hh / KRX;
+      const int rem = hh % KRX;
+      ry = (rem < KRX / 2) ? 0 : KRY - 1;
+      rx = 2 * (rem % (KRX / 2));
+    } else {
+      const int hh = (h - 2 * KRY * (KRX / 2) - 2 * KZ * (KRX / 2)) % (KZ * KY);
+      rz = 1 + hh / KY;
+      ry = 1 + hh % KY;
+      rx = 0;
+    }
+    const int jr = j0 - 1 + ry, kr = k0 - 1 + rz;
+    const int par = (jr + kr + 1) & 1;  // red: i + j + k even, i = i0 - 1 + rx
+    if (ry >= 1 && ry <= KY && rz >= 1 && rz <= KZ) rx = par ? KRX - 1 : 0;  // the red end of an inner row
+    else rx += par;
+    ring[n] = h < KRING ? (rx + 1) + KLX * ((ry + 1) + KLY * (rz + 1)) : -1;
+    if (h < KRING)
+      cr[n] = P::load(g, wrap_any(i0 - 1 + rx, nx), wrap_any(jr, ny), wrap_any(kr, nz), args);
+  }
+  T *const f = &sp[0][0][0];
+#pragma unroll
+  for (int n = 0; n < NLD; n++)
+    if (NPT % 256 == 0 || tid + 256 * n < NPT) f[tid + 256 * n] = old[n];
+  __syncthreads();
+  auto update = [&](int q, const Coef &c) -> T {
+    return P::update(c, f[q], f[q + 1], f[q - 1], f[q + KLX], f[q - KLX], f[q + KLX * KLY], f[q - KLX * KLY], args);
+  };
+  // red, in place: red points read black neighbours only
+  T vr[NP];
+  auto first_red = [&](int n) { return ((j0 + row(n) + k0 + plane(n)) & 1) == 0; };  // the pair's first point is red
+  auto at = [&](int n) { return (2 * m + 2) + KLX * ((row(n) + 2) + KLY * (plane(n) + 2)); };
+#pragma unroll
+  for (int n = 0; n < NP; n++) {
+    const int q = at(n) + (first_red(n) ? 0 : 1);
+    vr[n] = update(q, first_red(n) ? c0[n] : c1[n]);
+    f[q] = vr[n];
+  }
+#pragma unroll
+  for (int n = 0; n < KNR; n++)
+    if (ring[n] >= 0) f[ring[n]] = update(ring[n], cr[n]);
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < NP; n++) {
+    const int j = j0 + row(n), k = k0 + plane(n);
+    if (i >= nx || j >= ny || k >= nz) continue;
+    const bool fr = first_red(n);
+    const T vb = update(at(n) + (fr ? 1 : 0), fr ? c1[n] : c0[n]);
+    st2(pout, i + sy * j + sz * k, fr ? vr[n] : vb, fr ? vb : vr[n]);
+  }
+}
+
+template <typename T, typename P, int KY>
+__global__ void __launch_bounds__(256) k_rb_brick(Grid g, int nbx, int nby, int nb, const T *__restrict__ pin,
+                                                  T *__restrict__ pout, typename P::Args args) {
+  __shared__ T sp[KLZ][KY + 4][KLX];
+  const int w = blockIdx.x, b = (nb % 8 == 0) ? (w % 8) * (nb / 8) + w / 8 : w;
+  brick_tile<T, P, KY>(g, nbx, nby, b, pin, pout, args, sp);
+}
+
+// the three components of a sweep in one launch (visc_type -1 / 1)
+template <typename T, typename P0, typename P1, typename P2, int KY>
+__global__ void __launch_bounds__(256) k_rb_brick3(Grid g, int nbx, int nby, int nb, Ptr3<const T> pin, Ptr3<T> pout,
+                                                   typename P0::Args a0, typename P1::Args a1,
+                                                   typename P2::Args a2) {
+  __shared__ T sp[KLZ][KY + 4][KLX];
+  const int ns = 3 * nb, w = blockIdx.x, slot = (ns % 8 == 0) ? (w % 8) * (ns / 8) + w / 8 : w;
+  const int b = slot / 3, comp = slot - 3 * b;
+  if (comp == 0) brick_tile<T, P0, KY>(g, nbx, nby, b, pin.c[0], pout.c[0], a0, sp);
+  else if (comp == 1) brick_tile<T, P1, KY>(g, nbx, nby, b, pin.c[1], pout.c[1], a1, sp);
+  else brick_tile<T, P2, KY>(g, nbx, nby, b, pin.c[2], pout.c[2], a2, sp);
+}
+
+struct Bricks {
+  int nx, ny, n;
+};
+inline Bricks bricks(const Grid &g, int ky) {
+  const int nx = (g.n[0] + KX - 1) / KX, ny = (g.n[1] + ky - 1) / ky;
+  return {nx, ny, nx * ny * ((g.n[2] + KZ - 1) / KZ)};
+}
+
+// Rows of a brick: 8 (two pairs a thread, a smaller share of ring points)
+// where that still makes 768 workgroups, three on a compute unit, else 4.
+// Sweep of ncomp components, 4 rows / 8 rows in us: 32^3 FP64 7.2 / 9.2, 64^3
+// FP64 15.8 / 14.0 (three components) and 8.2 / 9.1 (cell-centred), 128 x 96 x
+// 64 FP64 36.2 / 33.6 and 14.9 / 13.5, 128^3 FP32 visc_type 2 30.1 / 26.9.
+// visc_type 2 and 3 in FP64 hold so many cross terms that two pairs a thread
+// leave two waves a SIMD: 4 rows there (128 x 96 x 64 17.3 / 18.0, 192 x 128 x
+// 96 44.2 / 45.2).
+inline int brick_rows(const Grid &g, int ncomp, bool cross64 = false) {
+  return !cross64 && ncomp * bricks(g, 8).n >= 768 ? 8 : 4;
+}
+
+// tx: the march's tile width (64, or 32 with 32 x 16 tiles); 0: the brick form
 template <typename T, typename P>
 void launch_rb(hipStream_t s, const Grid &g, int tz, int tx, const T *pin, T *pout, const typename P::Args &args) {
-  const T *q[5];
-  P::ptrs(args, q);
-  if (tuning().rb_variant == 1) {
-    const int nbx = g.n[0] / BX, nby = g.n[1] / BY, nbz = g.n[2] / BZ;
-    const int nb = nbx * nby * nbz;
-    hipLaunchKernelGGL((k_rb_block<T, P>), dim3(nb), dim3(256), 0, s, g, nbx, nby, nb, pin, pout, args, q[0], q[1],
-                       q[2], q[3], q[4]);
-    post_launch(s, kBlockName);
-    return;
-  }
-  const int fy = (tx == FX2) ? FY2 : FY;
-  const int ntx = g.n[0] / tx, nty = g.n[1] / fy, ntz = g.n[2] / tz;
-  const int ntiles = ntx * nty * ntz;
-  if (tuning().rb_variant == 2) {
+  if (tx == 0) {
+    const int ky = brick_rows(g, 1, P::CROSS && sizeof(T) == 8);
+    const Bricks b = bricks(g, ky);
     LaunchEvents *ev = launch_events();
-    // FP32 prefetches the next plane's coefficients (FP64 would lose occupancy)
-    const bool pf = sizeof(T) == 4 && tuning().rb_prefetch;
-    auto kern = (tx == FX2) ? (pf ? k_rb_march2<T, P, true, FX2> : k_rb_march2<T, P, false, FX2>)
-                            : (pf ? k_rb_march2<T, P, true, FX> : k_rb_march2<T, P, false, FX>);
-    if (ev->start) {
-      hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, tz, ntx, nty, ntiles, pin,
-                            pout, args, q[0], q[1], q[2], q[3], q[4]);
-      ev->start = ev->stop = nullptr;
-    } else {
-      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args, q[0], q[1],
-                         q[2], q[3], q[4]);
-    }
-    post_launch(s, kMarchName);
+    auto kern = ky == 8 ? k_rb_brick<T, P, 8> : k_rb_brick<T, P, 4>;
+    hipExtLaunchKernelGGL(kern, dim3(b.n), dim3(256), 0, s, ev->start, ev->stop, 0, g, b.nx, b.ny, b.n,
+                          pin, pout, args);
+    ev->start = ev->stop = nullptr;
+    post_launch(s, kBrickName);
     return;
   }
-  hipLaunchKernelGGL((k_rb_fused<T, P>), dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args,
-                     q[0], q[1], q[2], q[3], q[4]);
-  post_launch(s, kFusedName);
+  if constexpr (P::BRICK_ONLY) {
+    report_error("launch_rb: only the brick form is built for this viscosity type");
+  } else {
+    const T *q[5];
+    P::ptrs(args, q);
+    if (tuning().rb_variant == 1) {
+      const int nbx = g.n[0] / BX, nby = g.n[1] / BY, nbz = g.n[2] / BZ;
+      const int nb = nbx * nby * nbz;
+      hipLaunchKernelGGL((k_rb_block<T, P>), dim3(nb), dim3(256), 0, s, g, nbx, nby, nb, pin, pout, args, q[0], q[1],
+                         q[2], q[3], q[4]);
+      post_launch(s, kBlockName);
+      return;
+    }
+    const int fy = (tx == FX2) ? FY2 : FY;
+    const int ntx = g.n[0] / tx, nty = g.n[1] / fy, ntz = g.n[2] / tz;
+    const int ntiles = ntx * nty * ntz;
+    if (tuning().rb_variant == 2) {
+      LaunchEvents *ev = launch_events();
+      // FP32 prefetches the next plane's coefficients (FP64 would lose occupancy)
+      const bool pf = sizeof(T) == 4 && tuning().rb_prefetch;
+      auto kern = (tx == FX2) ? (pf ? k_rb_march2<T, P, true, FX2> : k_rb_march2<T, P, false, FX2>)
+                              : (pf ? k_rb_march2<T, P, true, FX> : k_rb_march2<T, P, false, FX>);
+      if (ev->start) {
+        hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, tz, ntx, nty, ntiles, pin,
+                              pout, args, q[0], q[1], q[2], q[3], q[4]);
+        ev->start = ev->stop = nullptr;
+      } else {
+        hipLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args, q[0], q[1],
+                           q[2], q[3], q[4]);
+      }
+      post_launch(s, kMarchName);
+      return;
+    }
+    hipLaunchKernelGGL((k_rb_fused<T, P>), dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args,
+                       q[0], q[1], q[2], q[3], q[4]);
+    post_launch(s, kFusedName);
+  }
 }
 
 // Residual r = rhs - L phi of one face component and its full-weighting
@@ -758,6 +925,17 @@ void launch_stag_three(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz,
   P1::ptrs(a1, q1);
   P2::ptrs(a2, q2);
   LaunchEvents *ev = launch_events();
+  if (tx == 0) {
+    const int ky = brick_rows(g, 3);
+    const Bricks b = bricks(g, ky);
+    const Ptr3<const T> in = {{pin[0], pin[1], pin[2]}};
+    auto kern = ky == 8 ? k_rb_brick3<T, P0, P1, P2, 8> : k_rb_brick3<T, P0, P1, P2, 4>;
+    hipExtLaunchKernelGGL(kern, dim3(3 * b.n), dim3(256), 0, s, ev->start, ev->stop, 0, g,
+                          b.nx, b.ny, b.n, in, p3(pout), a0, a1, a2);
+    ev->start = ev->stop = nullptr;
+    post_launch(s, kBrickName);
+    return;
+  }
   // FP32 prefetches the next plane's coefficients (FP64 would lose occupancy)
   const bool pf = sizeof(T) == 4 && tuning().rb_prefetch;
   if (tx == FX && np == 2) {
@@ -1117,8 +1295,12 @@ void launch_stag_one(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz, i
     a.e2 = cur[A == 2 ? 1 : 2];
   } else {
     // xy = 0, xz = 1, yz = 2; edges shared with (A, t1) and (A, t2)
-    a.e1 = (VISC == -1) ? K.bed[A == 2 ? 1 : 0] : nullptr;
-    a.e2 = (VISC == -1) ? K.bed[A == 0 ? 1 : 2] : nullptr;
+    a.e1 = (VISC < 0) ? K.bed[A == 2 ? 1 : 0] : nullptr;
+    a.e2 = (VISC < 0) ? K.bed[A == 0 ? 1 : 2] : nullptr;
+  }
+  if (VISC < -1) {
+    a.o1 = cur[A == 0 ? 1 : 0];
+    a.o2 = cur[A == 2 ? 1 : 2];
   }
   launch_rb<T, StagRB<T, A, VISC>>(s, g, tz, tx, pin, pout, a);
 }
@@ -1139,6 +1321,32 @@ bool fused_rb_takes_zeros() { return tuning().rb_variant == 2; }
 static int rb_target(int es) {
   const int t = tuning().rb_target > 0 ? tuning().rb_target : 1;
   return es == 8 ? 2 * t : t;
+}
+
+// Whether a level is swept in bricks: levels that are too small to stream,
+// and every level whose extents the plane-marching tiles do not divide (asked
+// after rb_tz), where the alternative is two colour passes a component.
+// min_tiles above its default of 64 workgroups counts bricks; at or below it
+// any level qualifies (one brick launch replaces two colour launches a
+// component).
+enum BrickUse { BRICK_THREE, BRICK_ONE, BRICK_CC };  // three components a launch, one, cell-centred
+static bool brick_ok(const Grid &g, int min_tiles, int ncomp) {
+  return tuning().rb_variant == 2 && tuning().rb_brick != 0 && g.dim == 3 && g.n[0] >= 4 && g.n[1] >= 4 &&
+         g.n[2] >= 4 && (min_tiles <= 64 || ncomp * bricks(g, 4).n >= min_tiles);
+}
+// The line between bricks and marching tiles.  Sweep in us, marching / brick:
+//   three components  FP64  64^3 16.8 / 14.0, 128x96x64 42.6 / 33.6, 192x128x96 95 / 102, 128^3 71 / 86
+//                     FP32  64^3 17.5 / 15.7, 128x96x64 31.3 / 25.7, 192x128x96 59 / 65, 128^3 42 / 59
+//   one (visc_type 2) FP64  64^3 11.3 / 9.1, 128^3 46.5 / 39.5, 192x192x128 92 / 93, 256^3 247 / 339
+//                     FP32  64^3 10.1 / 7.9, 128^3 28.7 / 26.9, 192x192x128 53 / 54, 256^3 167 / 198
+//   cell-centred      FP64  64^3 10.3 / 8.2, 128^3 36.8 / 30.5, 192x192x128 60 / 62, 256^3 200 / 241
+//                     FP32  64^3 9.5 / 7.3, 128x96x64 13.4 / 12.4, 128^3 20.7 / 23.5, 256^3 107 / 153
+static bool brick_level(const Grid &g, int min_tiles, int ncomp, BrickUse use, int es) {
+  const long most = tuning().rb_brick >= 0 ? tuning().rb_brick
+                    : use == BRICK_ONE     ? 4000000
+                    : use == BRICK_CC      ? (es == 8 ? 3000000 : 1200000)
+                                           : 1200000;
+  return g.N <= most && brick_ok(g, min_tiles, ncomp);
 }
 
 // Plane count per workgroup, or 0 when the level cannot use the fused
@@ -1167,17 +1375,24 @@ static int rb_tz(const Grid &g, int min_tiles, int es, int ncomp, int fx, int fy
 // plane-marching form only) 32 x 16 tiles on levels 32 points wide.  nsweep
 // launches of this shape make one sweep (the staggered components one after
 // another, 1 for the cell-centred field); together they must reach min_tiles.
-static int rb1_shape(const Grid &g, int min_tiles, int es, int &tx, int nsweep = 1) {
+static int rb1_shape(const Grid &g, int min_tiles, int es, int &tx, int nsweep = 1, BrickUse use = BRICK_CC) {
   tx = FX;
   if (tuning().rb_variant == 1) {
     if (g.dim != 3 || g.n[0] % BX != 0 || g.n[1] % BY != 0 || g.n[2] % BZ != 0) return 0;
     const int nb = (g.n[0] / BX) * (g.n[1] / BY) * (g.n[2] / BZ);
     return nsweep * nb >= min_tiles ? BZ : 0;
   }
-  const int tz = rb_tz(g, min_tiles, es, 1, FX, FY, nsweep);
+  if (brick_level(g, min_tiles, nsweep, use, es)) {
+    tx = 0;
+    return KZ;
+  }
+  int tz = rb_tz(g, min_tiles, es, 1, FX, FY, nsweep);
   if (tz > 0 || tuning().rb_variant != 2) return tz;
   tx = FX2;
-  return rb_tz(g, min_tiles, es, 1, FX2, FY2, nsweep);
+  tz = rb_tz(g, min_tiles, es, 1, FX2, FY2, nsweep);
+  if (tz > 0 || !brick_ok(g, min_tiles, nsweep)) return tz;
+  tx = 0;
+  return KZ;
 }
 
 int fused_rb_tz(const Grid &g, int min_tiles, int es, int ncomp) {
@@ -1189,15 +1404,20 @@ int fused_rb_tz(const Grid &g, int min_tiles, int es, int ncomp) {
 
 bool fused_rb_ok(const Grid &g, int visc, int min_tiles) {
   int tx;
-  return (visc == -1 || visc == 1 || visc == 2 || visc == 3) && rb1_shape(g, min_tiles, 4, tx, g.dim) > 0;
+  if (visc < -1) return brick_ok(g, min_tiles, g.dim);
+  return (visc == -1 || visc == 1 || visc == 2 || visc == 3) && rb1_shape(g, min_tiles, 4, tx, g.dim, BRICK_ONE) > 0;
 }
 
 template <typename T>
 void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega, const T *pin, T *pout,
                           const T *rhs, const StagCoef<T> &K, int min_tiles, const T *const cur[3]) {
   int tx = FX;
-  const int tz = rb1_shape(g, min_tiles, sizeof(T), tx, g.dim);
-  if (tz <= 0 || !fused_rb_ok(g, visc, min_tiles) || ((visc == 2 || visc == 3) && !cur)) {
+  int tz = rb1_shape(g, min_tiles, sizeof(T), tx, g.dim, BRICK_ONE);
+  if (visc < -1) {
+    tx = 0;
+    tz = KZ;
+  }
+  if (tz <= 0 || !fused_rb_ok(g, visc, min_tiles) || (visc != 1 && visc != -1 && !cur)) {
     report_error("launch_stag_rb_fused: level not eligible");
     return;
   }
@@ -1211,7 +1431,9 @@ void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega
   if (visc == -1) ONE(-1);
   else if (visc == 1) ONE(1);
   else if (visc == 2) ONE(2);
-  else ONE(3);
+  else if (visc == 3) ONE(3);
+  else if (visc == -2) ONE(-2);
+  else ONE(-3);
 #undef ONE
 }
 
@@ -1219,6 +1441,11 @@ void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega
 // 64 x 16 tiles, where tuning asks for them) and z-slab of the
 // three-component sweep; 0 when the level cannot use it
 static int rb3_shape(const Grid &g, int min_tiles, int es, int &tx, int &np) {
+  np = 1;
+  if (brick_level(g, min_tiles, 3, BRICK_THREE, es)) {
+    tx = 0;
+    return KZ;
+  }
   tx = FX;
   np = 2;
   if (tuning().rb_pairs == 2 && es == 4) {  // FP64 would need 80 KB of LDS per workgroup
@@ -1226,10 +1453,13 @@ static int rb3_shape(const Grid &g, int min_tiles, int es, int &tx, int &np) {
     if (tz2 > 0) return tz2;
   }
   np = 1;
-  const int tz = rb_tz(g, min_tiles, es, 3, FX, FY);
+  int tz = rb_tz(g, min_tiles, es, 3, FX, FY);
   if (tz > 0) return tz;
   tx = FX2;
-  return rb_tz(g, min_tiles, es, 3, FX2, FY2);
+  tz = rb_tz(g, min_tiles, es, 3, FX2, FY2);
+  if (tz > 0 || !brick_ok(g, min_tiles, 3)) return tz;
+  tx = 0;
+  return KZ;
 }
 
 bool fused_rb3_ok(const Grid &g, int visc, int min_tiles) {

@@ -1515,6 +1515,8 @@ static void apply_options(lmm_ctx *c, const lmm_kernel_options &o) {
   c->tune.rb_prefetch = o.sweep_prefetch;
   const char *pairs = getenv("LMM_SWEEP_PAIRS");
   c->tune.rb_pairs = (pairs && pairs[0] == '1') ? 1 : 2;
+  const char *bk = getenv("LMM_SWEEP_BRICK");
+  c->tune.rb_brick = bk ? atol(bk) : -1;
   const char *pt = getenv("LMM_PROLONG_TILED");
   c->tune.prolong_tiled = (pt && pt[0] == '0') ? 0 : 1;
   const char *cs = getenv("LMM_COARSE_SPLIT");
