@@ -29,10 +29,9 @@
 // compute_mass_fluxdiv.f90 runs as one cell pass (sp_chain_cell), which
 // writes only what the faces need (mole fractions, rho W chi, Gama unless
 // the mixture is ideal, zeta/T, the packed lower triangle of the Cholesky
-// factor of L-Onsager) and restores rho, then (up to 4 species) one face
-// pass computing both fluxes of every face (flux_total written once) and one
-// pass for both divergences, or (more species) a pass and a divergence per
-// flux (sp_chain_face).  Giving each cell
+// factor of L-Onsager) and restores rho, then one face pass computing both
+// fluxes of every face (flux_total written once) and one pass for both
+// divergences (sp_chain_face).  Giving each cell
 // its upper faces too (recomputed, so the face arrays need not be stored)
 // was tried: the two matrix-vector chains per face kept so many loads live
 // that the kernel ran at one wave per SIMD with spills from 5 species up.
@@ -589,59 +588,40 @@ __global__ void __launch_bounds__(STPB) k_sp_lonsager(Grid g, SpParams sp, const
 
 // ---------------- face fluxes ----------------
 
-// diffusive_mass_flux on the face between cells t (above) and m (below):
-// grad x, Gama_face grad x (identity when gama is null), + zeta_face grad T,
-// + baro_face gradp_baro, rhoWchi_face (...), correction_flux.
+// acc[r] += sum_c 0.5 (M(r, c) at t + at m) v[c], c ascending; LOWER: r >= c.
+// The loads of column c + 1 are issued before column c is summed, so a column's
+// wait overlaps the one before it.  The empty asm makes the indices of later
+// columns depend on the sums of earlier ones: scheduling fences alone let the
+// compiler load the whole matrix of both cells first (eight species: 256
+// registers and one wave per SIMD, 73 us at 384 x 320; now 121 and 61 us).
+template <int NS, bool LOWER>
+__device__ __forceinline__ void face_matvec(const double *M, long N, long t, long m, const double (&v)[NS],
+                                            double (&acc)[NS]) {
+  double a[2][NS], b[2][NS];
+#pragma unroll
+  for (int c = 0; c <= NS; c++) {
+    if (c < NS) {
+#pragma unroll
+      for (int r = 0; r < NS; r++)
+        if (!LOWER || r >= c) {
+          const long q = (long)(r + NS * c) * N;
+          a[c & 1][r] = M[q + t];
+          b[c & 1][r] = M[q + m];
+        }
+    }
+    if (c > 0) {
+#pragma unroll
+      for (int r = 0; r < NS; r++)
+        if (!LOWER || r >= c - 1) {
+          acc[r] = acc[r] + 0.5 * (a[(c - 1) & 1][r] + b[(c - 1) & 1][r]) * v[c - 1];
+          asm volatile("" : "+v"(t), "+v"(m), "+v"(acc[r]));
+        }
+    }
+  }
+}
+
 template <int NS>
-__device__ __forceinline__ void diff_face(const SpParams &sp, long N, double dxinv, long t, long m, const double *xm,
-                                          const double *rw, const double *gama, const double *temp, const double *zeta,
-                                          const double *baro, double gpb, double (&out)[NS]) {
-  // opaque copies of the cell indices: keeps the compiler from hoisting the
-  // 2*NS^2 per-lane addresses of this face out of a caller's loop (which
-  // would hold them all in VGPRs); no instruction is emitted
-  asm volatile("" : "+v"(t), "+v"(m));
-  double x[NS], y[NS];
-#pragma unroll
-  for (int s = 0; s < NS; s++) x[s] = (xm[(long)s * N + t] - xm[(long)s * N + m]) * dxinv;
-  if (gama) {
-    // column-outer order: each y[r] still sums c = 0, 1, ... in turn, and the
-    // scheduling fence after each column keeps only one column's loads live
-#pragma unroll
-    for (int r = 0; r < NS; r++) y[r] = 0.0;
-#pragma unroll
-    for (int c = 0; c < NS; c++) {
-#pragma unroll
-      for (int r = 0; r < NS; r++) {
-        const long q = (long)(r + NS * c) * N;
-        y[r] = y[r] + 0.5 * (gama[q + t] + gama[q + m]) * x[c];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
-    // Gama_face = I: the sum 0 + 0*x_0 + ... + 1*x_r + ... is 0 + x_r
-#pragma unroll
-    for (int r = 0; r < NS; r++) y[r] = 0.0 + x[r];
-  }
-  if (zeta) {
-    const double gT = (temp[t] - temp[m]) * dxinv;
-#pragma unroll
-    for (int s = 0; s < NS; s++) y[s] = y[s] + 0.5 * (zeta[(long)s * N + t] + zeta[(long)s * N + m]) * gT;
-  }
-  if (baro) {
-#pragma unroll
-    for (int s = 0; s < NS; s++) y[s] = y[s] + 0.5 * (baro[(long)s * N + t] + baro[(long)s * N + m]) * gpb;
-  }
-#pragma unroll
-  for (int r = 0; r < NS; r++) out[r] = 0.0;
-#pragma unroll
-  for (int c = 0; c < NS; c++) {
-#pragma unroll
-    for (int r = 0; r < NS; r++) {
-      const long q = (long)(r + NS * c) * N;
-      out[r] = out[r] + 0.5 * (rw[q + t] + rw[q + m]) * y[c];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
+__device__ __forceinline__ void correct_flux(const SpParams &sp, double (&out)[NS]) {
   if (sp.correct && NS > 1) {
     double sum = 0.0;
 #pragma unroll
@@ -650,41 +630,84 @@ __device__ __forceinline__ void diff_face(const SpParams &sp, long N, double dxi
   }
 }
 
+// Gama_face grad x + zeta_face grad T + baro_face gradp_baro of the face
+// between cells t (above) and m (below): the vector that
+// rhoWchi_face multiplies.  Gama null: identity.
+template <int NS>
+__device__ __forceinline__ void diff_drive(long N, double dxinv, long t, long m, const double *xm, const double *gama,
+                                           const double *temp, const double *zeta, const double *baro, double gpb,
+                                           double (&y)[NS]) {
+  double x[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) x[s] = (xm[(long)s * N + t] - xm[(long)s * N + m]) * dxinv;
+  if (gama) {
+#pragma unroll
+    for (int r = 0; r < NS; r++) y[r] = 0.0;
+    face_matvec<NS, false>(gama, N, t, m, x, y);
+  } else {
+    // Gama_face = I: the sum 0 + 0*x_0 + ... + 1*x_r + ... is 0 + x_r
+#pragma unroll
+    for (int r = 0; r < NS; r++) y[r] = 0.0 + x[r];
+  }
+  if (zeta) {
+    const double gT = (temp[t] - temp[m]) * dxinv;
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+      y[s] = y[s] + 0.5 * (zeta[(long)s * N + t] + zeta[(long)s * N + m]) * gT;
+  }
+  if (baro) {
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+      y[s] = y[s] + 0.5 * (baro[(long)s * N + t] + baro[(long)s * N + m]) * gpb;
+  }
+}
+
+// diffusive_mass_flux: rhoWchi_face times the above, correction_flux.
+template <int NS>
+__device__ __forceinline__ void diff_face(const SpParams &sp, long N, double dxinv, long t, long m, const double *xm,
+                                          const double *rw, const double *gama, const double *temp, const double *zeta,
+                                          const double *baro, double gpb, double (&out)[NS]) {
+  // opaque copies of the indices: keeps the compiler from hoisting this face's
+  // loads out of a caller's loop; no instruction is emitted
+  asm volatile("" : "+v"(t), "+v"(m));
+  double y[NS];
+  diff_drive<NS>(N, dxinv, t, m, xm, gama, temp, zeta, baro, gpb, y);
+#pragma unroll
+  for (int r = 0; r < NS; r++) out[r] = 0.0;
+  face_matvec<NS, false>(rw, N, t, m, y, out);
+  correct_flux<NS>(sp, out);
+}
+
+// sum_r w_r W_r of the face of cell t in direction d
+template <int NS>
+__device__ __forceinline__ void face_noise(long N, long t, int d, int dim, const double *W, int n_rngs,
+                                           const double *weights, double (&w)[NS]) {
+#pragma unroll
+  for (int s = 0; s < NS; s++) w[s] = 0.0;
+  for (int r = 0; r < n_rngs; r++) {
+    const double wr = weights[r];
+#pragma unroll
+    for (int s = 0; s < NS; s++) w[s] = w[s] + wr * __builtin_nontemporal_load(W + ((long)(r * dim + d) * NS + s) * N + t);
+  }
+}
+
 // stochastic flux on the face of cell t in direction d: variance *
 // L_face (sum_r w_r W_r), L_face the face average of the cell factors
 // (upper triangle zero, so only c <= r enters: adding 0*w leaves the sum's
-// bits unchanged), then correction_flux.  Packed (lpk) or full (Lf) factors.
-template <int NS, bool PACKED>
-__device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, long m, int d, int dim,
-                                           const double *L, const double *W, int n_rngs, const double *weights,
-                                           double variance, double (&out)[NS]) {
+// bits unchanged), then correction_flux.
+template <int NS>
+__device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, long m, int d, int dim, const double *L,
+                                           const double *W, int n_rngs, const double *weights, double variance,
+                                           double (&out)[NS]) {
   asm volatile("" : "+v"(t), "+v"(m));
   double w[NS];
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    double acc = 0.0;
-    for (int r = 0; r < n_rngs; r++) acc = acc + weights[r] * W[((long)(r * dim + d) * NS + s) * N + t];
-    w[s] = acc;
-  }
+  face_noise<NS>(N, t, d, dim, W, n_rngs, weights, w);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = 0.0;
-#pragma unroll
-  for (int c = 0; c < NS; c++) {
-#pragma unroll
-    for (int r = c; r < NS; r++) {
-      const long q = (long)(PACKED ? lpk_index<NS>(r, c) : r + NS * c) * N;
-      out[r] = out[r] + 0.5 * (L[q + t] + L[q + m]) * w[c];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  face_matvec<NS, true>(L, N, t, m, w, out);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = out[r] * variance;
-  if (sp.correct && NS > 1) {
-    double sum = 0.0;
-#pragma unroll
-    for (int s = 0; s < NS - 1; s++) sum = sum + out[s];
-    out[NS - 1] = -sum;
-  }
+  correct_flux<NS>(sp, out);
 }
 
 // flux_total: ft_zero set -> 0.0 + F (setval then add), else ft + F
@@ -703,17 +726,19 @@ __global__ void __launch_bounds__(STPB) k_sp_diff_flux(Grid g, SpParams sp, cons
   for (int d = 0; d < g.dim; d++) {
     const long m = at_sh(g, P, d, -1, -1, 0);
     double out[NS];
-    diff_face<NS>(sp, N, dxinv, t, m, xm, rw, gama, temp, zeta, baro, baro ? gpb.c[d][t] : 0.0, out);
+    diff_face<NS>(sp, N, dxinv, t, m, xm, rw, gama, temp, zeta, baro,
+                  baro ? gpb.c[d][t] : 0.0, out);
+    double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       flux[((long)d * NS + s) * N + t] = out[s];
-      const long q = (long)s * N + t;
-      ft.c[d][q] = (ft_zero ? 0.0 : ft.c[d][q]) + out[s];
+      const long q = (long)s * N;
+      f[q + t] = (ft_zero ? 0.0 : f[q + t]) + out[s];
     }
   }
 }
 
-template <int NS, bool PACKED>
+template <int NS>
 __global__ void __launch_bounds__(STPB) k_sp_stoch_flux(Grid g, SpParams sp, const double *L, const double *W,
                                                          int n_rngs, const double *weights, double variance,
                                                          double *flux, Ptr3<double> ft) {
@@ -726,11 +751,12 @@ __global__ void __launch_bounds__(STPB) k_sp_stoch_flux(Grid g, SpParams sp, con
   for (int d = 0; d < g.dim; d++) {
     const long m = at_sh(g, P, d, -1, -1, 0);
     double out[NS];
-    stoch_face<NS, PACKED>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
+    stoch_face<NS>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
+    double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       flux[((long)d * NS + s) * N + t] = out[s];
-      ft.c[d][(long)s * N + t] = ft.c[d][(long)s * N + t] + out[s];
+      f[(long)s * N + t] = f[(long)s * N + t] + out[s];
     }
   }
 }
@@ -759,32 +785,205 @@ __global__ void __launch_bounds__(STPB) k_sp_div(Grid g, const double *flux, dou
   }
 }
 
-// compute_mass_fluxdiv's face pass: both fluxes of each lower face in one
-// thread (the diffusive then the stochastic, fenced so their loads do not
-// pile up), flux_total = (0 + F_diff) + F_stoch written once.
-template <int NS>
-__global__ void __launch_bounds__(STPB) k_sp_chain_flux(Grid g, SpParams sp, SpFaceIn in, double *fd, double *fs,
-                                                         Ptr3<double> ft) {
-  const long t = xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= g.N) return;
-  int i, j, k;
-  decode(g, t, i, j, k);
-  const Pt P = make_pt(g, i, j, k);
-  const long N = g.N;
+// compute_mass_fluxdiv's face pass: both fluxes of each cell's lower faces in
+// one kernel, flux_total = (0 + F_diff) + F_stoch written once.
+//
+// A face needs the matrices of its two cells, NS^2 + NS (NS + 1) / 2 values
+// and more each, so a thread that walks its faces one by one reads its own
+// cell's once and its neighbours' per direction, long after they left the
+// XCD's 4 MB of L2 (the cells in flight there hold five times that).  Here a
+// workgroup owns a 32 x 8 tile of a plane and takes the matrices column by
+// column: the column is loaded once per cell (and for the tile's lower x and y
+// halo), passed through LDS, and applied to the faces of all directions; the
+// cell below in z reads it from memory beside the cell's own, when it is in L2.
+// The next column is loaded before the current one is applied.  128^3, four
+// species, two noise stages: 595 us face by face, 427 here (1.6 GB that a face
+// pass cannot do without, 3.7 TB/s; 64 x 4 tiles, with a larger halo, 481);
+// 384 x 320, eight species: 124 us in a pass and a divergence per flux, 49 for
+// this and the common divergence.  The noise is read and flux_total written
+// past the caches (427 against 447 us); the two fluxes are not, the divergence
+// reads them next.
+constexpr int FTX = 32, FTY = 8;
+constexpr int FHX = FTX + 1, FHY = FTY + 1;  // with the lower halo column and row
+constexpr int FHALO = FTX + FTY;
+
+template <int NS, int DIM>
+struct FaceTile {
+  static constexpr int NH = (FHALO * NS + STPB - 1) / STPB;
+  struct Col {
+    double own[NS], z[DIM == 3 ? NS : 1], halo[NH];
+  };
+  long N, t, mz;            // the thread's cell and the one below it in z
+  int at;                   // its place in a tile
+  long hc[NH];              // halo cells that the thread loads: cell,
+  int hr[NH], hat[NH];      // component (NS and more: none) and place
+  double (*tile)[NS][FHY * FHX];  // two columns
+
+  // Loads from here on wait for v (no instruction): left alone, the compiler
+  // loads whole matrices ahead of their columns, barriers or not.
+  __device__ __forceinline__ void after(double &v) {
+    asm volatile("" : "+v"(t), "+v"(mz), "+v"(v));
+#pragma unroll
+    for (int n = 0; n < NH; n++) asm volatile("" : "+v"(hc[n]), "+v"(v));
+  }
+  // component `index(r, c)` of M for r >= first(c)
+  template <class IX>
+  __device__ __forceinline__ void load(Col &a, const double *M, int lo, IX index) const {
+#pragma unroll
+    for (int r = 0; r < NS; r++)
+      if (r >= lo) {
+        a.own[r] = M[(long)index(r) * N + t];
+        if constexpr (DIM == 3) a.z[r] = M[(long)index(r) * N + mz];
+      }
+#pragma unroll
+    for (int n = 0; n < NH; n++)
+      if (hr[n] >= lo && hr[n] < NS) a.halo[n] = M[(long)index(hr[n]) * N + hc[n]];
+  }
+  __device__ __forceinline__ void put(const Col &a, int lo, int half) const {
+#pragma unroll
+    for (int r = 0; r < NS; r++)
+      if (r >= lo) tile[half][r][at] = a.own[r];
+#pragma unroll
+    for (int n = 0; n < NH; n++)
+      if (hr[n] >= lo && hr[n] < NS) tile[half][hr[n]][hat[n]] = a.halo[n];
+  }
+  // the value of the cell below in direction d
+  __device__ __forceinline__ double below(const Col &a, int d, int r, int half) const {
+    if (DIM == 3 && d == 2) return a.z[DIM == 3 ? r : 0];
+    return tile[half][r][d == 0 ? at - 1 : at - FHX];
+  }
+  // f(d, r, own, below), a reference to what it computed, of one vector
+  template <class F>
+  __device__ __forceinline__ void vec(const double *V, F f) {
+    Col a;
+    load(a, V, 0, [](int r) { return r; });
+    __syncthreads();
+    put(a, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < DIM; d++)
+#pragma unroll
+      for (int r = 0; r < NS; r++) after(f(d, r, a.own[r], below(a, d, r, 0)));
+  }
+  // acc[d][r] += 0.5 (M(r, c) here + below) v[d][c], c ascending
+  template <bool LOWER, class IX>
+  __device__ __forceinline__ void matvec(const double *M, const double (&v)[DIM][NS], double (&acc)[DIM][NS],
+                                         IX index) {
+    Col a, b;
+    load(a, M, 0, [&](int r) { return index(r, 0); });
+    __syncthreads();  // the tiles' last readers are done
+#pragma unroll
+    for (int c = 0; c < NS; c++) {
+      const int lo = LOWER ? c : 0;
+      if (c + 1 < NS) load(b, M, LOWER ? c + 1 : 0, [&](int r) { return index(r, c + 1); });
+      put(a, lo, c & 1);
+      // one barrier a column: a tile is written again two columns on, past the
+      // barrier that its readers reach after reading it
+      __syncthreads();
+#pragma unroll
+      for (int d = 0; d < DIM; d++)
+#pragma unroll
+        for (int r = 0; r < NS; r++)
+          if (r >= lo) {
+            acc[d][r] = acc[d][r] + 0.5 * (a.own[r] + below(a, d, r, c & 1)) * v[d][c];
+            after(acc[d][r]);
+          }
+      a = b;
+    }
+  }
+};
+
+template <int NS, int DIM>
+__global__ void __launch_bounds__(STPB) k_sp_chain_flux(Grid g, SpParams sp, SpFaceIn in, int nbx, int nz, double *fd,
+                                                         double *fs, Ptr3<double> ft) {
+  using Tile = FaceTile<NS, DIM>;
+  __shared__ double tile[2][NS][FHY * FHX];
+  // tiles along x, then z, then y: the plane below is a few workgroups back
+  const unsigned w = (unsigned)xcd_block(), bx = w % nbx, q = w / nbx, k = q % nz, by = q / nz;
+  const int nx = g.n[0], ny = g.n[1];
+  const long sy = g.s[1], sz = DIM == 3 ? g.s[2] : 0;
+  const int lx = threadIdx.x % FTX, ly = threadIdx.x / FTX, i0 = bx * FTX, j0 = by * FTY;
+  const bool inside = i0 + lx < nx && j0 + ly < ny;
+  // cells of a tile that hangs over the box: periodic images, nothing stored
+  const long plane = sz * k;
+  auto cell = [&](int i, int j) { return wrap_any(i, nx) + sy * wrap_any(j, ny) + plane; };
+  Tile T;
+  T.N = g.N;
+  T.t = cell(i0 + lx, j0 + ly);
+  T.mz = DIM == 3 ? T.t - plane + sz * (k == 0 ? nz - 1 : k - 1) : T.t;
+  T.at = (ly + 1) * FHX + lx + 1;
+  T.tile = tile;
+#pragma unroll
+  for (int n = 0; n < Tile::NH; n++) {
+    const int h = threadIdx.x + STPB * n, e = h % FHALO;  // e: the row below, then the column below
+    const int hx = e < FTX ? e : -1, hy = e < FTX ? -1 : e - FTX;
+    T.hr[n] = h / FHALO;
+    T.hc[n] = cell(i0 + hx, j0 + hy);
+    T.hat[n] = (hy + 1) * FHX + hx + 1;
+  }
+  const long N = g.N, t = T.t;
   const double dxinv = 1.0 / g.dx;
-  for (int d = 0; d < g.dim; d++) {
-    const long m = at_sh(g, P, d, -1, -1, 0);
-    double od[NS], os[NS];
-    diff_face<NS>(sp, N, dxinv, t, m, in.xm, in.rw, in.gama, in.temp, in.zeta, in.baro,
-                  in.baro ? in.gpb[d][t] : 0.0, od);
-    __builtin_amdgcn_sched_barrier(0);
-    stoch_face<NS, true>(sp, N, t, m, d, g.dim, in.lpk, in.W, in.n_rngs, in.weights, in.variance, os);
+  auto full = [](int r, int c) { return r + NS * c; };
+  double x[DIM][NS], y[DIM][NS];
+  T.vec(in.xm, [&](int d, int r, double a, double b) -> double & { return x[d][r] = (a - b) * dxinv; });
+  if (in.gama) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++)
+#pragma unroll
+      for (int r = 0; r < NS; r++) y[d][r] = 0.0;
+    T.template matvec<false>(in.gama, x, y, full);
+  } else {
+    // Gama_face = I: the sum 0 + 0*x_0 + ... + 1*x_r + ... is 0 + x_r
+#pragma unroll
+    for (int d = 0; d < DIM; d++)
+#pragma unroll
+      for (int r = 0; r < NS; r++) y[d][r] = 0.0 + x[d][r];
+  }
+  long m[DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; d++)
+    m[d] = d == 0 ? cell(i0 + lx - 1, j0 + ly) : (d == 1 ? cell(i0 + lx, j0 + ly - 1) : T.mz);
+  if (in.zeta) {
+    double gT[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) gT[d] = (in.temp[t] - in.temp[m[d]]) * dxinv;
+    T.vec(in.zeta, [&](int d, int r, double a, double b) -> double & {
+      return y[d][r] = y[d][r] + 0.5 * (a + b) * gT[d];
+    });
+  }
+  if (in.baro) {
+    double gp[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) gp[d] = in.gpb[d][t];
+    T.vec(in.baro, [&](int d, int r, double a, double b) -> double & {
+      return y[d][r] = y[d][r] + 0.5 * (a + b) * gp[d];
+    });
+  }
+  double od[DIM][NS], os[DIM][NS];
+#pragma unroll
+  for (int d = 0; d < DIM; d++)
+#pragma unroll
+    for (int r = 0; r < NS; r++) od[d][r] = os[d][r] = 0.0;
+  T.template matvec<false>(in.rw, y, od, full);
+  double wn[DIM][NS];
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+    correct_flux<NS>(sp, od[d]);
+    face_noise<NS>(N, T.t, d, DIM, in.W, in.n_rngs, in.weights, wn[d]);
+  }
+  T.template matvec<true>(in.lpk, wn, os, [](int r, int c) { return lpk_index<NS>(r, c); });
+  if (!inside) return;
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+#pragma unroll
+    for (int r = 0; r < NS; r++) os[d][r] = os[d][r] * in.variance;
+    correct_flux<NS>(sp, os[d]);
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       const long q = ((long)d * NS + s) * N + t;
-      fd[q] = od[s];
-      fs[q] = os[s];
-      ft.c[d][(long)s * N + t] = (0.0 + od[s]) + os[s];
+      fd[q] = od[d][s];
+      fs[q] = os[d][s];
+      __builtin_nontemporal_store((0.0 + od[d][s]) + os[d][s], ft.c[d] + (long)s * N + t);
     }
   }
 }
@@ -991,7 +1190,7 @@ template <int NS>
 struct RunStochastic {
   static int run(hipStream_t s, const Grid &g, const SpParams &sp, const double *L, const double *W, int nr,
                  const double *w, double var, double *flux, double *const ft[3], double *div, int inc) {
-    SLAUNCH((k_sp_stoch_flux<NS, false>), dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, L, W, nr, w, var, flux, p3(ft));
+    SLAUNCH(k_sp_stoch_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, L, W, nr, w, var, flux, p3(ft));
     SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, div, inc);
     return 0;
   }
@@ -1012,22 +1211,20 @@ struct RunChainFace {
   static int run(hipStream_t s, const Grid &g, const SpParams &sp, const SpFaceIn &in, double *flux, double *dd,
                  double *sd, double *const ft[3]) {
     SP_NEEDS2;
-    // up to 4 species both fluxes share one face pass (at 5 and more its
-    // registers drop it to 1-3 waves per SIMD: separate passes there)
-    if (in.W && NS <= 4) {  // flux holds 2 * dim * ns * N: the diffusive then the stochastic face fluxes
+    if (in.W) {  // flux holds 2 * dim * ns * N: the diffusive then the stochastic face fluxes
       double *fs = flux + (long)g.dim * NS * g.N;
-      SLAUNCH(k_sp_chain_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in, flux, fs, p3(ft));
+      const int nbx = (g.n[0] + FTX - 1) / FTX, nby = (g.n[1] + FTY - 1) / FTY, nz = g.dim == 3 ? g.n[2] : 1;
+      const dim3 nb(nbx * nby * nz);
+      if (g.dim == 3)
+        SLAUNCH((k_sp_chain_flux<NS, 3>), nb, dim3(STPB), 0, s, g, sp, in, nbx, nz, flux, fs, p3(ft));
+      else
+        SLAUNCH((k_sp_chain_flux<NS, 2>), nb, dim3(STPB), 0, s, g, sp, in, nbx, nz, flux, fs, p3(ft));
       SLAUNCH(k_sp_div2<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, dd, fs, sd);
       return 0;
     }
     SLAUNCH(k_sp_diff_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in.xm, in.rw, in.gama, in.temp, in.zeta,
             in.baro, cp3(in.baro ? in.gpb : nullptr), flux, p3(ft), 1);
     SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, dd, 0);
-    if (in.W) {
-      SLAUNCH((k_sp_stoch_flux<NS, true>), dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in.lpk, in.W, in.n_rngs,
-              in.weights, in.variance, flux, p3(ft));
-      SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, sd, 0);
-    }
     return 0;
   }
 };
