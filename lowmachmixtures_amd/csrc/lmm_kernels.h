@@ -84,21 +84,21 @@ template <typename T>
 void launch_stag_rb_fused3(hipStream_t s, const Grid &g, int visc, T omega, T *const pin[3], T *const pout[3],
                            T *const rhs[3], const StagCoef<T> &K, int min_tiles, bool zero_in);
 // Both components of one fused red-black sweep in one launch (2D, visc -1 /
-// 1, x a multiple of 64, y of 8, at least min_tiles workgroups); reads pin[a]
+// 1, even extents, at least min_tiles workgroups if more than 64); reads pin[a]
 // (zero_in: a field of zeros, pin not read), writes pout[a].
 bool fused_rb2d_ok(const Grid &g, int visc, int min_tiles);
 template <typename T>
 void launch_stag_rb2d(hipStream_t s, const Grid &g, int visc, T omega, T *const pin[3], T *const pout[3],
                       T *const rhs[3], const StagCoef<T> &K, bool zero_in);
-// One face component of a 2D fused red-black sweep of a visc_type 2 / 3
+// One face component of a 2D fused red-black sweep of a visc_type 2, 3, -2, -3
 // level (the components couple, so they go one after the other): reads the
 // component from pin and the other component's current state from other.
 bool fused_rb2d_comp_ok(const Grid &g, int visc, int min_tiles);
 template <typename T>
 void launch_stag_rb2d_comp(hipStream_t s, const Grid &g, int visc, int a, T omega, const T *pin, T *pout,
                            const T *rhs, const StagCoef<T> &K, const T *other);
-// The cell-centred red-black sweep of one 2D level in one launch (x a
-// multiple of 64, y of 8, at least min_tiles workgroups); a null pin is a
+// The cell-centred red-black sweep of one 2D level in one launch (even
+// extents, at least min_tiles workgroups if more than 64); a null pin is a
 // field of zeros.
 bool cc_rb2d_ok(const Grid &g, int min_tiles);
 template <typename T>

@@ -966,13 +966,13 @@ void launch_stag_three(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz,
 }
 
 // ---------------------------------------------------------------------------
-// 2D fused red-black sweep (visc_type -1 / 1): both face components in one
-// launch, a workgroup per (tile, component).  In 2D a component's colours
-// read only that component, red (i + j even) reads only black (old)
-// neighbours, so a workgroup stages the old field of its 64 x 8 tile with a
-// 2-point halo in LDS, computes the red values of the tile and its 1-point
-// ring, then the black values of the tile from them, and writes the tile:
-// the reference's colours 2a+1, 2a+2 (stag_mg_solver.f90:373-382, the 2D
+// 2D fused red-black sweep: both face components in one launch, a workgroup
+// per (tile, component), for visc_type -1 / 1; one component a launch for the
+// types that couple them.  In 2D a component's red points (i + j even) read
+// only its black (old) neighbours, so a workgroup stages the old field of its
+// tile with a 2-point halo in LDS, computes the red values of the tile and its
+// 1-point ring, then the black values of the tile from them, and writes the
+// tile: the reference's colours 2a+1, 2a+2 (stag_mg_solver.f90:373-382, the 2D
 // stag_applyop / stag_mg_update arithmetic term by term), in one pass over
 // memory instead of four colour passes.
 template <typename T, int A, int VISC>
@@ -980,11 +980,12 @@ struct Stag2RB {
   struct Args {
     T omega, dxsqinv;
     const T *rhs, *alpha, *beta, *bnd;  // bnd: node beta (2D edges)
-    const T *g1, *gamma;                // visc_type 2, 3: the other component; gamma
+    const T *g1, *gamma;                // visc_type 2, 3, -2, -3: the other component; gamma
   };
   struct Coef {
     T av, rhs, B0, B1, E10, E11;
-    T G[4];  // visc_type 2: the four cross-term values; 3: their sum in G[0]
+    T G[4];  // visc_type 2, -2, -3: the four cross-term values; 3: their sum in G[0]
+    T C0, Cm;  // visc_type -3: gamma of the point's two cells
   };
   static __device__ __forceinline__ Coef load(const Grid &g, int i, int j, const Args &a) {
     Coef c;
@@ -992,13 +993,26 @@ struct Stag2RB {
     const long p = i + sy * j;
     c.av = a.alpha[p];
     c.rhs = a.rhs[p];
-    if (VISC == -1) {
-      const long pma = (A == 0) ? wrapc(i - 1, g.n[0]) + sy * j : i + sy * wrapc(j - 1, g.n[1]);
-      const long p1p = (A == 0) ? i + sy * wrapc(j + 1, g.n[1]) : wrapc(i + 1, g.n[0]) + sy * j;
+    if (VISC < 0) {
+      const int nx = g.n[0], ny = g.n[1];
+      const int ia = (A == 0) ? wrapc(i - 1, nx) : i, ja = (A == 1) ? wrapc(j - 1, ny) : j;
+      const long pma = ia + sy * ja;
+      const long p1p = (A == 0) ? i + sy * wrapc(j + 1, ny) : wrapc(i + 1, nx) + sy * j;
       c.B0 = a.beta[p];
       c.B1 = a.beta[pma];
       c.E10 = a.bnd[p];
       c.E11 = a.bnd[p1p];
+      if (VISC < -1) {
+        const long q1 = (A == 0) ? ia + sy * wrapc(j + 1, ny) : wrapc(i + 1, nx) + sy * ja;
+        c.G[0] = a.g1[p1p];
+        c.G[1] = a.g1[p];
+        c.G[2] = a.g1[q1];
+        c.G[3] = a.g1[pma];
+      }
+      if (VISC == -3) {
+        c.C0 = a.gamma[p];
+        c.Cm = a.gamma[pma];
+      }
     } else if (VISC >= 2) {
       // pma: -1 along A; p1p: +1 along the other direction; q1: both shifts
       const int nx = g.n[0], ny = g.n[1];
@@ -1046,6 +1060,21 @@ struct Stag2RB {
       L = F * (c.av + ((T)14.0 * b * onethird + (T)2.0 * cg) * dxsqinv) -
           ((fpa + fpma) * (fourthirds * b + cg) + (fp1p + fp1m) * b + c.G[0] * (onethird * b + cg)) * dxsqinv;
       fac = c.av + ((T)(14.0 / 3.0) * b + (T)2.0 * cg) * dxsqinv;
+    } else if (VISC == -2) {
+      T dg = (T)2.0 * c.B0 + (T)2.0 * c.B1 + c.E11 + c.E10;
+      T off = (T)2.0 * fpa * c.B0 + (T)2.0 * fpma * c.B1 + fp1p * c.E11 + fp1m * c.E10 + c.G[0] * c.E11 -
+              c.G[1] * c.E10 - c.G[2] * c.E11 + c.G[3] * c.E10;
+      L = F * (c.av + dg * dxsqinv) - off * dxsqinv;
+      fac = c.av + ((T)2.0 * c.B0 + (T)2.0 * c.B1 + c.E10 + c.E11) * dxsqinv;
+    } else if (VISC == -3) {
+      const T fourthirds = (T)(4.0 / 3.0), twothirds = (T)(2.0 / 3.0);
+      const T B0 = c.B0, B1 = c.B1, E10 = c.E10, E11 = c.E11, G0 = c.C0, Gm = c.Cm;
+      T dg = fourthirds * B0 + G0 + fourthirds * B1 + Gm + E11 + E10;
+      T off = fpa * (fourthirds * B0 + G0) + fpma * (fourthirds * B1 + Gm) + fp1p * E11 + fp1m * E10 +
+              c.G[0] * (E11 - twothirds * B0 + G0) - c.G[1] * (E10 - twothirds * B0 + G0) -
+              c.G[2] * (E11 - twothirds * B1 + Gm) + c.G[3] * (E10 - twothirds * B1 + Gm);
+      L = F * (c.av + dg * dxsqinv) - off * dxsqinv;
+      fac = c.av + (fourthirds * B0 + G0 + fourthirds * B1 + Gm + E10 + E11) * dxsqinv;
     } else {
       T dg = c.B0 + c.B1 + c.E11 + c.E10;
       T off = fpa * c.B0 + fpma * c.B1 + fp1p * c.E11 + fp1m * c.E10;
@@ -1087,49 +1116,68 @@ struct CC2RB {
   }
 };
 
-constexpr int TX2D = 64, TY2D = 8;
+// A workgroup owns a 32 x 16 tile, an x-pair a thread.  Everything it reads --
+// the old field with a 2-point halo, the coefficients of the thread's pair and
+// of its red point of the 1-point ring -- is loaded at once, then red and black
+// are updated in LDS: a 2D level is a few hundred KB in the caches, and a
+// launch's time is the number of times that it waits for them (128^2 FP64, two
+// components: 4.5 us with the coefficients loaded after the field, 4.0 so).
+// Tiles may hang over the box: points beyond it are loaded from their periodic
+// images and not stored, so any even extents do.
+constexpr int TX2D = 32, TY2D = 16;
+constexpr int HX2D = TX2D + 4, HY2D = TY2D + 4, RX2D = TX2D + 2, RY2D = TY2D + 2;
 
 template <typename T, typename P>
 __device__ __forceinline__ void tile2d(const Grid &g, int ntx, int tile, const T *__restrict__ pin,
-                                       T *__restrict__ pout, const typename P::Args &args,
-                                       T (*sp)[TX2D + 4], T (*sr)[TX2D + 2]) {
-  constexpr int HX2 = TX2D + 4, HY2 = TY2D + 4, RX2 = TX2D + 2, RY2 = TY2D + 2;
+                                       T *__restrict__ pout, const typename P::Args &args, T *f) {
   const int bx = tile % ntx, by = tile / ntx;
   const int i0 = bx * TX2D, j0 = by * TY2D;
   const int nx = g.n[0], ny = g.n[1];
   const long sy = g.s[1];
   const int tid = threadIdx.x;
-  // the old field of the tile and a 2-point halo (a null input: zeros)
-  for (int q = tid; q < HY2 * HX2; q += 256) {
-    const int r = q / HX2, c = q - r * HX2;
-    sp[r][c] = pin ? pin[wrapc(i0 - 2 + c, nx) + sy * wrapc(j0 - 2 + r, ny)] : (T)0;
+  constexpr int NPT = HX2D * HY2D, NLD = (NPT + 255) / 256;
+  T old[NLD];
+#pragma unroll
+  for (int n = 0; n < NLD; n++) {
+    const int q = tid + 256 * n < NPT ? tid + 256 * n : NPT - 1;
+    const int x = q % HX2D, y = q / HX2D;
+    // a null input stands for a field of zeros
+    old[n] = pin ? pin[wrap_any(i0 - 2 + x, nx) + sy * wrap_any(j0 - 2 + y, ny)] : (T)0;
   }
-  __syncthreads();
-  // red points of the tile and its 1-point ring: region (row, rr) is point
-  // (i0 + rr - 1, j0 + row - 1); red where i + j is even (i0 is even)
-  constexpr int NRED2 = RY2 * (RX2 / 2);
-  for (int q = tid; q < NRED2; q += 256) {
-    const int row = q / (RX2 / 2), cc = q - row * (RX2 / 2);
-    const int jj = j0 + row - 1;
-    const int rr = 2 * cc + ((jj + 1) & 1);
-    const int hr = row + 1, hc = rr + 1;
-    const typename P::Coef c = P::load(g, wrapc(i0 + rr - 1, nx), wrapc(jj, ny), args);
-    const T xp = sp[hr][hc + 1], xm = sp[hr][hc - 1], yp = sp[hr + 1][hc], ym = sp[hr - 1][hc];
-    sr[row][rr] = P::update(c, sp[hr][hc], xp, xm, yp, ym, args);
+  const int m = tid % (TX2D / 2), row = tid / (TX2D / 2), i = i0 + 2 * m, j = j0 + row;
+  const int iw = wrap_any(i, nx), jw = wrap_any(j, ny);
+  const typename P::Coef c0 = P::load(g, iw, jw, args), c1 = P::load(g, iw + 1, jw, args);
+  // red points of the ring: two end rows, one end point of each inner row
+  constexpr int RING = 2 * (RX2D / 2) + TY2D;
+  typename P::Coef cr;
+  int ring = -1;
+  if (tid < RING) {
+    const bool end = tid < 2 * (RX2D / 2);
+    const int ry = end ? (tid < RX2D / 2 ? 0 : RY2D - 1) : 1 + tid - 2 * (RX2D / 2);
+    const int jr = j0 - 1 + ry;
+    const int par = (jr + 1) & 1;  // red: i + j even, i = i0 - 1 + rx
+    const int rx = end ? 2 * (tid % (RX2D / 2)) + par : (par ? RX2D - 1 : 0);
+    ring = (rx + 1) + HX2D * (ry + 1);
+    cr = P::load(g, wrap_any(i0 - 1 + rx, nx), wrap_any(jr, ny), args);
   }
+#pragma unroll
+  for (int n = 0; n < NLD; n++)
+    if (tid + 256 * n < NPT) f[tid + 256 * n] = old[n];
   __syncthreads();
-  // black: thread t owns the pair (2m, 2m+1) of tile row r
-  const int pr = tid / (TX2D / 2), pm = tid - pr * (TX2D / 2);
-  const int j = j0 + pr;
-  const bool first_red = (j & 1) == 0;  // column 2m is red when j is even
-  const int bc = 2 * pm + (first_red ? 1 : 0), rc = 2 * pm + (first_red ? 0 : 1);
-  const typename P::Coef cb = P::load(g, i0 + bc, j, args);
-  const int rrow = pr + 1, rcol = bc + 1;
-  const T xp = sr[rrow][rcol + 1], xm = sr[rrow][rcol - 1], yp = sr[rrow + 1][rcol], ym = sr[rrow - 1][rcol];
-  const T F = sp[pr + 2][bc + 2];
-  const T v = P::update(cb, F, xp, xm, yp, ym, args);
-  const T r = sr[rrow][rc + 1];
-  st2(pout, i0 + 2 * pm + sy * j, first_red ? r : v, first_red ? v : r);
+  auto update = [&](int q, const typename P::Coef &c) -> T {
+    return P::update(c, f[q], f[q + 1], f[q - 1], f[q + HX2D], f[q - HX2D], args);
+  };
+  // red, in place: red points read black neighbours only
+  const bool first_red = (j & 1) == 0;  // the pair's first point is red when j is even
+  const int at = (2 * m + 2) + HX2D * (row + 2);
+  const int qr = at + (first_red ? 0 : 1);
+  const T r = update(qr, first_red ? c0 : c1);
+  f[qr] = r;
+  if (ring >= 0) f[ring] = update(ring, cr);
+  __syncthreads();
+  if (i >= nx || j >= ny) return;
+  const T v = update(at + (first_red ? 1 : 0), first_red ? c1 : c0);
+  st2(pout, i + sy * j, first_red ? r : v, first_red ? v : r);
 }
 
 template <typename T, typename P0, typename P1>
@@ -1137,37 +1185,40 @@ __global__ void __launch_bounds__(256) k_rb_tile2d(Grid g, int ntx, int ntiles, 
                                                    T *__restrict__ pout0, const T *__restrict__ pin1,
                                                    T *__restrict__ pout1, typename P0::Args a0,
                                                    typename P1::Args a1) {
-  __shared__ T sp[TY2D + 4][TX2D + 4];
-  __shared__ T sr[TY2D + 2][TX2D + 2];
+  __shared__ T f[HX2D * HY2D];
   const int nslots = 2 * ntiles, w = blockIdx.x;
   int slot = w;
   if (nslots % 8 == 0) slot = (w % 8) * (nslots / 8) + w / 8;
   const int tile = slot / 2, comp = slot - 2 * tile;
   if (comp == 0)
-    tile2d<T, P0>(g, ntx, tile, pin0, pout0, a0, sp, sr);
+    tile2d<T, P0>(g, ntx, tile, pin0, pout0, a0, f);
   else
-    tile2d<T, P1>(g, ntx, tile, pin1, pout1, a1, sp, sr);
+    tile2d<T, P1>(g, ntx, tile, pin1, pout1, a1, f);
 }
 
 template <typename T, typename P>
 __global__ void __launch_bounds__(256) k_rb_tile2d1(Grid g, int ntx, int ntiles, const T *__restrict__ pin,
                                                     T *__restrict__ pout, typename P::Args a) {
-  __shared__ T sp[TY2D + 4][TX2D + 4];
-  __shared__ T sr[TY2D + 2][TX2D + 2];
+  __shared__ T f[HX2D * HY2D];
   const int w = blockIdx.x;
   const int tile = (ntiles % 8 == 0) ? (w % 8) * (ntiles / 8) + w / 8 : w;
-  tile2d<T, P>(g, ntx, tile, pin, pout, a, sp, sr);
+  tile2d<T, P>(g, ntx, tile, pin, pout, a, f);
 }
 
 }  // namespace
 
-// 2D levels are fused from 16 workgroups on (a lower threshold than 3D's:
-// a 2D level has no z-slabs to spread, and its colour passes are as short)
-static int min_tiles_2d(int min_tiles) { return min_tiles < 16 ? min_tiles : 16; }
+static int tiles2d(const Grid &g) { return ((g.n[0] + TX2D - 1) / TX2D) * ((g.n[1] + TY2D - 1) / TY2D); }
+
+// Every 2D level of even extents is swept in tiles: one launch (visc_type -1,
+// 1) or one a component against two colour launches a component, each as long
+// as a tile's (192 x 160 FP64 visc_type -2, a component: 4.15 against 2 x 3.2 us).
+// min_tiles above its default of 64 workgroups counts them, two components'.
+static bool even2d(const Grid &g, int min_tiles) {
+  return g.dim == 2 && g.n[0] % 2 == 0 && g.n[1] % 2 == 0 && (min_tiles <= 64 || 2 * tiles2d(g) >= min_tiles);
+}
 
 bool fused_rb2d_ok(const Grid &g, int visc, int min_tiles) {
-  return g.dim == 2 && (visc == -1 || visc == 1) && g.n[0] % TX2D == 0 && g.n[1] % TY2D == 0 &&
-         2 * (g.n[0] / TX2D) * (g.n[1] / TY2D) >= min_tiles_2d(min_tiles);
+  return (visc == -1 || visc == 1) && even2d(g, min_tiles);
 }
 
 template <typename T, int VISC>
@@ -1177,7 +1228,7 @@ static void launch_rb2d(hipStream_t s, const Grid &g, T omega, T dxsqinv, T *con
   using P1 = Stag2RB<T, 1, VISC>;
   typename P0::Args a0 = {omega, dxsqinv, rhs[0], K.alpha[0], K.beta, K.bed[0]};
   typename P1::Args a1 = {omega, dxsqinv, rhs[1], K.alpha[1], K.beta, K.bed[0]};
-  const int ntx = g.n[0] / TX2D, ntiles = ntx * (g.n[1] / TY2D);
+  const int ntx = (g.n[0] + TX2D - 1) / TX2D, ntiles = tiles2d(g);
   LaunchEvents *ev = launch_events();
   hipExtLaunchKernelGGL((k_rb_tile2d<T, P0, P1>), dim3(2 * ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx,
                         ntiles, pin[0], pout[0], pin[1], pout[1], a0, a1);
@@ -1204,8 +1255,7 @@ template void launch_stag_rb2d<float>(hipStream_t, const Grid &, int, float, flo
                                       float *const[3], const StagCoef<float> &, bool);
 
 bool fused_rb2d_comp_ok(const Grid &g, int visc, int min_tiles) {
-  return g.dim == 2 && (visc == 2 || visc == 3) && g.n[0] % TX2D == 0 && g.n[1] % TY2D == 0 &&
-         2 * (g.n[0] / TX2D) * (g.n[1] / TY2D) >= min_tiles_2d(min_tiles);
+  return (visc < -1 || visc > 1) && even2d(g, min_tiles);
 }
 
 template <typename T, int A, int VISC>
@@ -1221,7 +1271,7 @@ static void launch_rb2d_one(hipStream_t s, const Grid &g, T omega, const T *pin,
   a.bnd = K.bed[0];
   a.g1 = g1;
   a.gamma = K.gamma;
-  const int ntx = g.n[0] / TX2D, ntiles = ntx * (g.n[1] / TY2D);
+  const int ntx = (g.n[0] + TX2D - 1) / TX2D, ntiles = tiles2d(g);
   LaunchEvents *ev = launch_events();
   hipExtLaunchKernelGGL((k_rb_tile2d1<T, P>), dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx, ntiles,
                         pin, pout, a);
@@ -1236,13 +1286,15 @@ void launch_stag_rb2d_comp(hipStream_t s, const Grid &g, int visc, int a, T omeg
     report_error("launch_stag_rb2d_comp: level not eligible");
     return;
   }
-  if (visc == 2) {
-    if (a == 0) launch_rb2d_one<T, 0, 2>(s, g, omega, pin, pout, rhs, K, other);
-    else launch_rb2d_one<T, 1, 2>(s, g, omega, pin, pout, rhs, K, other);
-  } else {
-    if (a == 0) launch_rb2d_one<T, 0, 3>(s, g, omega, pin, pout, rhs, K, other);
-    else launch_rb2d_one<T, 1, 3>(s, g, omega, pin, pout, rhs, K, other);
-  }
+  auto go = [&](auto v) {
+    constexpr int V = decltype(v)::value;
+    if (a == 0) launch_rb2d_one<T, 0, V>(s, g, omega, pin, pout, rhs, K, other);
+    else launch_rb2d_one<T, 1, V>(s, g, omega, pin, pout, rhs, K, other);
+  };
+  if (visc == 2) go(Const<2>());
+  else if (visc == 3) go(Const<3>());
+  else if (visc == -2) go(Const<-2>());
+  else go(Const<-3>());
 }
 template void launch_stag_rb2d_comp<double>(hipStream_t, const Grid &, int, int, double, const double *, double *,
                                             const double *, const StagCoef<double> &, const double *);
@@ -1250,8 +1302,7 @@ template void launch_stag_rb2d_comp<float>(hipStream_t, const Grid &, int, int, 
                                            const float *, const StagCoef<float> &, const float *);
 
 bool cc_rb2d_ok(const Grid &g, int min_tiles) {
-  return g.dim == 2 && g.n[0] % TX2D == 0 && g.n[1] % TY2D == 0 &&
-         (g.n[0] / TX2D) * (g.n[1] / TY2D) >= min_tiles_2d(min_tiles);
+  return even2d(g, min_tiles);
 }
 
 template <typename T>
@@ -1265,7 +1316,7 @@ void launch_cc_rb2d(hipStream_t s, const Grid &g, const T *pin, T *pout, const T
   args.rhs = rhs;
   args.ax = a[0];
   args.ay = a[1];
-  const int ntx = g.n[0] / TX2D, ntiles = ntx * (g.n[1] / TY2D);
+  const int ntx = (g.n[0] + TX2D - 1) / TX2D, ntiles = tiles2d(g);
   LaunchEvents *ev = launch_events();
   hipExtLaunchKernelGGL((k_rb_tile2d1<T, CC2RB<T>>), dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx,
                         ntiles, pin, pout, args);
