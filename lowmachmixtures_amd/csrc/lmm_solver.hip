@@ -85,6 +85,8 @@ struct lmm_ctx {
   double *partial2 = nullptr;  // per-block cell sums
   double *scal = nullptr;      // device scalars
   double *hscal = nullptr;     // pinned host mirror
+  std::vector<int> armed;      // its entries that launched reductions have yet to write
+  bool armed_twice = false;    // one of them by two launches
   double *ainv[3] = {nullptr, nullptr, nullptr};
   double *alpha_theta[3] = {nullptr, nullptr, nullptr};
   double *scaled_beta = nullptr, *scaled_gamma = nullptr, *scaled_bed[3] = {nullptr, nullptr, nullptr};
@@ -392,6 +394,7 @@ static void free_levels(std::vector<SLevel<T>> &S, std::vector<CLevel<T>> &CC, b
 }
 
 static void drop_graphs(lmm_ctx *c) {
+  if (!c->pgraphs.empty() && c->stream) hipStreamSynchronize(c->stream);
   for (auto &kv : c->pgraphs)
     if (kv.second.exec) hipGraphExecDestroy(kv.second.exec);
   c->pgraphs.clear();
@@ -567,20 +570,77 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
   }
 }
 
+// ------------------------- results on the host ---------------------------
+
+// The pinned host mirror of a device scalar slot: the reductions write both,
+// so the host reads a result without a copy.
+static double *mirror(lmm_ctx *c, const double *slot) { return c->hscal + (slot - c->scal); }
+
+// A signalling NaN, which no arithmetic returns: an entry of the mirror that
+// holds it has not been written yet.
+static constexpr uint64_t UNWRITTEN = 0x7ff4a5a5c3c3f00dull;
+
+// Marks the n entries from h on that the reduction launched next will write.
+static constexpr int FINALIZE_WRITES[3] = {1, 3, 4};  // by launch_finalize's op
+static double *arm(lmm_ctx *c, double *h, int n) {
+  for (int q = 0; q < n; q++) {
+    const int e = (int)(h + q - c->hscal);
+    if (std::find(c->armed.begin(), c->armed.end(), e) != c->armed.end()) c->armed_twice = true;
+    else c->armed.push_back(e);
+    __atomic_store_n(reinterpret_cast<uint64_t *>(h + q), UNWRITTEN, __ATOMIC_RELAXED);
+  }
+  return h;
+}
+
+// Waits until every armed entry is written.  Each entry is written whole and
+// tells by itself that it is there, so no order between them is needed; a
+// wait that finds nothing armed or an entry armed twice (the first write
+// would pass for the second), or that a millisecond does not end, is a stream
+// synchronisation, which also is what reports errors.  A solve of a small box
+// waits some 80 times: the synchronisation's signal and wake-up cost 5 to 20 us
+// more a time than the poll (10 launches and the wait 58 against 36 us).
+static void wait_results(lmm_ctx *c) {
+  bool all = !c->armed.empty() && !c->armed_twice;
+  if (all) {
+    const auto t0 = std::chrono::steady_clock::now();
+    size_t n = 0;
+    for (unsigned spin = 1;; spin++) {
+      while (n < c->armed.size() &&
+             __atomic_load_n(reinterpret_cast<const uint64_t *>(c->hscal + c->armed[n]), __ATOMIC_ACQUIRE) != UNWRITTEN)
+        n++;
+      if (n == c->armed.size()) break;
+      __builtin_ia32_pause();
+      if (spin % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) {
+        all = false;
+        break;
+      }
+    }
+  }
+  if (!all) hipStreamSynchronize(c->stream);
+  c->armed.clear();
+  c->armed_twice = false;
+}
+
+// n results from device slot dev on, from their host mirror
+static void fetch(lmm_ctx *c, const double *dev, int n, double *host) {
+  wait_results(c);
+  memcpy(host, mirror(c, dev), sizeof(double) * n);
+}
+
 // max |rhs - L phi| per component on level 0 (FP64), synchronises
 static void resid_inf(lmm_ctx *c, SLevel<double> &L, double *const phi[3], double *const rhs[3], double out[3]) {
   launch_stag_residual<double>(c->stream, L.g, c->prm.visc_type, phi, rhs, L.res, L.K());
   launch_face_maxabs(c->stream, L.g, L.res, c->partial);
-  launch_finalize_max(c->stream, L.g, c->partial, c->hscal);
-  hipStreamSynchronize(c->stream);
+  launch_finalize_max(c->stream, L.g, c->partial, arm(c, c->hscal, 3));
+  wait_results(c);
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
 }
 
 // max |rhs| per component on level 0 (FP64), synchronises
 static void rhs_inf(lmm_ctx *c, SLevel<double> &L, double *const rhs[3], double out[3]) {
   launch_face_maxabs(c->stream, L.g, rhs, c->partial);
-  launch_finalize_max(c->stream, L.g, c->partial, c->hscal);
-  hipStreamSynchronize(c->stream);
+  launch_finalize_max(c->stream, L.g, c->partial, arm(c, c->hscal, 3));
+  wait_results(c);
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
 }
 
@@ -734,8 +794,8 @@ static double cell_inf(lmm_ctx *c, const Grid &g, const double *a) {
   g1.dim = 1;  // the face reduction over one array
   const double *r[3] = {a, nullptr, nullptr};
   launch_face_maxabs(c->stream, g1, r, c->partial);
-  launch_finalize_max(c->stream, g1, c->partial, c->hscal);
-  hipStreamSynchronize(c->stream);
+  launch_finalize_max(c->stream, g1, c->partial, arm(c, c->hscal, 3));
+  wait_results(c);
   return c->hscal[0];
 }
 
@@ -989,16 +1049,12 @@ static void precon64(lmm_ctx *c, const SV &b, const SV &x, double theta_alpha) {
 
 // ------------------------- reductions to host ----------------------------
 
-// The pinned host mirror of a device scalar slot: the reductions write both,
-// so the host reads a result after a stream synchronisation without a copy
-// (fetch).
-static double *mirror(lmm_ctx *c, const double *slot) { return c->hscal + (slot - c->scal); }
-
 // dot / norm of Stokes vectors; result in a device slot and its host mirror
 static void stokes_dot_dev(lmm_ctx *c, const double *a, const double *b, double *slot, int op) {
   ProfScope ps(c, "krylov", (double)c->g.N * 8.0 * 2 * (c->g.dim + 1));
   launch_stokes_dot(c->stream, c->g, a, b, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, slot, op, c->prm.p_norm_weight, mirror(c, slot));
+  launch_finalize(c->stream, c->g, c->partial, slot, op, c->prm.p_norm_weight,
+                  arm(c, mirror(c, slot), FINALIZE_WRITES[op]));
 }
 
 // Modified Gram-Schmidt of w against V_0..V_{i-1} (gmres.f90:338-358): the
@@ -1025,14 +1081,9 @@ static void mgs(lmm_ctx *c, const VF &Vk, int i, double *H, double *nrm) {
     ProfScope ps(c, "krylov", (double)L * 8.0 * (last ? 3 : 4));
     launch_axmy_dot(s, c->g, c->w, Vk(k - 1), H + k - 1, last ? nullptr : Vk(k), c->partial);
     double *slot = last ? nrm : H + k;
-    launch_finalize(s, c->g, c->partial, slot, last ? 1 : 0, c->prm.p_norm_weight, mirror(c, slot));
+    launch_finalize(s, c->g, c->partial, slot, last ? 1 : 0, c->prm.p_norm_weight,
+                    arm(c, mirror(c, slot), FINALIZE_WRITES[last ? 1 : 0]));
   }
-}
-
-// n results from device slot dev on, from their host mirror
-static void fetch(lmm_ctx *c, const double *dev, int n, double *host) {
-  hipStreamSynchronize(c->stream);
-  memcpy(host, mirror(c, dev), sizeof(double) * n);
 }
 
 // ------------------------- GMRES host scalars (gmres.f90:517-605) --------
@@ -1261,6 +1312,7 @@ static void precon32(lmm_ctx *c, const double *v64, float *z32, double theta_alp
   if (graphs_usable(c)) {
     lmm_ctx::PGraph &e = c->pgraphs[z32];
     if (e.exec && e.theta != theta_alpha) {
+      hipStreamSynchronize(s);  // its last launch has returned (results may have been polled for)
       hipGraphExecDestroy(e.exec);
       e.exec = nullptr;
     }
@@ -1319,7 +1371,7 @@ static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, 
     ProfScope ps(c, "krylov", (double)L * 8.0 * (nv + 1));
     launch_cgs_dots(s, g, c->w, vl, nv, c->partial_cgs);
     launch_cgs_finalize(s, g, c->partial_cgs, nv, sig2.data() + k0, c->prm.p_norm_weight, dslot + k0, cslot + k0,
-                        mirror(c, dslot + k0));
+                        arm(c, mirror(c, dslot + k0), nv));
   }
   for (int k0 = 0; k0 < i; k0 += CGS_MAXV) {
     const int nv = std::min(CGS_MAXV, i - k0);
@@ -1329,7 +1381,7 @@ static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, 
     ProfScope ps(c, "krylov", (double)L * (8.0 * (nv + 2) + (last ? 4.0 : 0.0)));
     launch_cgs_update(s, g, (k0 == 0) ? c->w : Vk(i), vl, nv, cslot + k0, Vk(i), last ? c->b32 : nullptr, c->partial);
   }
-  launch_finalize(s, g, c->partial, nslot, 1, c->prm.p_norm_weight, mirror(c, nslot));
+  launch_finalize(s, g, c->partial, nslot, 1, c->prm.p_norm_weight, arm(c, mirror(c, nslot), FINALIZE_WRITES[1]));
   double hb[3 * 32 + 3];
   fetch(c, dslot, 83, hb);
   for (int k = 0; k < i; k++) hs.h(k + 1, i) = sig[i - 1] * sig[k] * hb[k];
@@ -2275,7 +2327,8 @@ int lmm_stag_inner_prod(lmm_ctx *c, lmm_field *const m1[3], lmm_field *const m2[
   launch_fill<double>(c->stream, c->r + dim * N, N, 0.0);
   launch_fill<double>(c->stream, c->w + dim * N, N, 0.0);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
+                  arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
   double h[4];
   fetch(c, c->scal + 4100, 4, h);
   for (int d = 0; d < 3; d++) prod_val[d] = d < dim ? h[d] : 0.0;
@@ -2291,7 +2344,8 @@ int lmm_cc_inner_prod(lmm_ctx *c, lmm_field *m1, lmm_field *m2, double *prod_val
   hipMemcpyAsync(c->r + dim * N, m1->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   hipMemcpyAsync(c->w + dim * N, m2->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
+                  arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
   double h[4];
   fetch(c, c->scal + 4100, 4, h);
   *prod_val = h[3];
@@ -3873,7 +3927,8 @@ int lmm_cnn_error_reduction(lmm_cnn *nn, lmm_field *const alpha_fc[3], lmm_field
     learned_stage(c, b.u, b.p, z.u, z.p);
     err2(slot + 4);
     double h[6];
-    fetch(c, c->scal + 4300, 6, h);
+    hipStreamSynchronize(c->stream);
+    memcpy(h, slot, sizeof h);
     const double n0 = h[0] + h[1];
     sp += std::sqrt((h[2] + h[3]) / n0);
     sl += std::sqrt((h[4] + h[5]) / n0);
