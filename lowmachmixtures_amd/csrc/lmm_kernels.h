@@ -183,6 +183,21 @@ template <typename T>
 void launch_cc_prolong_add(hipStream_t s, const Grid &gf, T *fine, const T *coarse);
 
 // ---- elementwise / conversions ----
+// FP32 copies of l.n arrays of n values each
+constexpr int CONVERT_MAX = 8;
+struct ConvertList {
+  float *dst[CONVERT_MAX];
+  const double *src[CONVERT_MAX];
+  int n;
+  void add(float *d, const double *s) {
+    dst[n] = d;
+    src[n++] = s;
+  }
+};
+void launch_convert_list(hipStream_t s, const ConvertList &l, long n);
+// zeros into a level's face arrays
+template <typename T>
+void launch_zero_faces(hipStream_t s, const Grid &g, T *const x[3]);
 template <typename T>
 void launch_fill(hipStream_t s, T *x, long n, T v);
 template <typename T>

@@ -192,30 +192,29 @@ void launch_stag_restrict(hipStream_t s, const Grid &gc, T *const fine[3], T *co
                      p3(coarse));
 }
 
-template <typename T, int D, int A>
-__global__ void __launch_bounds__(256) k_stag_prolong(Grid gf, Grid gc, T *fine, const T *__restrict__ C) {
-  long t = xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= gf.N) return;
-  prolong_at<T, D, A>(gf, gc, fine, C, t);
-}
-
 // Two x-neighbours (2m, 2m+1) per thread: one vector load and store of the
-// fine pair; each point gets prolong_value as in the one-point kernel, and
-// for the x-face component the even and odd point no longer sit in
-// alternate lanes of a wave.
-template <typename T, int A>
-__global__ void __launch_bounds__(256) k_stag_prolong2(Grid gf, Grid gc, T *fine, const T *__restrict__ C) {
+// fine pair; for the x-face component the even and odd point do not sit in
+// alternate lanes of a wave.  Every component in one launch (blockIdx.y): on
+// the levels that take this path a launch's time is its latency (32^3 FP64
+// 3 x 4.4 us, 4.8 in one; 128^2 2 x 4.4, 4.6).  A level that has a coarser one
+// has even extents, so the points always pair.
+template <typename T, int D>
+__global__ void __launch_bounds__(256) k_stag_prolong2(Grid gf, Grid gc, Ptr3<T> fine, Ptr3<T> coarse) {
   const long t = xcd_block() * blockDim.x + threadIdx.x;
   if (2 * t >= gf.N) return;
   int c0[3];
   decode(gf, 2 * t, c0[0], c0[1], c0[2]);
   const int c1[3] = {c0[0] + 1, c0[1], c0[2]};
   const long p = 2 * t;
-  T f0, f1;
-  ld2(fine, p, f0, f1);
-  f0 = prolong_value<T, 3, A>(gf, gc, C, c0, f0);
-  f1 = prolong_value<T, 3, A>(gf, gc, C, c1, f1);
-  st2(fine, p, f0, f1);
+  with_component<D>((int)blockIdx.y, [&](auto A) {
+    T *const f = fine.c[A.value];
+    const T *const C = coarse.c[A.value];
+    T f0, f1;
+    ld2(f, p, f0, f1);
+    f0 = prolong_value<T, D, A.value>(gf, gc, C, c0, f0);
+    f1 = prolong_value<T, D, A.value>(gf, gc, C, c1, f1);
+    st2(f, p, f0, f1);
+  });
 }
 
 // Tiled prolongation of the three face components (3D; fine level with x a
@@ -283,32 +282,19 @@ __global__ void __launch_bounds__(256) k_stag_prolong_tiled(Grid gf, Grid gc, Pt
 template <typename T>
 void launch_stag_prolong(hipStream_t s, const Grid &gf, T *const fine[3], T *const coarse[3]) {
   Grid gc = coarsen(gf);
-  dim3 grid(nblk(gf.N));
+  Ptr3<T> F, Cc;
+  for (int d = 0; d < 3; d++) {
+    F.c[d] = d < gf.dim ? fine[d] : nullptr;
+    Cc.c[d] = d < gf.dim ? coarse[d] : nullptr;
+  }
   if (gf.dim == 3 && tuning().prolong_tiled && gf.n[0] % PTX == 0 && gf.n[1] % PTY == 0 && gf.n[2] % PTZ == 0) {
     const int ntx = gf.n[0] / PTX, nty = gf.n[1] / PTY, ntz = gf.n[2] / PTZ;
-    Ptr3<T> F, Cc;
-    for (int d = 0; d < 3; d++) {
-      F.c[d] = fine[d];
-      Cc.c[d] = coarse[d];
-    }
     LAUNCH(k_stag_prolong_tiled<T>, dim3(ntx * nty * ntz, 3), dim3(256), 0, s, gf, gc, F, Cc, ntx, nty);
     return;
   }
-  if (gf.dim == 3 && gf.n[0] % 2 == 0) {
-    dim3 grid2(nblk(gf.N / 2));
-    LAUNCH((k_stag_prolong2<T, 0>), grid2, dim3(TPB), 0, s, gf, gc, fine[0], coarse[0]);
-    LAUNCH((k_stag_prolong2<T, 1>), grid2, dim3(TPB), 0, s, gf, gc, fine[1], coarse[1]);
-    LAUNCH((k_stag_prolong2<T, 2>), grid2, dim3(TPB), 0, s, gf, gc, fine[2], coarse[2]);
-    return;
-  }
-  if (gf.dim == 2) {
-    LAUNCH((k_stag_prolong<T, 2, 0>), grid, dim3(TPB), 0, s, gf, gc, fine[0], coarse[0]);
-    LAUNCH((k_stag_prolong<T, 2, 1>), grid, dim3(TPB), 0, s, gf, gc, fine[1], coarse[1]);
-  } else {
-    LAUNCH((k_stag_prolong<T, 3, 0>), grid, dim3(TPB), 0, s, gf, gc, fine[0], coarse[0]);
-    LAUNCH((k_stag_prolong<T, 3, 1>), grid, dim3(TPB), 0, s, gf, gc, fine[1], coarse[1]);
-    LAUNCH((k_stag_prolong<T, 3, 2>), grid, dim3(TPB), 0, s, gf, gc, fine[2], coarse[2]);
-  }
+  const dim3 grid(nblk(gf.N / 2), gf.dim);
+  if (gf.dim == 3) LAUNCH((k_stag_prolong2<T, 3>), grid, dim3(TPB), 0, s, gf, gc, F, Cc);
+  else LAUNCH((k_stag_prolong2<T, 2>), grid, dim3(TPB), 0, s, gf, gc, F, Cc);
 }
 
 template <typename T>
@@ -485,6 +471,31 @@ __global__ void k_fill(T *x, long n, T v) {
 template <typename T>
 void launch_fill(hipStream_t s, T *x, long n, T v) {
   if (n > 0) LAUNCH(k_fill<T>, dim3(nblk(n)), dim3(TPB), 0, s, x, n, v);
+}
+
+// zeros into the face arrays of a level, one launch
+template <typename T>
+__global__ void k_zero_faces(Ptr3<T> x, long n) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  T *const p = blockIdx.y == 0 ? x.c[0] : (blockIdx.y == 1 ? x.c[1] : x.c[2]);
+  p[t] = (T)0;
+}
+template <typename T>
+void launch_zero_faces(hipStream_t s, const Grid &g, T *const x[3]) {
+  Ptr3<T> X;
+  for (int d = 0; d < 3; d++) X.c[d] = d < g.dim ? x[d] : nullptr;
+  LAUNCH(k_zero_faces<T>, dim3(nblk(g.N), g.dim), dim3(TPB), 0, s, X, g.N);
+}
+
+// FP32 copies of up to CONVERT_MAX arrays of n values, one launch: a level's
+// coefficient arrays were a launch each, of 1.8 us on most levels.
+__global__ void k_convert_list(ConvertList l, long n) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) l.dst[blockIdx.y][t] = (float)l.src[blockIdx.y][t];
+}
+void launch_convert_list(hipStream_t s, const ConvertList &l, long n) {
+  if (n > 0 && l.n > 0) LAUNCH(k_convert_list, dim3(nblk(n), l.n), dim3(TPB), 0, s, l, n);
 }
 
 template <typename T>
@@ -1652,6 +1663,7 @@ void launch_stoch_m_force(hipStream_t s, const Grid &g, double *const force[3], 
                                         T *const[3], const StagCoef<T> &);                                   \
   template void launch_stag_restrict<T>(hipStream_t, const Grid &, T *const[3], T *const[3], int);           \
   template void launch_stag_prolong<T>(hipStream_t, const Grid &, T *const[3], T *const[3]);                 \
+  template void launch_zero_faces<T>(hipStream_t, const Grid &, T *const[3]);                                \
   template void launch_cc_restrict<T>(hipStream_t, const Grid &, const T *, T *);                            \
   template void launch_edge_restrict<T>(hipStream_t, const Grid &, T *const[3], T *const[3]);                \
   template void launch_nodal_restrict<T>(hipStream_t, const Grid &, const T *, T *);                         \

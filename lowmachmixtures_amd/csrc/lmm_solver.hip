@@ -472,16 +472,20 @@ static void prepare_coefs(lmm_ctx *c, const CoefIn &in, double theta_alpha, doub
   if (need32) {
     auto &S32 = c->s32;
     for (int n = 0; n < c->nl_s; n++) {
-      long N = S[n].g.N;
-      for (int d = 0; d < dim; d++) launch_convert<float, double>(s, S32[n].alpha[d], S[n].alpha[d], N);
-      launch_convert<float, double>(s, S32[n].beta, S[n].beta, N);
-      launch_convert<float, double>(s, S32[n].gamma, S[n].gamma, N);
-      for (int e = 0; e < ne_of(dim); e++) launch_convert<float, double>(s, S32[n].bed[e], S[n].bed[e], N);
+      ConvertList l = {};
+      for (int d = 0; d < dim; d++) l.add(S32[n].alpha[d], S[n].alpha[d]);
+      l.add(S32[n].beta, S[n].beta);
+      l.add(S32[n].gamma, S[n].gamma);
+      for (int e = 0; e < ne_of(dim); e++) l.add(S32[n].bed[e], S[n].bed[e]);
+      launch_convert_list(s, l, S[n].g.N);
     }
     auto &C = c->c64;
     auto &C32 = c->c32;
-    for (int n = 0; n < c->nl_c; n++)
-      for (int d = 0; d < dim; d++) launch_convert<float, double>(s, C32[n].a[d], C[n].a[d], C[n].g.N);
+    for (int n = 0; n < c->nl_c; n++) {
+      ConvertList l = {};
+      for (int d = 0; d < dim; d++) l.add(C32[n].a[d], C[n].a[d]);
+      launch_convert_list(s, l, C[n].g.N);
+    }
   }
 }
 
@@ -683,8 +687,7 @@ static void stag_vcycles(lmm_ctx *c, std::vector<SLevel<T>> &S, T *const phi0[3]
     }
     if (allzero) {
       // stag_mg_solver.f90:276-306 returns the guess: zero here
-      if (phi_zero)
-        for (int d = 0; d < dim; d++) launch_fill<T>(c->stream, phi0[d], S[0].g.N, (T)0);
+      if (phi_zero) launch_zero_faces<T>(c->stream, S[0].g, phi0);
       return;
     }
     if (anyzero)
@@ -723,12 +726,12 @@ static void stag_vcycles(lmm_ctx *c, std::vector<SLevel<T>> &S, T *const phi0[3]
   };
   const bool zero0 = phi_zero && !need_check && takes_zeros(0);
   if (phi_zero && !zero0)
-    for (int d = 0; d < dim; d++) launch_fill<T>(c->stream, phi0[d], S[0].g.N, (T)0);
+    launch_zero_faces<T>(c->stream, S[0].g, phi0);
   auto zin = [&](int n, int vc) { return (n == 0) ? (zero0 && vc == 1) : takes_zeros(n); };
   for (int vc = 1; vc <= p.stag_mg_max_vcycles; vc++) {
     for (int n = 1; n < nc; n++)
       if (!takes_zeros(n))
-        for (int d = 0; d < dim; d++) launch_fill<T>(c->stream, S[n].phi[d], S[n].g.N, (T)0);
+        launch_zero_faces<T>(c->stream, S[n].g, S[n].phi);
     for (int n = 0; n < std::min(nc, nl - 1); n++) {
       T *const *ph = (n == 0) ? phi0 : S[n].phi;
       T *const *rh = (n == 0) ? rhs0 : S[n].rhs;
@@ -1007,7 +1010,7 @@ static void learned_stage(lmm_ctx *c, float *const vu[3], const float *vp, float
   cnn_forward(nn->net, 1, gn, nn->xin, nn->yout);
   launch_cnn_unpack(s, gc, nn->yout, nn->ss, c->partial, nn->ss + 2, S[lc].phi, C[lc].phi);
   for (int n = lc - 1; n >= 1; n--) {
-    for (int d = 0; d < 3; d++) launch_fill<float>(s, S[n].phi[d], S[n].g.N, 0.f);
+    launch_zero_faces<float>(s, S[n].g, S[n].phi);
     launch_fill<float>(s, C[n].phi, C[n].g.N, 0.f);
     launch_stag_prolong<float>(s, S[n].g, S[n].phi, S[n + 1].phi);
     launch_cc_prolong_add<float>(s, C[n].g, C[n].phi, C[n + 1].phi);
@@ -2299,7 +2302,7 @@ int lmm_diffusive_m_fluxdiv(lmm_ctx *c, lmm_field *m_update[3], lmm_field *const
   for (int d = 0; d < dim; d++)
     if (m_update[d]->d == umac[d]->d) return set_err(c, LMM_ERR_ARG, "m_update and umac must be distinct fields");
   auto &L = c->s64[0];
-  for (int d = 0; d < dim; d++) launch_fill<double>(c->stream, L.alpha[d], c->g.N, 0.0);
+  launch_zero_faces<double>(c->stream, c->g, L.alpha);
   L.beta = eta->d;
   L.gamma = kappa->d;
   for (int e = 0; e < ne_of(dim); e++) L.bed[e] = eta_ed[e]->d;
