@@ -333,7 +333,9 @@ void launch_eta(hipStream_t s, const Grid &g, double *eta, double *kappa, const 
 
 // ---- fluctuating and diffusive fluxes ----
 // width > 0: the scaled fluxes are written to work (2*(dim + 2*ne)*N doubles,
-// ne = 1 in 2D, 3 in 3D) and filtered (multifab_filter) before the divergence
+// ne = 1 in 2D, 3 in 3D) and filtered (multifab_filter) before the divergence;
+// weights: the nstages stages' on the host, passed by value
+constexpr int STOCH_MAX_STAGES = 8;
 void launch_stoch_m_force(hipStream_t s, const Grid &g, double *const force[3], const double *Wcc,
                           double *const Wed[3], int nstages, const double *weights, long stage_stride_cc,
                           long stage_stride_ed, const double *eta, double *const eta_ed[3],

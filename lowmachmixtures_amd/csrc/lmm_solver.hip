@@ -99,7 +99,6 @@ struct lmm_ctx {
   // stochastic noise held by the context (init_m_stochastic)
   int n_rngs = 0;
   double *Wcc = nullptr, *Wed = nullptr;
-  double *dweights = nullptr;
   double *stoch_work = nullptr;  // filtered stochastic fluxes (filtering_width > 0)
   // Smoother kernels: fused red-black sweeps on levels with at least
   // fused_min_tiles workgroups in a launch (32^3 and up), colour-by-colour kernels
@@ -1726,7 +1725,7 @@ int lmm_ctx_destroy(lmm_ctx *c) {
   for (void *p : {(void *)c->partial, (void *)c->partial_cgs, (void *)c->partial2, (void *)c->scal, (void *)c->scaled_beta,
                   (void *)c->scaled_gamma, (void *)c->V, (void *)c->r, (void *)c->w, (void *)c->tmp, (void *)c->b,
                   (void *)c->x, (void *)c->Z32, (void *)c->b32, (void *)c->mac_rhs, (void *)c->phi_cc,
-                  (void *)c->mac_rhs32, (void *)c->Wcc, (void *)c->Wed, (void *)c->dweights, (void *)c->stoch_work,
+                  (void *)c->mac_rhs32, (void *)c->Wcc, (void *)c->Wed, (void *)c->stoch_work,
                   (void *)c->Wmass, (void *)c->dweights_mass, (void *)c->sp_work, (void *)c->iw})
     dfree(p);
   for (int d = 0; d < 3; d++) {
@@ -2526,13 +2525,11 @@ int lmm_init_m_stochastic(lmm_ctx *c, int n_rngs) {
   if (!c || n_rngs < 1 || n_rngs > 8) return LMM_ERR_ARG;
   dfree(c->Wcc);
   dfree(c->Wed);
-  dfree(c->dweights);
   long N = c->g.N;
   int dim = c->g.dim, ne = ne_of(dim);
   c->Wcc = dalloc<double>(c->stream, (long)n_rngs * dim * N);
   c->Wed = dalloc<double>(c->stream, (long)n_rngs * ne * 2 * N);
-  c->dweights = dalloc<double>(c->stream, 8);
-  if (!c->Wcc || !c->Wed || !c->dweights) return set_err(c, LMM_ERR_NOMEM, "noise allocation failed");
+  if (!c->Wcc || !c->Wed) return set_err(c, LMM_ERR_NOMEM, "noise allocation failed");
   c->n_rngs = n_rngs;
   return LMM_OK;
 }
@@ -2606,7 +2603,7 @@ int lmm_field_fill_normal(lmm_field *f, uint64_t seed, uint64_t step, int64_t v0
 }
 
 static int stoch_common(lmm_ctx *c, lmm_field *force[3], const double *Wcc, double *const Wed[3], int nst,
-                        const double *w_dev, long scc, long sed, lmm_field *eta, lmm_field *const eta_ed[3],
+                        const double *weights, long scc, long sed, lmm_field *eta, lmm_field *const eta_ed[3],
                         lmm_field *temp, lmm_field *const temp_ed[3], double variance) {
   int dim = c->g.dim, ne = ne_of(dim);
   int rc;
@@ -2627,7 +2624,7 @@ static int stoch_common(lmm_ctx *c, lmm_field *force[3], const double *Wcc, doub
     c->stoch_work = dalloc<double>(c->stream, 2L * (dim + 2 * ne) * c->g.N);
     if (!c->stoch_work) return set_err(c, LMM_ERR_NOMEM, "cannot allocate the filtering work arrays");
   }
-  launch_stoch_m_force(c->stream, c->g, f, Wcc, Wed, nst, w_dev, scc, sed, eta->d, ee, temp->d, te, variance, width,
+  launch_stoch_m_force(c->stream, c->g, f, Wcc, Wed, nst, weights, scc, sed, eta->d, ee, temp->d, te, variance, width,
                        c->stoch_work);
   return finish(c);
 }
@@ -2642,12 +2639,9 @@ int lmm_stochastic_m_fluxdiv(lmm_ctx *c, lmm_field *stoch_m_force[3], lmm_field 
   for (int d = 0; d < dim; d++) dv *= c->g.dx;
   // stochastic_m_fluxdiv.f90:135: product(dx(n,1:dm))
   double variance = std::sqrt(variance_coef_mom * 2.0 * k_B / (dv * dt));
-  memcpy(c->hscal, weights, sizeof(double) * c->n_rngs);
-  HIPCHK(c, hipMemcpyAsync(c->dweights, c->hscal, sizeof(double) * c->n_rngs, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   double *Wed[3] = {nullptr, nullptr, nullptr};
   for (int e = 0; e < ne; e++) Wed[e] = c->Wed + (long)e * 2 * N;
-  return stoch_common(c, stoch_m_force, c->Wcc, Wed, c->n_rngs, c->dweights, (long)dim * N, (long)ne * 2 * N, eta,
+  return stoch_common(c, stoch_m_force, c->Wcc, Wed, c->n_rngs, weights, (long)dim * N, (long)ne * 2 * N, eta,
                       eta_ed, temperature, temperature_ed, variance);
 }
 
@@ -2663,10 +2657,8 @@ int lmm_stoch_m_force(lmm_ctx *c, lmm_field *stoch_m_force[3], lmm_field *W_cc, 
     if (!field_ok(c, W_ed[e], ek + e, 2)) return set_err(c, LMM_ERR_ARG, "W_ed[%d] must have 2 components", e);
     Wed[e] = W_ed[e]->d;
   }
-  c->hscal[0] = 1.0;
-  HIPCHK(c, hipMemcpyAsync(c->scal + 4200, c->hscal, sizeof(double), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return stoch_common(c, stoch_m_force, W_cc->d, Wed, 1, c->scal + 4200, 0, 0, eta, eta_ed, temperature,
+  const double one = 1.0;
+  return stoch_common(c, stoch_m_force, W_cc->d, Wed, 1, &one, 0, 0, eta, eta_ed, temperature,
                       temperature_ed, variance);
 }
 
