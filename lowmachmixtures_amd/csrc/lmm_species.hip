@@ -797,12 +797,13 @@ __global__ void __launch_bounds__(STPB) k_sp_div(Grid g, const double *flux, dou
 // halo), passed through LDS, and applied to the faces of all directions; the
 // cell below in z reads it from memory beside the cell's own, when it is in L2.
 // The next column is loaded before the current one is applied.  128^3, four
-// species, two noise stages: 595 us face by face, 427 here (1.6 GB that a face
-// pass cannot do without, 3.7 TB/s; 64 x 4 tiles, with a larger halo, 481);
-// 384 x 320, eight species: 124 us in a pass and a divergence per flux, 49 for
-// this and the common divergence.  The noise is read and flux_total written
-// past the caches (427 against 447 us); the two fluxes are not, the divergence
-// reads them next.
+// species, two noise stages: 595 us face by face, 427 to 471 here from run to
+// run (1.6 GB that a face pass cannot do without, 3.4 to 3.7 TB/s; 64 x 4
+// tiles, with a larger halo, 481 where these took 446); 384 x 320, eight
+// species: 124 us in a pass and a divergence per flux, 49 for this and the
+// common divergence.  The noise is read and flux_total written past the caches
+// (427 against 447 us in one run); the two fluxes are not, the divergence reads
+// them next.
 constexpr int FTX = 32, FTY = 8;
 constexpr int FHX = FTX + 1, FHY = FTY + 1;  // with the lower halo column and row
 constexpr int FHALO = FTX + FTY;
