@@ -22,6 +22,7 @@
 #include "lmm_cnn.h"
 #include "lmm_species.h"
 #include "lmm_kernels.h"
+#include "lmm_results.h"
 
 using namespace lmm;
 
@@ -85,8 +86,11 @@ struct lmm_ctx {
   double *partial2 = nullptr;  // per-block cell sums
   double *scal = nullptr;      // device scalars
   double *hscal = nullptr;     // pinned host mirror
-  std::vector<int> armed;      // its entries that launched reductions have yet to write
-  bool armed_twice = false;    // one of them by two launches
+  HostResults results;         // its entries that launched reductions have yet to write
+  // microseconds a wait polls for them before it synchronises the stream;
+  // LMM_POLL_US in the environment changes it, 0: always synchronise
+  long poll_us = 1000;
+  bool lost = false;           // a result did not arrive: the call in progress fails
   double *ainv[3] = {nullptr, nullptr, nullptr};
   double *alpha_theta[3] = {nullptr, nullptr, nullptr};
   double *scaled_beta = nullptr, *scaled_gamma = nullptr, *scaled_bed[3] = {nullptr, nullptr, nullptr};
@@ -579,72 +583,48 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
 // so the host reads a result without a copy.
 static double *mirror(lmm_ctx *c, const double *slot) { return c->hscal + (slot - c->scal); }
 
-// A signalling NaN, which no arithmetic returns: an entry of the mirror that
-// holds it has not been written yet.
-static constexpr uint64_t UNWRITTEN = 0x7ff4a5a5c3c3f00dull;
-
 // Marks the n entries from h on that the reduction launched next will write.
 static constexpr int FINALIZE_WRITES[3] = {1, 3, 4};  // by launch_finalize's op
-static double *arm(lmm_ctx *c, double *h, int n) {
-  for (int q = 0; q < n; q++) {
-    const int e = (int)(h + q - c->hscal);
-    if (std::find(c->armed.begin(), c->armed.end(), e) != c->armed.end()) c->armed_twice = true;
-    else c->armed.push_back(e);
-    __atomic_store_n(reinterpret_cast<uint64_t *>(h + q), UNWRITTEN, __ATOMIC_RELAXED);
-  }
-  return h;
-}
+static double *arm(lmm_ctx *c, double *h, int n) { return c->results.arm(h, n); }
 
-// Waits until every armed entry is written.  Each entry is written whole and
-// tells by itself that it is there, so no order between them is needed; a
-// wait that finds nothing armed or an entry armed twice (the first write
-// would pass for the second), or that a millisecond does not end, is a stream
-// synchronisation, which also is what reports errors.  A solve of a small box
-// waits some 80 times: the synchronisation's signal and wake-up cost 5 to 20 us
-// more a time than the poll (10 launches and the wait 58 against 36 us).
-static void wait_results(lmm_ctx *c) {
-  bool all = !c->armed.empty() && !c->armed_twice;
-  if (all) {
-    const auto t0 = std::chrono::steady_clock::now();
-    size_t n = 0;
-    for (unsigned spin = 1;; spin++) {
-      while (n < c->armed.size() &&
-             __atomic_load_n(reinterpret_cast<const uint64_t *>(c->hscal + c->armed[n]), __ATOMIC_ACQUIRE) != UNWRITTEN)
-        n++;
-      if (n == c->armed.size()) break;
-      __builtin_ia32_pause();
-      if (spin % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) {
-        all = false;
-        break;
-      }
-    }
-  }
-  if (!all) hipStreamSynchronize(c->stream);
-  c->armed.clear();
-  c->armed_twice = false;
+// Waits until every armed entry is written (HostResults::wait).  A solve of a
+// small box waits some 80 times: a stream synchronisation's signal and wake-up
+// cost 5 to 20 us more a time than the poll (10 launches and the wait 58
+// against 36 us).  false: the device failed or a reduction never ran, so what
+// the caller would read is no result; the call in progress returns an error.
+static bool wait_results(lmm_ctx *c) {
+  hipError_t e = hipSuccess;
+  if (c->results.wait(c->poll_us, [&] { return (e = hipStreamSynchronize(c->stream)) == hipSuccess; })) return !c->lost;
+  c->lost = true;
+  set_err(c, LMM_ERR_DEVICE, "waiting for a reduction: %s",
+          e != hipSuccess ? hipGetErrorString(e) : first_error()[0] ? first_error() : "its result was not written");
+  return false;
 }
 
 // n results from device slot dev on, from their host mirror
-static void fetch(lmm_ctx *c, const double *dev, int n, double *host) {
-  wait_results(c);
+static bool fetch(lmm_ctx *c, const double *dev, int n, double *host) {
+  if (!wait_results(c)) return false;
   memcpy(host, mirror(c, dev), sizeof(double) * n);
+  return true;
 }
 
 // max |rhs - L phi| per component on level 0 (FP64), synchronises
-static void resid_inf(lmm_ctx *c, SLevel<double> &L, double *const phi[3], double *const rhs[3], double out[3]) {
+static bool resid_inf(lmm_ctx *c, SLevel<double> &L, double *const phi[3], double *const rhs[3], double out[3]) {
   launch_stag_residual<double>(c->stream, L.g, c->prm.visc_type, phi, rhs, L.res, L.K());
   launch_face_maxabs(c->stream, L.g, L.res, c->partial);
   launch_finalize_max(c->stream, L.g, c->partial, arm(c, c->hscal, 3));
-  wait_results(c);
+  if (!wait_results(c)) return false;
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
+  return true;
 }
 
 // max |rhs| per component on level 0 (FP64), synchronises
-static void rhs_inf(lmm_ctx *c, SLevel<double> &L, double *const rhs[3], double out[3]) {
+static bool rhs_inf(lmm_ctx *c, SLevel<double> &L, double *const rhs[3], double out[3]) {
   launch_face_maxabs(c->stream, L.g, rhs, c->partial);
   launch_finalize_max(c->stream, L.g, c->partial, arm(c, c->hscal, 3));
-  wait_results(c);
+  if (!wait_results(c)) return false;
   for (int d = 0; d < 3; d++) out[d] = c->hscal[d];
+  return true;
 }
 
 // One call of stag_mg_solver (stag_mg_solver.f90:37-868) on prepared levels.
@@ -675,8 +655,7 @@ static void stag_vcycles(lmm_ctx *c, std::vector<SLevel<T>> &S, T *const phi0[3]
     // With a zero guess (apply_precon zeroes x_u first, apply_precon.f90:88-90)
     // the initial residual L 0 - rhs is -rhs bit for bit, so max |rhs| is
     // taken without reading phi0, whose contents are not the guess.
-    if (phi_zero) rhs_inf(c, S[0], rhs0, resid0);
-    else resid_inf(c, S[0], phi0, rhs0, resid0);
+    if (!(phi_zero ? rhs_inf(c, S[0], rhs0, resid0) : resid_inf(c, S[0], phi0, rhs0, resid0))) return;
     bool allzero = true, anyzero = false;
     double mx = 0;
     for (int d = 0; d < dim; d++) {
@@ -775,7 +754,7 @@ static void stag_vcycles(lmm_ctx *c, std::vector<SLevel<T>> &S, T *const phi0[3]
     if constexpr (std::is_same<T, double>::value) {
      if (vc < p.stag_mg_max_vcycles) {
       double r[3];
-      resid_inf(c, S[0], phi0, rhs0, r);
+      if (!resid_inf(c, S[0], phi0, rhs0, r)) return;
       bool done = true;
       for (int d = 0; d < dim; d++)
         if (!(r[d] / resid0[d] < p.stag_mg_rel_tol)) done = false;
@@ -790,15 +769,16 @@ static void stag_vcycles(lmm_ctx *c, std::vector<SLevel<T>> &S, T *const phi0[3]
 // abs_eps of the cell-centred multigrid's stopping test (macproject.f90:423)
 static constexpr double CC_ABS_EPS = 1e-16;
 
-// max |a| over a cell array of grid g (FP64), synchronises
-static double cell_inf(lmm_ctx *c, const Grid &g, const double *a) {
+// out = max |a| over a cell array of grid g (FP64), synchronises
+static bool cell_inf(lmm_ctx *c, const Grid &g, const double *a, double &out) {
   Grid g1 = g;
   g1.dim = 1;  // the face reduction over one array
   const double *r[3] = {a, nullptr, nullptr};
   launch_face_maxabs(c->stream, g1, r, c->partial);
   launch_finalize_max(c->stream, g1, c->partial, arm(c, c->hscal, 3));
-  wait_results(c);
-  return c->hscal[0];
+  if (!wait_results(c)) return false;
+  out = c->hscal[0];
+  return true;
 }
 
 template <typename T>
@@ -826,7 +806,7 @@ static void cc_vcycles(lmm_ctx *c, std::vector<CLevel<T>> &C, T *phi0, const T *
   double bnorm = 0.0;
   if constexpr (std::is_same<T, double>::value) {
     if (check) {
-      bnorm = cell_inf(c, c->g, rhs0);
+      if (!cell_inf(c, c->g, rhs0, bnorm)) return;
       if (bnorm <= p.mg_rel_tol * bnorm || bnorm <= CC_ABS_EPS) {
         launch_fill<T>(c->stream, phi0, c->g.N, (T)0);
         return;
@@ -908,7 +888,8 @@ static void cc_vcycles(lmm_ctx *c, std::vector<CLevel<T>> &C, T *phi0, const T *
     if constexpr (std::is_same<T, double>::value) {
       if (check && cyc + 1 < p.mg_max_vcycles) {
         launch_cc_residual<T>(c->stream, C[0].g, phi0, rhs0, C[0].res, C[0].a);
-        const double r = cell_inf(c, c->g, C[0].res);
+        double r;
+        if (!cell_inf(c, c->g, C[0].res, r)) return;
         if (r <= p.mg_rel_tol * bnorm || r <= CC_ABS_EPS) break;
       }
     }
@@ -1205,7 +1186,7 @@ static int gmres_ref(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
   stokes_dot_dev(c, c->tmp, c->tmp, c->scal + 3000, 1);
   stokes_dot_dev(c, c->b, c->b, c->scal + 3004, 1);
   double hb[8];
-  fetch(c, c->scal + 3000, 8, hb);
+  if (!fetch(c, c->scal + 3000, 8, hb)) return LMM_ERR_DEVICE;
   double norm_pre_b = hb[0], norm_b = hb[4];
   info->norm_pre_rhs = norm_pre_b;
   info->norm_b = norm_b;
@@ -1222,7 +1203,7 @@ static int gmres_ref(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
     stokes_dot_dev(c, c->tmp, c->tmp, c->scal + 3008, 1);
     precon64(c, tmp, r, theta_alpha);
     stokes_dot_dev(c, c->r, c->r, c->scal + 3012, 1);
-    fetch(c, c->scal + 3008, 8, hb);
+    if (!fetch(c, c->scal + 3008, 8, hb)) return LMM_ERR_DEVICE;
     norm_resid_Stokes = hb[0];
     norm_resid = hb[4];
     if (iter == 0) norm_init_resid = norm_resid;
@@ -1260,7 +1241,7 @@ static int gmres_ref(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
       double *col = dH + (long)(m + 1) * (i - 1);
       mgs(c, Vk, i, col, col + i);
       launch_div_by(s, Vk(i), c->w, L, col + i);
-      fetch(c, dH + (long)(m + 1) * (i - 1), i + 1, &hs.h(1, i));
+      if (!fetch(c, dH + (long)(m + 1) * (i - 1), i + 1, &hs.h(1, i))) return LMM_ERR_DEVICE;
       if (hs.h(i + 1, i) == 0.0) {
         brk = true;
         break;
@@ -1359,7 +1340,7 @@ static void precon32(lmm_ctx *c, const double *v64, float *z32, double theta_alp
 // |V_i|, so H(i+1, i) = sig[i-1] |V_i| and sig[i] = 1/|V_i|.  Two passes over
 // the basis per step instead of 2i, and no separate normalisation pass.
 template <typename VF>
-static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, Hess &hs) {
+static bool cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, Hess &hs) {
   hipStream_t s = c->stream;
   const Grid &g = c->g;
   const long L = (long)(g.dim + 1) * g.N;
@@ -1385,11 +1366,12 @@ static void cgs_step(lmm_ctx *c, const VF &Vk, int i, std::vector<double> &sig, 
   }
   launch_finalize(s, g, c->partial, nslot, 1, c->prm.p_norm_weight, arm(c, mirror(c, nslot), FINALIZE_WRITES[1]));
   double hb[3 * 32 + 3];
-  fetch(c, dslot, 83, hb);
+  if (!fetch(c, dslot, 83, hb)) return false;
   for (int k = 0; k < i; k++) hs.h(k + 1, i) = sig[i - 1] * sig[k] * hb[k];
   const double nv = hb[80];
   hs.h(i + 1, i) = sig[i - 1] * nv;
   sig[i] = (nv > 0.0) ? 1.0 / nv : 0.0;
+  return true;
 }
 
 static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
@@ -1406,7 +1388,7 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
   double *dH = c->scal;
   double hb[8];
   stokes_dot_dev(c, c->b, c->b, c->scal + 3004, 1);
-  fetch(c, c->scal + 3004, 4, hb);
+  if (!fetch(c, c->scal + 3004, 4, hb)) return LMM_ERR_DEVICE;
   double norm_b = hb[0];
   info->norm_b = norm_b;
   info->norm_pre_rhs = 0.0;
@@ -1424,10 +1406,14 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
   c->learned_on = (p.precision == LMM_LEARNED && c->cnn != nullptr);
   c->learned_applied = 0;
   info->learned_fallback = 0;
+  auto lost = [&] {
+    c->learned_on = false;
+    return LMM_ERR_DEVICE;
+  };
   for (;;) {
     residual_dev(c, x, c->tmp);
     stokes_dot_dev(c, c->tmp, c->tmp, c->scal + 3008, 1);
-    fetch(c, c->scal + 3008, 4, hb);
+    if (!fetch(c, c->scal + 3008, 4, hb)) return lost();
     rnorm = hb[0];
     if (p.gmres_verbose >= 1) printf("lmm fgmres outer %d total %d |r|/|b| %.10e\n", iter, total_iter, rnorm / norm_b);
     if (rnorm <= p.gmres_rel_tol * norm_b || rnorm <= p.gmres_abs_tol) {
@@ -1453,7 +1439,7 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
         precon32(c, Vk(i - 1), Zk(i - 1), theta_alpha, attempt == 0 && b32_fresh);
         apply_matrix_z32(c, Zk(i - 1), w);
         if (c->flex_cgs) {
-          cgs_step(c, Vk, i, sig, hs);  // writes V(i) and its FP32 copy
+          if (!cgs_step(c, Vk, i, sig, hs)) return lost();  // writes V(i) and its FP32 copy
           b32_fresh = true;
         } else {
           double *col = dH + (long)(m + 1) * (i - 1), *sl = col + i;
@@ -1461,7 +1447,7 @@ static int gmres_flex(lmm_ctx *c, double theta_alpha, lmm_gmres_info *info) {
           if (c->fused_krylov) launch_div_by_f32(s, Vk(i), c->b32, c->w, L, sl);
           else launch_div_by(s, Vk(i), c->w, L, sl);
           b32_fresh = c->fused_krylov;
-          fetch(c, dH + (long)(m + 1) * (i - 1), i + 1, &hs.h(1, i));
+          if (!fetch(c, dH + (long)(m + 1) * (i - 1), i + 1, &hs.h(1, i))) return lost();
         }
         bool finite = true;
         for (int k = 1; k <= i + 1; k++) finite = finite && std::isfinite(hs.h(k, i));
@@ -1575,6 +1561,8 @@ static void apply_options(lmm_ctx *c, const lmm_kernel_options &o) {
   c->tune.prolong_tiled = (pt && pt[0] == '0') ? 0 : 1;
   const char *cs = getenv("LMM_COARSE_SPLIT");
   c->tune.coarse_split = (cs && cs[0] == '0') ? 0 : 1;
+  const char *po = getenv("LMM_POLL_US");
+  c->poll_us = po ? atol(po) : 1000;
   const char *r3 = getenv("LMM_RR_THREE");
   c->tune.rr_three = (r3 && r3[0] == '0') ? 0 : 1;
   c->precon_graph = o.precon_graph != 0;
@@ -2073,6 +2061,11 @@ double *lmm_field_device_ptr(lmm_field *f) { return f ? f->d : nullptr; }
 // ---------------- operators ----------------
 
 static int finish(lmm_ctx *c) {
+  if (c->lost) {  // the message is wait_results'
+    c->lost = false;
+    if (!c->defer_sync) hipStreamSynchronize(c->stream);
+    return LMM_ERR_DEVICE;
+  }
   if (c->defer_sync) {
     if (first_error()[0]) return set_err(c, LMM_ERR_DEVICE, "kernel %s", first_error());
     hipError_t e = hipGetLastError();
@@ -2332,7 +2325,7 @@ int lmm_stag_inner_prod(lmm_ctx *c, lmm_field *const m1[3], lmm_field *const m2[
   launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
                   arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
   double h[4];
-  fetch(c, c->scal + 4100, 4, h);
+  if (!fetch(c, c->scal + 4100, 4, h)) return finish(c);
   for (int d = 0; d < 3; d++) prod_val[d] = d < dim ? h[d] : 0.0;
   return finish(c);
 }
@@ -2349,7 +2342,7 @@ int lmm_cc_inner_prod(lmm_ctx *c, lmm_field *m1, lmm_field *m2, double *prod_val
   launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
                   arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
   double h[4];
-  fetch(c, c->scal + 4100, 4, h);
+  if (!fetch(c, c->scal + 4100, 4, h)) return finish(c);
   *prod_val = h[3];
   return finish(c);
 }
