@@ -158,7 +158,9 @@ const char *lmm_ctx_last_error(const lmm_ctx *ctx);
  * nothing; on = 0: off.  family: "stag_smooth_l0" / "cc_smooth_l0" (finest
  * level sweeps), "stag_smooth" / "cc_smooth" (coarser levels),
  * "stag_rb_fused", "stag_restrict_l0", "stag_restrict", "stag_rr_fused",
- * "stag_prolong", "stag_coarse", "cc_coarse", "apply_matrix", "krylov". */
+ * "stag_prolong", "stag_coarse", "cc_coarse", "apply_matrix", "krylov";
+ * "stag_sweep_<form>" / "cc_sweep_<form>" only count the fused sweeps' launches
+ * by form: brick4, brick8, march, march_pairs, march_narrow, plane, block, tile2d. */
 int lmm_ctx_set_profiling(lmm_ctx *ctx, int on);
 int lmm_ctx_kernel_stats(lmm_ctx *ctx, const char *family, int64_t *launches, double *total_ms,
                          double *algorithmic_bytes);

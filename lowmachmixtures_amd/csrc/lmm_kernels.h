@@ -26,9 +26,9 @@ struct Tuning {
   int rb_target = 768;  // workgroups the z-slab choice aims for (FP32; FP64 twice)
   int am_dz = 32;       // z depth of the operator's brick order (0: row order)
   int rb_prefetch = 0;  // FP32 fused sweep: load the next plane's coefficients one step ahead
-  // 3D levels up to this many cells sweep in bricks, and every one whose
-  // extents the marching tiles do not divide; 0: none do; -1: the measured rule
+  // 3D levels up to this many cells sweep in bricks; 0: none do; -1: the measured rule
   long rb_brick = -1;
+  int rb_brick_rows = 0;  // rows of a brick where it can have 8: 4 or 8; 0: the measured rule
   int rb_pairs = 2;     // FP32 three-component sweep: point pairs per thread (2: 64 x 16 tiles)
   int prolong_tiled = 1;  // 3D staggered prolongation from coarse values staged in LDS
   int coarse_split = 1;   // coarse staggered V-cycle: one workgroup per component (visc_type -1 / 1)
@@ -52,6 +52,10 @@ struct LaunchEvents {
   hipEvent_t start, stop;
 };
 LaunchEvents *launch_events();
+// The form of the fused sweep launched last on this thread: "brick4",
+// "brick8", "march" (64 x 8 tiles), "march_pairs" (64 x 16), "march_narrow"
+// (32 x 16), "plane", "block" or "tile2d".
+const char *&sweep_form();
 const char *first_error();
 void clear_first_error();
 // records a host-side launch error (first one wins) for the next status check
@@ -64,22 +68,19 @@ struct Faces {
 };
 
 // ---- staggered operator ----
-// Fused red-black sweep of one component (3D, visc_type -1, 1, 2, 3): reads
-// the old field from pin, writes the new one to pout (lmm_smooth.hip); the
-// form and the z-slab target come from tuning().  visc_type 2 and 3 read the
-// other components from cur (their state at this component's turn in the
-// colour order).
-// z-slab thickness for element size es (4 or 8 bytes) when one launch
-// sweeps ncomp components, 0: not eligible
-int fused_rb_tz(const Grid &g, int min_tiles, int es, int ncomp);
-bool fused_rb_ok(const Grid &g, int visc, int min_tiles);
+// Fused red-black sweep of one component (3D): reads the old field from pin,
+// writes the new one to pout (lmm_smooth.hip); the form and the z-slab target
+// come from tuning() and the element size es (4 or 8 bytes).  The coupled
+// visc_types read the other components from cur (their state at this
+// component's turn in the colour order).
+bool fused_rb_ok(const Grid &g, int visc, int min_tiles, int es);
 template <typename T>
 void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega, const T *pin, T *pout,
                           const T *rhs, const StagCoef<T> &K, int min_tiles, const T *const cur[3] = nullptr);
 // All three components of one fused sweep in one launch (3D, visc -1 / 1,
-// the paired plane-marching form); reads pin[a] (zero_in: a field of zeros,
+// the paired plane-marching form or bricks); reads pin[a] (zero_in: a field of zeros,
 // pin not read), writes pout[a].
-bool fused_rb3_ok(const Grid &g, int visc, int min_tiles);
+bool fused_rb3_ok(const Grid &g, int visc, int min_tiles, int es);
 template <typename T>
 void launch_stag_rb_fused3(hipStream_t s, const Grid &g, int visc, T omega, T *const pin[3], T *const pout[3],
                            T *const rhs[3], const StagCoef<T> &K, int min_tiles, bool zero_in);
@@ -111,9 +112,10 @@ template <typename T>
 bool launch_stag_resid_restrict(hipStream_t s, const Grid &g, const Grid &gc, int visc, T *const phi[3],
                                 T *const rhs[3], T *const crhs[3], const StagCoef<T> &K);
 // whether the fused sweeps take a null input as a field of zeros (the
-// paired plane-marching form does)
+// paired plane-marching form and the bricks do)
 bool fused_rb_takes_zeros();
 // The same fused sweep for the cell-centred red-black Gauss-Seidel (3D).
+bool cc_rb_ok(const Grid &g, int min_tiles, int es);
 template <typename T>
 void launch_cc_rb_fused(hipStream_t s, const Grid &g, const T *pin, T *pout, const T *rhs, T *const a[3],
                         int min_tiles);

@@ -323,7 +323,7 @@ __device__ __forceinline__ void st2(T *a, long p, T x0, T x1) {
 template <typename T, int A, int VISC>
 struct StagRB {
   static constexpr bool BRICK_ONLY = VISC < -1;  // the plane-marching forms are not built for it
-  static constexpr bool CROSS = VISC >= 2;
+  static constexpr bool BRICK8 = false;  // bricks of 8 rows: never chosen for one component
   struct Args {
     T omega, dxsqinv;
     const T *rhs, *alpha, *beta, *e1, *e2;
@@ -585,7 +585,7 @@ struct StagRB {
 // arithmetic of cc_apply / the red-black update of lmm_points.h.
 template <typename T>
 struct CCRB {
-  static constexpr bool BRICK_ONLY = false, CROSS = false;
+  static constexpr bool BRICK_ONLY = false, BRICK8 = true;
   struct Args {
     T inv;
     const T *rhs, *ax, *ay, *az;

@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(256) k_rb_block(Grid g, int nbx, int nby, int 
   }
 }
 
-// Brick form of the same sweep for small levels and for extents that the
+// Brick form of the same sweep for small levels and for some extents that the
 // plane-marching tiles do not divide: a workgroup owns a 32 x KY x 4 brick,
 // KY / 4 x-pairs a thread.  Everything the brick reads from memory -- the old
 // field with a 2-point halo, the coefficients of the thread's pair and of its
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(256) k_rb_block(Grid g, int nbx, int nby, int 
 // per plane, which is all the time of a level that fills the GPU only once.
 // The ring is computed again by the neighbours (1.7 updates per point at KY =
 // 4, 1.5 at 8), so the marching form, which streams, wins on large levels
-// (brick_level has both sides).
+// (brick_pays has both sides).
 // Bricks may hang over the box: points beyond it are loaded from their
 // periodic images and not stored.
 constexpr int KX = 32, KZ = 4;
@@ -658,29 +658,35 @@ inline Bricks bricks(const Grid &g, int ky) {
   return {nx, ny, nx * ny * ((g.n[2] + KZ - 1) / KZ)};
 }
 
-// Rows of a brick: 8 (two pairs a thread, a smaller share of ring points)
-// where that still makes 768 workgroups, three on a compute unit, else 4.
-// Sweep of ncomp components, 4 rows / 8 rows in us: 32^3 FP64 7.2 / 9.2, 64^3
-// FP64 15.8 / 14.0 (three components) and 8.2 / 9.1 (cell-centred), 128 x 96 x
-// 64 FP64 36.2 / 33.6 and 14.9 / 13.5, 128^3 FP32 visc_type 2 30.1 / 26.9.
-// visc_type 2 and 3 in FP64 hold so many cross terms that two pairs a thread
-// leave two waves a SIMD: 4 rows there (128 x 96 x 64 17.3 / 18.0, 192 x 128 x
-// 96 44.2 / 45.2).
-inline int brick_rows(const Grid &g, int ncomp, bool cross64 = false) {
-  return !cross64 && ncomp * bricks(g, 8).n >= 768 ? 8 : 4;
+// Rows of a brick of the three-component and of the cell-centred sweep: 8 (two
+// pairs a thread, a smaller share of ring points) where that still makes 768
+// workgroups, three on a compute unit, and hangs little further over the box,
+// else 4.  Sweep in us, 4 rows / 8 rows: three components 32^3 FP64 7.2 / 9.2,
+// 64^3 FP64 15.8 / 14.0, 128 x 96 x 64 FP64 38.4 / 34.6, 256 x 12 x 256 FP64
+// 37.2 / 43.2; cell-centred 64^3 FP64 8.2 / 9.1, 128 x 96 x 64 FP64 15.1 /
+// 13.4, 256 x 12 x 256 FP64 15.1 / 18.0.  The one-component staggered form takes
+// levels of at most 512 bricks (brick_pays) and has 4 rows.
+inline int brick_rows(const Grid &g, int ncomp) {
+  const int rows = tuning().rb_brick_rows;
+  if (rows == 4 || rows == 8) return rows;
+  const int n4 = bricks(g, 4).n, n8 = bricks(g, 8).n;
+  return ncomp * n8 >= 768 && 10 * n8 <= 5.5 * n4 ? 8 : 4;
 }
 
 // tx: the march's tile width (64, or 32 with 32 x 16 tiles); 0: the brick form
 template <typename T, typename P>
 void launch_rb(hipStream_t s, const Grid &g, int tz, int tx, const T *pin, T *pout, const typename P::Args &args) {
   if (tx == 0) {
-    const int ky = brick_rows(g, 1, P::CROSS && sizeof(T) == 8);
+    int ky = 4;
+    auto kern = k_rb_brick<T, P, 4>;
+    if constexpr (P::BRICK8)
+      if ((ky = brick_rows(g, 1)) == 8) kern = k_rb_brick<T, P, 8>;
     const Bricks b = bricks(g, ky);
     LaunchEvents *ev = launch_events();
-    auto kern = ky == 8 ? k_rb_brick<T, P, 8> : k_rb_brick<T, P, 4>;
     hipExtLaunchKernelGGL(kern, dim3(b.n), dim3(256), 0, s, ev->start, ev->stop, 0, g, b.nx, b.ny, b.n,
                           pin, pout, args);
     ev->start = ev->stop = nullptr;
+    sweep_form() = ky == 8 ? "brick8" : "brick4";
     post_launch(s, kBrickName);
     return;
   }
@@ -694,6 +700,7 @@ void launch_rb(hipStream_t s, const Grid &g, int tz, int tx, const T *pin, T *po
       const int nb = nbx * nby * nbz;
       hipLaunchKernelGGL((k_rb_block<T, P>), dim3(nb), dim3(256), 0, s, g, nbx, nby, nb, pin, pout, args, q[0], q[1],
                          q[2], q[3], q[4]);
+      sweep_form() = "block";
       post_launch(s, kBlockName);
       return;
     }
@@ -714,11 +721,13 @@ void launch_rb(hipStream_t s, const Grid &g, int tz, int tx, const T *pin, T *po
         hipLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args, q[0], q[1],
                            q[2], q[3], q[4]);
       }
+      sweep_form() = tx == FX2 ? "march_narrow" : "march";
       post_launch(s, kMarchName);
       return;
     }
     hipLaunchKernelGGL((k_rb_fused<T, P>), dim3(ntiles), dim3(256), 0, s, g, tz, ntx, nty, ntiles, pin, pout, args,
                        q[0], q[1], q[2], q[3], q[4]);
+    sweep_form() = "plane";
     post_launch(s, kFusedName);
   }
 }
@@ -933,6 +942,7 @@ void launch_stag_three(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz,
     hipExtLaunchKernelGGL(kern, dim3(3 * b.n), dim3(256), 0, s, ev->start, ev->stop, 0, g,
                           b.nx, b.ny, b.n, in, p3(pout), a0, a1, a2);
     ev->start = ev->stop = nullptr;
+    sweep_form() = ky == 8 ? "brick8" : "brick4";
     post_launch(s, kBrickName);
     return;
   }
@@ -962,6 +972,7 @@ void launch_stag_three(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz,
                           q0[4], q1[0], q1[1], q1[2], q1[3], q1[4], q2[0], q2[1], q2[2], q2[3], q2[4]);
   }
   ev->start = ev->stop = nullptr;
+  sweep_form() = tx == FX2 ? "march_narrow" : np == 2 ? "march_pairs" : "march";
   post_launch(s, kMarch3Name);
 }
 
@@ -1233,6 +1244,7 @@ static void launch_rb2d(hipStream_t s, const Grid &g, T omega, T dxsqinv, T *con
   hipExtLaunchKernelGGL((k_rb_tile2d<T, P0, P1>), dim3(2 * ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx,
                         ntiles, pin[0], pout[0], pin[1], pout[1], a0, a1);
   ev->start = ev->stop = nullptr;
+  sweep_form() = "tile2d";
   post_launch(s, "k_rb_tile2d");
 }
 
@@ -1276,6 +1288,7 @@ static void launch_rb2d_one(hipStream_t s, const Grid &g, T omega, const T *pin,
   hipExtLaunchKernelGGL((k_rb_tile2d1<T, P>), dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx, ntiles,
                         pin, pout, a);
   ev->start = ev->stop = nullptr;
+  sweep_form() = "tile2d";
   post_launch(s, "k_rb_tile2d1");
 }
 
@@ -1321,6 +1334,7 @@ void launch_cc_rb2d(hipStream_t s, const Grid &g, const T *pin, T *pout, const T
   hipExtLaunchKernelGGL((k_rb_tile2d1<T, CC2RB<T>>), dim3(ntiles), dim3(256), 0, s, ev->start, ev->stop, 0, g, ntx,
                         ntiles, pin, pout, args);
   ev->start = ev->stop = nullptr;
+  sweep_form() = "tile2d";
   post_launch(s, "k_rb_tile2d1");
 }
 template void launch_cc_rb2d<double>(hipStream_t, const Grid &, const double *, double *, const double *,
@@ -1358,6 +1372,11 @@ void launch_stag_one(hipStream_t s, const Grid &g, T omega, T dxsqinv, int tz, i
 
 }  // namespace
 
+const char *&sweep_form() {
+  static thread_local const char *form = "";
+  return form;
+}
+
 LaunchEvents *launch_events() {
   static thread_local LaunchEvents ev = {nullptr, nullptr};
   return &ev;
@@ -1374,31 +1393,55 @@ static int rb_target(int es) {
   return es == 8 ? 2 * t : t;
 }
 
-// Whether a level is swept in bricks: levels that are too small to stream,
-// and every level whose extents the plane-marching tiles do not divide (asked
-// after rb_tz), where the alternative is two colour passes a component.
-// min_tiles above its default of 64 workgroups counts bricks; at or below it
-// any level qualifies (one brick launch replaces two colour launches a
-// component).
-enum BrickUse { BRICK_THREE, BRICK_ONE, BRICK_CC };  // three components a launch, one, cell-centred
+// What one launch sweeps: the three components (visc_type -1 / 1), one
+// component, or the cell-centred field.
+enum SweepUse { SWEEP_THREE, SWEEP_ONE, SWEEP_CC };
+
+// Whether a level can be swept in bricks.  min_tiles above its default of 64
+// workgroups counts them; at or below it any level qualifies.
 static bool brick_ok(const Grid &g, int min_tiles, int ncomp) {
   return tuning().rb_variant == 2 && tuning().rb_brick != 0 && g.dim == 3 && g.n[0] >= 4 && g.n[1] >= 4 &&
          g.n[2] >= 4 && (min_tiles <= 64 || ncomp * bricks(g, 4).n >= min_tiles);
 }
-// The line between bricks and marching tiles.  Sweep in us, marching / brick:
-//   three components  FP64  64^3 16.8 / 14.0, 128x96x64 42.6 / 33.6, 192x128x96 95 / 102, 128^3 71 / 86
-//                     FP32  64^3 17.5 / 15.7, 128x96x64 31.3 / 25.7, 192x128x96 59 / 65, 128^3 42 / 59
-//   one (visc_type 2) FP64  64^3 11.3 / 9.1, 128^3 46.5 / 39.5, 192x192x128 92 / 93, 256^3 247 / 339
-//                     FP32  64^3 10.1 / 7.9, 128^3 28.7 / 26.9, 192x192x128 53 / 54, 256^3 167 / 198
-//   cell-centred      FP64  64^3 10.3 / 8.2, 128^3 36.8 / 30.5, 192x192x128 60 / 62, 256^3 200 / 241
-//                     FP32  64^3 9.5 / 7.3, 128x96x64 13.4 / 12.4, 128^3 20.7 / 23.5, 256^3 107 / 153
-static bool brick_level(const Grid &g, int min_tiles, int ncomp, BrickUse use, int es) {
-  const long most = tuning().rb_brick >= 0 ? tuning().rb_brick
-                    : use == BRICK_ONE     ? 4000000
-                    : use == BRICK_CC      ? (es == 8 ? 3000000 : 1200000)
-                                           : 1200000;
-  return g.N <= most && brick_ok(g, min_tiles, ncomp);
+// Whether bricks are the form to take for such a level; marches: the
+// plane-marching tiles divide it, otherwise the alternative is two colour
+// passes a component.  A brick that hangs over the box works on points that it
+// does not store, so beside the size it is the bricks' fill that draws the
+// line.  us a sweep of one level back to back (three: a third of it),
+// colour passes / march (- where its tiles do not divide) / bricks:
+//   three         FP64  64x32x32 6.0/3.6/2.9   64^3 7.6/5.4/4.5    128x96x64 15.8/14.2/11.5  192x128x96 41/31/34
+//                       36^3 5.9/-/3.1         80^3 10.5/-/9.8     224^3 240/182/186         24x256x256 28/-/26
+//                       8x64x64 5.8/-/3.4      8x128x128 5.8/-/8.0 16x128x128 7.5/-/8.2      8x256x256 10/-/26
+//                 FP32  64^3 8.6/5.2/3.9       128x96x64 11/9.9/8.1  16x128x128 8.3/-/6.7    16x256x256 13/-/20
+//   visc_type 2   FP64  32^3 5.9/9.0/6.8       64^3 7.6/10.0/8.2   48^3 6.2/-/8.1            128x96x64 13/22/16
+//                       112^3 24/-/30          128^3 33/45/37      8x128x128 5.9/-/12        16x256x256 17/-/37
+//                 FP32  32^3 6.2/9.1/6.5       64^3 9.1/9.8/7.6    48^3 7.4/-/7.5            128x96x64 12/15/12
+//   visc_type -2  FP64  32^3 6.2/-/7.4         64^3 8.3/-/9.4      128^3 46/-/52             192x128x96 51/-/61
+//                 FP32  32^3 7.2/-/7.0         64^3 9.0/-/8.4      128^3 28/-/32             192x128x96 31/-/36
+//   visc_type -3  FP64  32^3 6.1/-/7.7         64^3 8.6/-/9.9      128^3 49/-/65             FP32 128^3 30/-/35
+//   cell-centred  FP64  32^3 5.8/9.0/6.4       64^3 7.1/9.9/8.1    48^3 5.9/-/7.6            128^3 33/36/30
+//                       80^3 9.6/-/12          160^3 59/51/54      8x128x128 5.7/-/11        16x256x256 17/-/30
+//                 FP32  32^3 6.7/-/6.4         64^3 7.4/9.4/7.9    128^3 20/19/22            112^3 15/-/20
+// On the smallest levels every form is bound by its launches.  Bricks make
+// half as many there as the colour passes: one solve takes as long (visc_type
+// 2, -2, -3 32^3 within 5 %), sixteen on the four hardware queues 1 to 6 % less.
+static bool brick_pays(const Grid &g, SweepUse use, int visc, int es, bool marches) {
+  if (tuning().rb_brick > 0) return g.N <= tuning().rb_brick;
+  const long n4 = bricks(g, 4).n;
+  const double fill = (double)g.N / (n4 * (KX * 4 * KZ));
+  if (use == SWEEP_THREE)
+    return bricks(g, 8).n <= (es == 8 ? 400 : 700) || (fill >= 0.7 && (!marches || g.N <= 1200000));
+  if (n4 <= 128) return true;
+  if (use == SWEEP_ONE) return visc >= -1 && n4 <= 512 && fill >= 0.85;
+  return fill >= 0.85 && (g.N <= (es == 8 ? 3000000 : 1200000) || (es == 8 && !marches));
 }
+// Whether the one-component sweep of a level too large for bricks marches; the
+// colour passes, which ping-pong nothing, are the faster form below (visc_type
+// 2, us as above, colour / march: FP64 128^3 33 / 45, 192x192x128 77 / 90, 192^3
+// 119 / 121, 256^3 345 / 245; FP32 128^3 22 / 27, 192x192x128 43 / 48, 192^3 62 /
+// 79, 224^3 122 / 129, 256^3 205 / 166; visc_type 3 FP32 256x128x128 39 / 36,
+// elsewhere like 2).
+static bool march_pays(const Grid &g, int es) { return g.N > (es == 8 ? 6000000 : 8000000); }
 
 // Plane count per workgroup, or 0 when the level cannot use the fused
 // sweep.  The plane-marching forms take the thickest z-slab (at most 32
@@ -1422,53 +1465,52 @@ static int rb_tz(const Grid &g, int min_tiles, int es, int ncomp, int fx, int fy
   return tz;
 }
 
-// z-slab and tile width of a one-component fused sweep: 64 x 8 tiles, or (the
-// plane-marching form only) 32 x 16 tiles on levels 32 points wide.  nsweep
-// launches of this shape make one sweep (the staggered components one after
-// another, 1 for the cell-centred field); together they must reach min_tiles.
-static int rb1_shape(const Grid &g, int min_tiles, int es, int &tx, int nsweep = 1, BrickUse use = BRICK_CC) {
+// z-slab and tile width of a fused sweep of one array: bricks (width 0), 64 x 8
+// tiles, or (the plane-marching form only) 32 x 16 tiles on levels 32 points
+// wide; 0: the level is left to the colour kernels.  nsweep launches of this
+// shape make one sweep (the staggered components one after another, 1 for the
+// cell-centred field); together they must reach min_tiles.  min_tiles = 1 asks
+// for a fused sweep wherever one exists, whichever form is the faster.
+static int rb1_shape(const Grid &g, SweepUse use, int visc, int min_tiles, int es, int &tx) {
+  const int nsweep = use == SWEEP_ONE ? g.dim : 1;
+  const bool marches_visc = visc >= -1;
   tx = FX;
   if (tuning().rb_variant == 1) {
-    if (g.dim != 3 || g.n[0] % BX != 0 || g.n[1] % BY != 0 || g.n[2] % BZ != 0) return 0;
+    if (!marches_visc || g.dim != 3 || g.n[0] % BX != 0 || g.n[1] % BY != 0 || g.n[2] % BZ != 0) return 0;
     const int nb = (g.n[0] / BX) * (g.n[1] / BY) * (g.n[2] / BZ);
     return nsweep * nb >= min_tiles ? BZ : 0;
   }
-  if (brick_level(g, min_tiles, nsweep, use, es)) {
+  int tz = marches_visc ? rb_tz(g, min_tiles, es, 1, FX, FY, nsweep) : 0;
+  if (tuning().rb_variant != 2) return tz;
+  if (tz == 0 && marches_visc) {
+    tx = FX2;
+    tz = rb_tz(g, min_tiles, es, 1, FX2, FY2, nsweep);
+  }
+  const bool forced = min_tiles <= 1, bricks_ok = brick_ok(g, min_tiles, nsweep);
+  if (bricks_ok && (brick_pays(g, use, visc, es, tz > 0) || (forced && tz == 0))) {
     tx = 0;
     return KZ;
   }
-  int tz = rb_tz(g, min_tiles, es, 1, FX, FY, nsweep);
-  if (tz > 0 || tuning().rb_variant != 2) return tz;
-  tx = FX2;
-  tz = rb_tz(g, min_tiles, es, 1, FX2, FY2, nsweep);
-  if (tz > 0 || !brick_ok(g, min_tiles, nsweep)) return tz;
-  tx = 0;
-  return KZ;
+  if (use == SWEEP_ONE && (visc < -1 || visc > 1) && !forced && tuning().rb_brick < 0 && !march_pays(g, es)) return 0;
+  return tz;
 }
 
-int fused_rb_tz(const Grid &g, int min_tiles, int es, int ncomp) {
+bool cc_rb_ok(const Grid &g, int min_tiles, int es) {
   int tx;
-  if (ncomp == 1) return rb1_shape(g, min_tiles, es, tx);
-  if (tuning().rb_variant == 1) return rb1_shape(g, min_tiles, es, tx);
-  return rb_tz(g, min_tiles, es, ncomp, FX, FY);
+  return rb1_shape(g, SWEEP_CC, 0, min_tiles, es, tx) > 0;
 }
 
-bool fused_rb_ok(const Grid &g, int visc, int min_tiles) {
+bool fused_rb_ok(const Grid &g, int visc, int min_tiles, int es) {
   int tx;
-  if (visc < -1) return brick_ok(g, min_tiles, g.dim);
-  return (visc == -1 || visc == 1 || visc == 2 || visc == 3) && rb1_shape(g, min_tiles, 4, tx, g.dim, BRICK_ONE) > 0;
+  return rb1_shape(g, SWEEP_ONE, visc, min_tiles, es, tx) > 0;
 }
 
 template <typename T>
 void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega, const T *pin, T *pout,
                           const T *rhs, const StagCoef<T> &K, int min_tiles, const T *const cur[3]) {
   int tx = FX;
-  int tz = rb1_shape(g, min_tiles, sizeof(T), tx, g.dim, BRICK_ONE);
-  if (visc < -1) {
-    tx = 0;
-    tz = KZ;
-  }
-  if (tz <= 0 || !fused_rb_ok(g, visc, min_tiles) || (visc != 1 && visc != -1 && !cur)) {
+  const int tz = rb1_shape(g, SWEEP_ONE, visc, min_tiles, sizeof(T), tx);
+  if (tz <= 0 || (visc != 1 && visc != -1 && !cur)) {
     report_error("launch_stag_rb_fused: level not eligible");
     return;
   }
@@ -1492,30 +1534,25 @@ void launch_stag_rb_fused(hipStream_t s, const Grid &g, int visc, int a, T omega
 // 64 x 16 tiles, where tuning asks for them) and z-slab of the
 // three-component sweep; 0 when the level cannot use it
 static int rb3_shape(const Grid &g, int min_tiles, int es, int &tx, int &np) {
-  np = 1;
-  if (brick_level(g, min_tiles, 3, BRICK_THREE, es)) {
+  int tz = 0;
+  auto tiles = [&](int x, int y, int pairs) {
+    tx = x;
+    np = pairs;
+    return tz = rb_tz(g, min_tiles, es, 3, x, y * pairs);
+  };
+  // FP64 would need 80 KB of LDS per workgroup for two pairs a thread
+  if (!(tuning().rb_pairs == 2 && es == 4 && tiles(FX, FY, 2)) && !tiles(FX, FY, 1)) tiles(FX2, FY2, 1);
+  if (brick_ok(g, min_tiles, 3) && (brick_pays(g, SWEEP_THREE, -1, es, tz > 0) || (min_tiles <= 1 && tz == 0))) {
     tx = 0;
+    np = 1;
     return KZ;
   }
-  tx = FX;
-  np = 2;
-  if (tuning().rb_pairs == 2 && es == 4) {  // FP64 would need 80 KB of LDS per workgroup
-    const int tz2 = rb_tz(g, min_tiles, es, 3, FX, 2 * FY);
-    if (tz2 > 0) return tz2;
-  }
-  np = 1;
-  int tz = rb_tz(g, min_tiles, es, 3, FX, FY);
-  if (tz > 0) return tz;
-  tx = FX2;
-  tz = rb_tz(g, min_tiles, es, 3, FX2, FY2);
-  if (tz > 0 || !brick_ok(g, min_tiles, 3)) return tz;
-  tx = 0;
-  return KZ;
+  return tz;
 }
 
-bool fused_rb3_ok(const Grid &g, int visc, int min_tiles) {
+bool fused_rb3_ok(const Grid &g, int visc, int min_tiles, int es) {
   int tx, np;
-  return tuning().rb_variant == 2 && (visc == -1 || visc == 1) && rb3_shape(g, min_tiles, 4, tx, np) > 0;
+  return tuning().rb_variant == 2 && (visc == -1 || visc == 1) && rb3_shape(g, min_tiles, es, tx, np) > 0;
 }
 
 template <typename T>
@@ -1542,7 +1579,7 @@ void launch_cc_rb_fused(hipStream_t s, const Grid &g, const T *pin, T *pout, con
   args.ay = a[1];
   args.az = a[2];
   int tx = FX;
-  const int tz = rb1_shape(g, min_tiles, sizeof(T), tx);
+  const int tz = rb1_shape(g, SWEEP_CC, 0, min_tiles, sizeof(T), tx);
   if (tz <= 0) {
     report_error("launch_cc_rb_fused: level not eligible");
     return;

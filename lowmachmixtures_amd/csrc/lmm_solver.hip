@@ -284,6 +284,11 @@ struct ProfScope {
   }
 };
 
+// counts the fused sweep launched last under the name of its form
+static void count_form(lmm_ctx *c, const char *multigrid) {
+  if (c->prof) c->fam[std::string(multigrid) + sweep_form()].launches++;
+}
+
 static void prof_flush(lmm_ctx *c) {
   for (auto &kv : c->fam) {
     for (auto &ev : kv.second.pending) {
@@ -520,10 +525,10 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
         hipMemcpyAsync(phi[d], L.res[d], sizeof(T) * L.g.N, hipMemcpyDeviceToDevice, c->stream);
       continue;
     }
-    const bool x3 = c->fused && c->fused3 && fused_rb3_ok(L.g, p.visc_type, c->fused_min_tiles);
+    const bool x3 = c->fused && c->fused3 && fused_rb3_ok(L.g, p.visc_type, c->fused_min_tiles, sizeof(T));
     const bool x2 = c->fused && fused_rb2d_ok(L.g, p.visc_type, c->fused_min_tiles);
     const bool x2c = c->fused && fused_rb2d_comp_ok(L.g, p.visc_type, c->fused_min_tiles);
-    if (x2 || x2c || x3 || (c->fused && fused_rb_ok(L.g, p.visc_type, c->fused_min_tiles))) {
+    if (x2 || x2c || x3 || (c->fused && fused_rb_ok(L.g, p.visc_type, c->fused_min_tiles, sizeof(T)))) {
       // sweep m reads one buffer and writes the other (phi <-> L.res); an
       // odd sweep count ends with a copy back
       T *const *src = (m % 2 == 0) ? phi : L.res;
@@ -536,6 +541,7 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
         ProfScope pf(c, "stag_rb_fused", bytes);
         ProfScope ps(c, fam, bytes, true);
         launch_stag_rb2d<T>(c->stream, L.g, p.visc_type, (T)p.stag_mg_omega, src, dst, rhs, K, zin);
+        count_form(c, "stag_sweep_");
       } else if (x3) {
         // all components in one launch: each array is compulsory once per
         // sweep (beta_cc and the edges shared by the components)
@@ -546,6 +552,7 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
         ProfScope ps(c, fam, bytes, true);
         launch_stag_rb_fused3<T>(c->stream, L.g, p.visc_type, (T)p.stag_mg_omega, src, dst, rhs, K,
                                  c->fused_min_tiles, zin);
+        count_form(c, "stag_sweep_");
       } else {
         // one component at a time; visc_type 2 and 3 read the other
         // components in their state at this component's turn of the colour
@@ -561,6 +568,7 @@ static void smooth(lmm_ctx *c, SLevel<T> &L, T *const phi[3], T *const rhs[3], i
           else
             launch_stag_rb_fused<T>(c->stream, L.g, p.visc_type, a, (T)p.stag_mg_omega, src[a], dst[a], rhs[a], K,
                                     c->fused_min_tiles, cur);
+          count_form(c, "stag_sweep_");
         }
       }
       if (m == nsweeps - 1 && m % 2 == 0)
@@ -638,7 +646,7 @@ template <typename T>
 static bool sweep_takes_zeros(lmm_ctx *c, const SLevel<T> &L) {
   const lmm_params &p = c->prm;
   return c->fused && p.stag_mg_smoother == 1 &&
-         ((c->fused3 && fused_rb3_ok(L.g, p.visc_type, c->fused_min_tiles)) ||
+         ((c->fused3 && fused_rb3_ok(L.g, p.visc_type, c->fused_min_tiles, sizeof(T))) ||
           fused_rb2d_ok(L.g, p.visc_type, c->fused_min_tiles));
 }
 
@@ -787,7 +795,7 @@ static void cc_vcycles(lmm_ctx *c, std::vector<CLevel<T>> &C, T *phi0, const T *
   int nl = c->nl_c;
   auto fused2d_at = [&](int n) { return c->fused && cc_rb2d_ok(C[n].g, c->fused_min_tiles); };
   auto fused_at = [&](int n) {
-    return fused2d_at(n) || (c->fused && fused_rb_tz(C[n].g, c->fused_min_tiles, 4, 1) > 0);
+    return fused2d_at(n) || (c->fused && cc_rb_ok(C[n].g, c->fused_min_tiles, sizeof(T)));
   };
   // a level's first down-leg sweep from its zero guess can take the zeros
   // without reading them (every point of its output is written): then phi is
@@ -828,6 +836,7 @@ static void cc_vcycles(lmm_ctx *c, std::vector<CLevel<T>> &C, T *phi0, const T *
         T *dst = (m % 2 == 0) ? C[n].res : ph;
         if (fused2d_at(n)) launch_cc_rb2d<T>(c->stream, C[n].g, src, dst, rh, C[n].a);
         else launch_cc_rb_fused<T>(c->stream, C[n].g, src, dst, rh, C[n].a, c->fused_min_tiles);
+        count_form(c, "cc_sweep_");
       }
       if (sweeps % 2 == 1) hipMemcpyAsync(ph, C[n].res, sizeof(T) * C[n].g.N, hipMemcpyDeviceToDevice, c->stream);
       return;
@@ -1557,6 +1566,8 @@ static void apply_options(lmm_ctx *c, const lmm_kernel_options &o) {
   c->tune.rb_pairs = (pairs && pairs[0] == '1') ? 1 : 2;
   const char *bk = getenv("LMM_SWEEP_BRICK");
   c->tune.rb_brick = bk ? atol(bk) : -1;
+  const char *br = getenv("LMM_BRICK_ROWS");
+  c->tune.rb_brick_rows = br ? atoi(br) : 0;
   const char *pt = getenv("LMM_PROLONG_TILED");
   c->tune.prolong_tiled = (pt && pt[0] == '0') ? 0 : 1;
   const char *cs = getenv("LMM_COARSE_SPLIT");
@@ -1821,7 +1832,7 @@ static int time_fine_sweeps(lmm_ctx *c, std::vector<SLevel<T>> &S, std::vector<C
       for (void *r : tmp) dfree(r);
       return LMM_ERR_NOMEM;
     }
-  const bool cc_fused = c->fused && fused_rb_tz(Z.g, c->fused_min_tiles, 4, 1) > 0;
+  const bool cc_fused = c->fused && cc_rb_ok(Z.g, c->fused_min_tiles, sizeof(T));
   auto run = [&]() {
     smooth<T>(c, L, phi, rhs, reps);
     if (cc_fused)

@@ -1,0 +1,57 @@
+"""Which form of the fused sweep a level takes by default (kernel_stats counts
+each form's launches): bricks where they pay, the colour kernels where bricks
+hang far over the box or a single component's are many, at the edges of the
+rule; and the same bits whatever the form."""
+import pytest
+
+from lowmachmixtures_amd import problems as P
+from lowmachmixtures_amd import stokes as S
+from tests.helpers import bit_equal
+
+pytestmark = pytest.mark.gpu
+
+FORMS = ["brick4", "brick8", "march", "march_pairs", "march_narrow", "plane", "block", "tile2d"]
+
+
+def forms(ctx, multigrid):
+    return {f for f in FORMS if ctx.kernel_stats(f"{multigrid}_sweep_{f}")["launches"] > 0}
+
+
+# one-level boxes: box, visc_type, precision, form of the staggered and of the cell-centred sweep (None: colour)
+CASES = [
+    ((32, 32, 32), -1, "fp64", "brick4", "brick4"),
+    ((64, 64, 64), -1, "fp64", "brick8", "brick4"),
+    ((64, 64, 64), -1, "fp32", "brick8", "brick4"),
+    ((16, 64, 64), 1, "fp64", "brick4", None),       # thin, but few bricks; cell-centred: half of each in the box
+    ((8, 128, 128), -1, "fp64", None, None),         # a quarter of each brick lies in the box
+    ((8, 128, 128), -1, "fp32", "brick8", None),
+    ((128, 12, 128), -1, "fp32", "brick4", "brick4"),  # 8 rows would hang over by a third
+    ((32, 32, 32), -2, "fp64", "brick4", "brick4"),  # launch-bound
+    ((32, 32, 32), -3, "fp32", "brick4", "brick4"),
+    ((64, 32, 32), 2, "fp64", "brick4", "brick4"),
+    ((64, 64, 64), 3, "fp64", "brick4", "brick4"),
+    ((64, 64, 64), -2, "fp64", None, "brick4"),      # one component, variable coefficients
+    ((64, 64, 64), -3, "fp32", None, "brick4"),
+    ((48, 48, 48), 2, "fp64", None, None),           # three quarters full
+    ((96, 64, 64), 2, "fp32", None, "brick4"),       # more than 512 bricks a component
+]
+
+
+@pytest.mark.parametrize("n,visc,prec,stag,cc", CASES)
+def test_form_by_default(n, visc, prec, stag, cc, monkeypatch):
+    pb = P.small_problem(3, n, visc_type=visc, seed=51, contrast=20.0)
+    b_u = P.rhs_from_noise_host(pb)
+    kw = dict(visc_type=visc, stag_mg_minwidth=min(n), mg_minwidth=min(n), gmres_max_iter=2,
+              precision=S.FP32_MG if prec == "fp32" else S.FP64)
+    sol = []
+    for smoother in (None, "colour"):
+        if smoother:
+            monkeypatch.setenv("LMM_SMOOTHER", smoother)
+        with S.Context(3, pb.n, pb.dx, **kw) as ctx:
+            dp = S.DeviceProblem(ctx, pb, rhs=b_u)
+            ctx.profiling(True)
+            dp.solve()
+            want = (set(), set()) if smoother else ({stag} - {None}, {cc} - {None})
+            assert (forms(ctx, "stag"), forms(ctx, "cc")) == want
+            sol.append(dp.solution())
+    assert bit_equal(sol[0][0], sol[1][0]) and bit_equal(sol[0][1], sol[1][1])
