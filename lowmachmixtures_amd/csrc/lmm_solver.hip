@@ -2333,9 +2333,8 @@ int lmm_stag_inner_prod(lmm_ctx *c, lmm_field *const m1[3], lmm_field *const m2[
   launch_fill<double>(c->stream, c->r + dim * N, N, 0.0);
   launch_fill<double>(c->stream, c->w + dim * N, N, 0.0);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
-                  arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
-  double h[4];
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
+  double h[4];  // not armed: a poll before the synchronisation that finish makes only adds to it
   if (!fetch(c, c->scal + 4100, 4, h)) return finish(c);
   for (int d = 0; d < 3; d++) prod_val[d] = d < dim ? h[d] : 0.0;
   return finish(c);
@@ -2350,9 +2349,8 @@ int lmm_cc_inner_prod(lmm_ctx *c, lmm_field *m1, lmm_field *m2, double *prod_val
   hipMemcpyAsync(c->r + dim * N, m1->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   hipMemcpyAsync(c->w + dim * N, m2->d, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
   launch_stokes_dot(c->stream, c->g, c->r, c->w, c->partial);
-  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0,
-                  arm(c, mirror(c, c->scal + 4100), FINALIZE_WRITES[2]));
-  double h[4];
+  launch_finalize(c->stream, c->g, c->partial, c->scal + 4100, 2, 1.0, mirror(c, c->scal + 4100));
+  double h[4];  // not armed: a poll before the synchronisation that finish makes only adds to it
   if (!fetch(c, c->scal + 4100, 4, h)) return finish(c);
   *prod_val = h[3];
   return finish(c);
