@@ -594,7 +594,7 @@ __global__ void __launch_bounds__(STPB) k_sp_lonsager(Grid g, SpParams sp, const
 // columns depend on the sums of earlier ones: scheduling fences alone let the
 // compiler load the whole matrix of both cells first (eight species: 256
 // registers and one wave per SIMD, 73 us at 384 x 320; now 121 and 61 us).
-template <int NS, bool LOWER>
+template <int NS, bool LOWER, bool PACKED = false>
 __device__ __forceinline__ void face_matvec(const double *M, long N, long t, long m, const double (&v)[NS],
                                             double (&acc)[NS]) {
   double a[2][NS], b[2][NS];
@@ -604,7 +604,7 @@ __device__ __forceinline__ void face_matvec(const double *M, long N, long t, lon
 #pragma unroll
       for (int r = 0; r < NS; r++)
         if (!LOWER || r >= c) {
-          const long q = (long)(r + NS * c) * N;
+          const long q = (long)(PACKED ? lpk_index<NS>(r, c) : r + NS * c) * N;
           a[c & 1][r] = M[q + t];
           b[c & 1][r] = M[q + m];
         }
@@ -694,8 +694,8 @@ __device__ __forceinline__ void face_noise(long N, long t, int d, int dim, const
 // stochastic flux on the face of cell t in direction d: variance *
 // L_face (sum_r w_r W_r), L_face the face average of the cell factors
 // (upper triangle zero, so only c <= r enters: adding 0*w leaves the sum's
-// bits unchanged), then correction_flux.
-template <int NS>
+// bits unchanged), then correction_flux.  Packed or full factors.
+template <int NS, bool PACKED>
 __device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, long m, int d, int dim, const double *L,
                                            const double *W, int n_rngs, const double *weights, double variance,
                                            double (&out)[NS]) {
@@ -704,7 +704,7 @@ __device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, l
   face_noise<NS>(N, t, d, dim, W, n_rngs, weights, w);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = 0.0;
-  face_matvec<NS, true>(L, N, t, m, w, out);
+  face_matvec<NS, true, PACKED>(L, N, t, m, w, out);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = out[r] * variance;
   correct_flux<NS>(sp, out);
@@ -751,7 +751,7 @@ __global__ void __launch_bounds__(STPB) k_sp_stoch_flux(Grid g, SpParams sp, con
   for (int d = 0; d < g.dim; d++) {
     const long m = at_sh(g, P, d, -1, -1, 0);
     double out[NS];
-    stoch_face<NS>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
+    stoch_face<NS, false>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
     double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -989,6 +989,35 @@ __global__ void __launch_bounds__(STPB) k_sp_chain_flux(Grid g, SpParams sp, SpF
   }
 }
 
+// The same face by face, both fluxes of each lower face in one thread: for
+// boxes that would leave most of every tile empty (face_tiles).
+template <int NS>
+__global__ void __launch_bounds__(STPB) k_sp_face_flux(Grid g, SpParams sp, SpFaceIn in, double *fd, double *fs,
+                                                        Ptr3<double> ft) {
+  const long t = xcd_block() * blockDim.x + threadIdx.x;
+  if (t >= g.N) return;
+  int i, j, k;
+  decode(g, t, i, j, k);
+  const Pt P = make_pt(g, i, j, k);
+  const long N = g.N;
+  const double dxinv = 1.0 / g.dx;
+  for (int d = 0; d < g.dim; d++) {
+    const long m = at_sh(g, P, d, -1, -1, 0);
+    double od[NS], os[NS];
+    diff_face<NS>(sp, N, dxinv, t, m, in.xm, in.rw, in.gama, in.temp, in.zeta, in.baro,
+                  in.baro ? in.gpb[d][t] : 0.0, od);
+    stoch_face<NS, true>(sp, N, t, m, d, g.dim, in.lpk, in.W, in.n_rngs, in.weights, in.variance, os);
+    double *const f = ft.c[d];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const long q = ((long)d * NS + s) * N + t;
+      fd[q] = od[s];
+      fs[q] = os[s];
+      f[(long)s * N + t] = (0.0 + od[s]) + os[s];
+    }
+  }
+}
+
 // compute_div of two species face-flux sets in one pass
 template <int NS>
 __global__ void __launch_bounds__(STPB) k_sp_div2(Grid g, const double *fa, double *da, const double *fb,
@@ -1207,6 +1236,15 @@ struct RunChainCell {
     return 0;
   }
 };
+// Whether compute_mass_fluxdiv's face pass goes in tiles: not in 3D boxes of
+// fewer than 12 cells in x, unless the tiles are so few that neither form fills
+// the GPU.  The whole call in us, face by face / in tiles: 4 x 256 x 256 two
+// species 73 / 113, four 138 / 251, eight 536 / 1016; 8 x 256 x 256 four
+// 274 / 335; 10 x 160 x 160 four 138 / 148; 12 x 160 x 160 four 179 / 163 (two
+// 75 / 78); 8 x 8 x 512 (512 tiles) four 56 / 50.  Thin in y (256 x 4 x 256 four
+// species 138 / 123) and in 2D (4 x 8192 four 52 / 50) the tiles win.
+inline bool face_tiles(const Grid &g, int ntiles) { return g.dim == 2 || g.n[0] >= 12 || ntiles <= 1024; }
+
 template <int NS>
 struct RunChainFace {
   static int run(hipStream_t s, const Grid &g, const SpParams &sp, const SpFaceIn &in, double *flux, double *dd,
@@ -1216,7 +1254,9 @@ struct RunChainFace {
       double *fs = flux + (long)g.dim * NS * g.N;
       const int nbx = (g.n[0] + FTX - 1) / FTX, nby = (g.n[1] + FTY - 1) / FTY, nz = g.dim == 3 ? g.n[2] : 1;
       const dim3 nb(nbx * nby * nz);
-      if (g.dim == 3)
+      if (!face_tiles(g, nbx * nby * nz))
+        SLAUNCH(k_sp_face_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in, flux, fs, p3(ft));
+      else if (g.dim == 3)
         SLAUNCH((k_sp_chain_flux<NS, 3>), nb, dim3(STPB), 0, s, g, sp, in, nbx, nz, flux, fs, p3(ft));
       else
         SLAUNCH((k_sp_chain_flux<NS, 2>), nb, dim3(STPB), 0, s, g, sp, in, nbx, nz, flux, fs, p3(ft));
