@@ -589,14 +589,26 @@ __global__ void __launch_bounds__(STPB) k_sp_lonsager(Grid g, SpParams sp, const
 // ---------------- face fluxes ----------------
 
 // acc[r] += sum_c 0.5 (M(r, c) at t + at m) v[c], c ascending; LOWER: r >= c.
-// The loads of column c + 1 are issued before column c is summed, so a column's
+// AHEAD: the loads of column c + 1 are issued before column c is summed, so a column's
 // wait overlaps the one before it.  The empty asm makes the indices of later
 // columns depend on the sums of earlier ones: scheduling fences alone let the
 // compiler load the whole matrix of both cells first (eight species: 256
 // registers and one wave per SIMD, 73 us at 384 x 320; now 121 and 61 us).
-template <int NS, bool LOWER, bool PACKED = false>
+// Otherwise a column is loaded and summed in turn (diff_ahead).
+template <int NS, bool LOWER, bool PACKED = false, bool AHEAD = true>
 __device__ __forceinline__ void face_matvec(const double *M, long N, long t, long m, const double (&v)[NS],
                                             double (&acc)[NS]) {
+  auto at = [&](int r, int c) { return (long)(PACKED ? lpk_index<NS>(r, c) : r + NS * c) * N; };
+  if constexpr (!AHEAD) {
+#pragma unroll
+    for (int c = 0; c < NS; c++) {
+#pragma unroll
+      for (int r = 0; r < NS; r++)
+        if (!LOWER || r >= c) acc[r] = acc[r] + 0.5 * (M[at(r, c) + t] + M[at(r, c) + m]) * v[c];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return;
+  }
   double a[2][NS], b[2][NS];
 #pragma unroll
   for (int c = 0; c <= NS; c++) {
@@ -604,9 +616,8 @@ __device__ __forceinline__ void face_matvec(const double *M, long N, long t, lon
 #pragma unroll
       for (int r = 0; r < NS; r++)
         if (!LOWER || r >= c) {
-          const long q = (long)(PACKED ? lpk_index<NS>(r, c) : r + NS * c) * N;
-          a[c & 1][r] = M[q + t];
-          b[c & 1][r] = M[q + m];
+          a[c & 1][r] = M[at(r, c) + t];
+          b[c & 1][r] = M[at(r, c) + m];
         }
     }
     if (c > 0) {
@@ -633,7 +644,7 @@ __device__ __forceinline__ void correct_flux(const SpParams &sp, double (&out)[N
 // Gama_face grad x + zeta_face grad T + baro_face gradp_baro of the face
 // between cells t (above) and m (below): the vector that
 // rhoWchi_face multiplies.  Gama null: identity.
-template <int NS>
+template <int NS, bool AHEAD>
 __device__ __forceinline__ void diff_drive(long N, double dxinv, long t, long m, const double *xm, const double *gama,
                                            const double *temp, const double *zeta, const double *baro, double gpb,
                                            double (&y)[NS]) {
@@ -643,7 +654,7 @@ __device__ __forceinline__ void diff_drive(long N, double dxinv, long t, long m,
   if (gama) {
 #pragma unroll
     for (int r = 0; r < NS; r++) y[r] = 0.0;
-    face_matvec<NS, false>(gama, N, t, m, x, y);
+    face_matvec<NS, false, false, AHEAD>(gama, N, t, m, x, y);
   } else {
     // Gama_face = I: the sum 0 + 0*x_0 + ... + 1*x_r + ... is 0 + x_r
 #pragma unroll
@@ -663,7 +674,7 @@ __device__ __forceinline__ void diff_drive(long N, double dxinv, long t, long m,
 }
 
 // diffusive_mass_flux: rhoWchi_face times the above, correction_flux.
-template <int NS>
+template <int NS, bool AHEAD = true>
 __device__ __forceinline__ void diff_face(const SpParams &sp, long N, double dxinv, long t, long m, const double *xm,
                                           const double *rw, const double *gama, const double *temp, const double *zeta,
                                           const double *baro, double gpb, double (&out)[NS]) {
@@ -671,15 +682,15 @@ __device__ __forceinline__ void diff_face(const SpParams &sp, long N, double dxi
   // loads out of a caller's loop; no instruction is emitted
   asm volatile("" : "+v"(t), "+v"(m));
   double y[NS];
-  diff_drive<NS>(N, dxinv, t, m, xm, gama, temp, zeta, baro, gpb, y);
+  diff_drive<NS, AHEAD>(N, dxinv, t, m, xm, gama, temp, zeta, baro, gpb, y);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = 0.0;
-  face_matvec<NS, false>(rw, N, t, m, y, out);
+  face_matvec<NS, false, false, AHEAD>(rw, N, t, m, y, out);
   correct_flux<NS>(sp, out);
 }
 
-// sum_r w_r W_r of the face of cell t in direction d
-template <int NS>
+// sum_r w_r W_r of the face of cell t in direction d; PAST: read past the caches
+template <int NS, bool PAST = true>
 __device__ __forceinline__ void face_noise(long N, long t, int d, int dim, const double *W, int n_rngs,
                                            const double *weights, double (&w)[NS]) {
 #pragma unroll
@@ -687,7 +698,10 @@ __device__ __forceinline__ void face_noise(long N, long t, int d, int dim, const
   for (int r = 0; r < n_rngs; r++) {
     const double wr = weights[r];
 #pragma unroll
-    for (int s = 0; s < NS; s++) w[s] = w[s] + wr * __builtin_nontemporal_load(W + ((long)(r * dim + d) * NS + s) * N + t);
+    for (int s = 0; s < NS; s++) {
+      const double *p = W + ((long)(r * dim + d) * NS + s) * N + t;
+      w[s] = w[s] + wr * (PAST ? __builtin_nontemporal_load(p) : *p);
+    }
   }
 }
 
@@ -695,13 +709,13 @@ __device__ __forceinline__ void face_noise(long N, long t, int d, int dim, const
 // L_face (sum_r w_r W_r), L_face the face average of the cell factors
 // (upper triangle zero, so only c <= r enters: adding 0*w leaves the sum's
 // bits unchanged), then correction_flux.  Packed or full factors.
-template <int NS, bool PACKED>
+template <int NS, bool PACKED, bool PAST>
 __device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, long m, int d, int dim, const double *L,
                                            const double *W, int n_rngs, const double *weights, double variance,
                                            double (&out)[NS]) {
   asm volatile("" : "+v"(t), "+v"(m));
   double w[NS];
-  face_noise<NS>(N, t, d, dim, W, n_rngs, weights, w);
+  face_noise<NS, PAST>(N, t, d, dim, W, n_rngs, weights, w);
 #pragma unroll
   for (int r = 0; r < NS; r++) out[r] = 0.0;
   face_matvec<NS, true, PACKED>(L, N, t, m, w, out);
@@ -711,7 +725,7 @@ __device__ __forceinline__ void stoch_face(const SpParams &sp, long N, long t, l
 }
 
 // flux_total: ft_zero set -> 0.0 + F (setval then add), else ft + F
-template <int NS>
+template <int NS, bool AHEAD>
 __global__ void __launch_bounds__(STPB) k_sp_diff_flux(Grid g, SpParams sp, const double *xm, const double *rw,
                                                         const double *gama, const double *temp, const double *zeta,
                                                         const double *baro, Ptr3<const double> gpb, double *flux,
@@ -726,8 +740,8 @@ __global__ void __launch_bounds__(STPB) k_sp_diff_flux(Grid g, SpParams sp, cons
   for (int d = 0; d < g.dim; d++) {
     const long m = at_sh(g, P, d, -1, -1, 0);
     double out[NS];
-    diff_face<NS>(sp, N, dxinv, t, m, xm, rw, gama, temp, zeta, baro,
-                  baro ? gpb.c[d][t] : 0.0, out);
+    diff_face<NS, AHEAD>(sp, N, dxinv, t, m, xm, rw, gama, temp, zeta, baro,
+                         baro ? gpb.c[d][t] : 0.0, out);
     double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -738,7 +752,7 @@ __global__ void __launch_bounds__(STPB) k_sp_diff_flux(Grid g, SpParams sp, cons
   }
 }
 
-template <int NS>
+template <int NS, bool PAST>
 __global__ void __launch_bounds__(STPB) k_sp_stoch_flux(Grid g, SpParams sp, const double *L, const double *W,
                                                          int n_rngs, const double *weights, double variance,
                                                          double *flux, Ptr3<double> ft) {
@@ -751,7 +765,7 @@ __global__ void __launch_bounds__(STPB) k_sp_stoch_flux(Grid g, SpParams sp, con
   for (int d = 0; d < g.dim; d++) {
     const long m = at_sh(g, P, d, -1, -1, 0);
     double out[NS];
-    stoch_face<NS, false>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
+    stoch_face<NS, false, PAST>(sp, N, t, m, d, g.dim, L, W, n_rngs, weights, variance, out);
     double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -991,7 +1005,7 @@ __global__ void __launch_bounds__(STPB) k_sp_chain_flux(Grid g, SpParams sp, SpF
 
 // The same face by face, both fluxes of each lower face in one thread: for
 // boxes that would leave most of every tile empty (face_tiles).
-template <int NS>
+template <int NS, bool PAST>
 __global__ void __launch_bounds__(STPB) k_sp_face_flux(Grid g, SpParams sp, SpFaceIn in, double *fd, double *fs,
                                                         Ptr3<double> ft) {
   const long t = xcd_block() * blockDim.x + threadIdx.x;
@@ -1006,7 +1020,7 @@ __global__ void __launch_bounds__(STPB) k_sp_face_flux(Grid g, SpParams sp, SpFa
     double od[NS], os[NS];
     diff_face<NS>(sp, N, dxinv, t, m, in.xm, in.rw, in.gama, in.temp, in.zeta, in.baro,
                   in.baro ? in.gpb[d][t] : 0.0, od);
-    stoch_face<NS, true>(sp, N, t, m, d, g.dim, in.lpk, in.W, in.n_rngs, in.weights, in.variance, os);
+    stoch_face<NS, true, PAST>(sp, N, t, m, d, g.dim, in.lpk, in.W, in.n_rngs, in.weights, in.variance, os);
     double *const f = ft.c[d];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -1201,12 +1215,40 @@ struct RunLonsager {
     return 0;
   }
 };
+// Whether the diffusive face pass loads a column ahead: not for 5 and 6 species
+// whose matrices exceed the 256 MB of the last-level cache, which gain nothing
+// from it (128^3, diffusive_mass_fluxdiv in us, ahead / in turn: 5 species 708 /
+// 681, 6 974 / 948, 8 species at 96^3 694 / 832; 512^2, in the cache: 5 species
+// 67 / 69, 6 84 / 89, 8 129 / 151; at 2 to 4 no difference).
+template <int NS>
+inline bool diff_ahead(const Grid &g) {
+  return (NS != 5 && NS != 6) || (double)NS * NS * g.N * sizeof(double) <= 256e6;
+}
+template <int NS>
+inline auto diff_kernel(const Grid &g) {
+  auto k = k_sp_diff_flux<NS, true>;
+  if constexpr (NS == 5 || NS == 6)
+    if (!diff_ahead<NS>(g)) k = k_sp_diff_flux<NS, false>;
+  return k;
+}
+// Whether a face-by-face pass reads the noise past the caches: of which it
+// uses every value once, but below about 55 MB it finds the noise in them
+// (stochastic_mass_fluxdiv in us, past / through, two stages: 128^3 two species,
+// 201 MB, 181 / 200; 512^2 two, 17 MB, 44.5 / 43.3, four, 34 MB, 60.5 / 59.0; 8 x
+// 256 x 256 two, 50 MB, 64.9 / 60.2, four, 101 MB, 114 / 129).  From 6 species on
+// the pass is the faster past them at any size (64 x 48 x 32 six, 28 MB, 66.7 /
+// 69.7, eight 82.7 / 86.7).
+template <int NS>
+inline bool noise_past(const Grid &g, int n_rngs) {
+  return NS >= 6 || (double)n_rngs * g.dim * NS * g.N * sizeof(double) > 55e6;
+}
+
 template <int NS>
 struct RunDiffusive {
   static int run(hipStream_t s, const Grid &g, const SpParams &sp, const double *xm, const double *rw,
                  const double *G, const double *T, const double *z, const double *baro, const double *const gpb[3],
                  double *flux, double *const ft[3], double *div) {
-    SLAUNCH(k_sp_diff_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, xm, rw, G, T, z, baro, cp3(gpb), flux,
+    SLAUNCH(diff_kernel<NS>(g), dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, xm, rw, G, T, z, baro, cp3(gpb), flux,
             p3(ft), 0);
     SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, div, 0);
     return 0;
@@ -1220,7 +1262,10 @@ template <int NS>
 struct RunStochastic {
   static int run(hipStream_t s, const Grid &g, const SpParams &sp, const double *L, const double *W, int nr,
                  const double *w, double var, double *flux, double *const ft[3], double *div, int inc) {
-    SLAUNCH(k_sp_stoch_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, L, W, nr, w, var, flux, p3(ft));
+    auto kern = k_sp_stoch_flux<NS, true>;
+    if constexpr (NS < 6)
+      if (!noise_past<NS>(g, nr)) kern = k_sp_stoch_flux<NS, false>;
+    SLAUNCH(kern, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, L, W, nr, w, var, flux, p3(ft));
     SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, div, inc);
     return 0;
   }
@@ -1239,8 +1284,8 @@ struct RunChainCell {
 // Whether compute_mass_fluxdiv's face pass goes in tiles: not in 3D boxes of
 // fewer than 12 cells in x, unless the tiles are so few that neither form fills
 // the GPU.  The whole call in us, face by face / in tiles: 4 x 256 x 256 two
-// species 73 / 113, four 138 / 251, eight 536 / 1016; 8 x 256 x 256 four
-// 274 / 335; 10 x 160 x 160 four 138 / 148; 12 x 160 x 160 four 179 / 163 (two
+// species 68 / 113, four 136 / 250, eight 534 / 1014; 8 x 256 x 256 four
+// 275 / 341; 10 x 160 x 160 four 136 / 147; 12 x 160 x 160 four 179 / 163 (two
 // 75 / 78); 8 x 8 x 512 (512 tiles) four 56 / 50.  Thin in y (256 x 4 x 256 four
 // species 138 / 123) and in 2D (4 x 8192 four 52 / 50) the tiles win.
 inline bool face_tiles(const Grid &g, int ntiles) { return g.dim == 2 || g.n[0] >= 12 || ntiles <= 1024; }
@@ -1254,8 +1299,11 @@ struct RunChainFace {
       double *fs = flux + (long)g.dim * NS * g.N;
       const int nbx = (g.n[0] + FTX - 1) / FTX, nby = (g.n[1] + FTY - 1) / FTY, nz = g.dim == 3 ? g.n[2] : 1;
       const dim3 nb(nbx * nby * nz);
+      auto face = k_sp_face_flux<NS, true>;
+      if constexpr (NS < 6)
+        if (!noise_past<NS>(g, in.n_rngs)) face = k_sp_face_flux<NS, false>;
       if (!face_tiles(g, nbx * nby * nz))
-        SLAUNCH(k_sp_face_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in, flux, fs, p3(ft));
+        SLAUNCH(face, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in, flux, fs, p3(ft));
       else if (g.dim == 3)
         SLAUNCH((k_sp_chain_flux<NS, 3>), nb, dim3(STPB), 0, s, g, sp, in, nbx, nz, flux, fs, p3(ft));
       else
@@ -1263,7 +1311,7 @@ struct RunChainFace {
       SLAUNCH(k_sp_div2<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, dd, fs, sd);
       return 0;
     }
-    SLAUNCH(k_sp_diff_flux<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in.xm, in.rw, in.gama, in.temp, in.zeta,
+    SLAUNCH(diff_kernel<NS>(g), dim3(sblk(g.N)), dim3(STPB), 0, s, g, sp, in.xm, in.rw, in.gama, in.temp, in.zeta,
             in.baro, cp3(in.baro ? in.gpb : nullptr), flux, p3(ft), 1);
     SLAUNCH(k_sp_div<NS>, dim3(sblk(g.N)), dim3(STPB), 0, s, g, flux, dd, 0);
     return 0;

@@ -1,5 +1,6 @@
-"""The face-by-face form of compute_mass_fluxdiv's face pass, which boxes too thin
-for tiles take.  The oracle's operations in the oracle's order: the same bits."""
+"""The face-by-face forms of the species face passes: boxes too thin for tiles
+(compute_mass_fluxdiv), noise beyond and within the caches, matrices beyond the
+last-level cache.  The oracle's operations in the oracle's order: the same bits."""
 import numpy as np
 import pytest
 
@@ -37,3 +38,56 @@ def _chain(n, ns, stages, **kw):
 def test_thin_boxes(n, ns, ideal):
     _chain(n, ns, 1, is_ideal_mixture=ideal)
 
+
+def test_thin_box_noise_past_the_caches():
+    _chain((8, 8, 9216), 2, 2)  # 57 MB of noise
+
+
+def test_stochastic_flux_noise_past_the_caches():
+    n, ns, n_rngs = (64, 96, 96), 2, 2  # 57 MB
+    rng = np.random.default_rng(53)
+    shape = tuple(reversed(n))
+    kn = _knobs(ns, rng, k_B=0.3)
+    sp, g = O.species(ns, **kn), O.geom(3, n, 0.5)
+    rho = _rho(ns, shape, rng, tiny=False)
+    rt, x, mt = O.convert_cons_to_prim(g, sp, rho)
+    Db, Dt, H = O.compute_mixture_properties(g, sp, shape)
+    G = O.compute_Gama(g, sp, x, H)
+    chi, _ = O.compute_chi(g, sp, rho, rt, x, Db, Dt, np.ones(shape))
+    W = _mass_noise(77, n_rngs, 3, ns, shape)
+    want, want_ft = O.stochastic_mass_fluxdiv(g, sp, rho, rt, x, mt, chi, G, [np.zeros((ns,) + shape)] * 3, 0.01, W,
+                                              [0.75, -0.5])
+    with S.Context(3, n, 0.5, stag_mg_minwidth=64, mg_minwidth=64) as ctx:
+        S.set_species(ctx, ns, **kn)
+        S.init_mass_stochastic(ctx, n_rngs)
+        S.fill_mass_stochastic(ctx, 77)
+        ft, div = [ctx.field(S.FACE_X + d, ns) for d in range(3)], ctx.field(S.CELL, ns)
+        S.stochastic_mass_fluxdiv(ctx, ctx.field(S.CELL, ns, rho), ctx.field(S.CELL, 1, rt), ctx.field(S.CELL, ns, x),
+                                  ctx.field(S.CELL, 1, mt), ctx.field(S.CELL, ns * ns, chi),
+                                  ctx.field(S.CELL, ns * ns, G), div, ft, 0.01, [0.75, -0.5])
+        assert bit_equal(div.download(), want)
+        assert bit_equal([f.download() for f in ft], want_ft)
+
+
+@pytest.mark.parametrize("ns,copies", [(5, 10), (6, 8)])
+def test_matrices_beyond_the_last_level_cache(ns, copies):
+    """A box of copies of a smaller one has the smaller one's fluxes, copied: the
+    larger one's matrices exceed 256 MB, the smaller one's do not."""
+    n = (64, 64, 32)
+    rng = np.random.default_rng(ns)
+
+    def run(m):
+        N = (n[0], n[1], n[2] * m)
+        with S.Context(3, N, 0.5, stag_mg_minwidth=min(N), mg_minwidth=min(N)) as ctx:
+            S.set_species(ctx, ns, **kn)
+            f = [ctx.field(S.CELL, a.shape[0], np.tile(a, (1, m, 1, 1))) for a in fields]
+            ft, div = [ctx.field(S.FACE_X + d, ns) for d in range(3)], ctx.field(S.CELL, ns)
+            S.diffusive_mass_fluxdiv(ctx, ns, f[0], f[1], f[2], f[3], f[4], div, f[5], f[6], None, ft)
+            return [div.download()] + [q.download() for q in ft]
+
+    kn = _knobs(ns, rng)
+    shape = tuple(reversed(n))
+    fields = [rng.uniform(0.2, 1.0, (k,) + shape) for k in (ns, 1, ns, ns * ns, ns * ns, 1, ns)]
+    small, large = run(1), run(copies)
+    assert ns * ns * np.prod(n) * copies * 8 > 256e6 > ns * ns * np.prod(n) * 8
+    assert bit_equal(large, [np.tile(a, (1, copies, 1, 1)) for a in small])
