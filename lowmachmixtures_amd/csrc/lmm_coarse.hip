@@ -7,8 +7,8 @@
 // one workgroup of 1024 threads runs the whole coarse part of the V-cycle --
 // down-leg smoothing, residual and restriction on every coarse level, the
 // bottom smoothing, then prolongation and up-leg smoothing -- with a
-// workgroup barrier between dependent passes.  Every point is computed by the
-// same device function as in the one-launch-per-pass kernels, in the same
+// workgroup barrier between dependent passes.  Every point is computed with the
+// arithmetic of the one-launch-per-pass kernels, in the same
 // order of passes, so the result is bit for bit that of the separate launches
 // (and of the reference's stag_mg_solver / F_MG level loops).  For
 // visc_type -1 and 1 a face component's operator reads only that component,
@@ -23,8 +23,8 @@ namespace lmm {
 namespace {
 
 constexpr int CTPB = 1024;
-const char kStagCoarseName[] = "k_stag_coarse_vcycle";
-const char kCCCoarseName[] = "k_cc_coarse_vcycle";
+const char kStagCoarseName[] = "k_stag_coarse_lds";
+const char kCCCoarseName[] = "k_cc_coarse_lds";
 
 template <typename T>
 struct SLevelDesc {
@@ -33,12 +33,12 @@ struct SLevelDesc {
   StagCoef<T> K;
 };
 
+// visc: -1 or 1
 template <typename T>
 struct SCoarseArgs {
   SLevelDesc<T> L[COARSE_MAX_LEVELS];
   int m;                 // coarse levels held in L[0..m-1], finest first
   int visc, nd, nu, nb;  // visc_type, sweeps down / up / bottom
-  int split;             // 1: workgroup a handles component a only
   T omega;
 };
 
@@ -51,14 +51,13 @@ __device__ void blk_fill(T *x, long n, T v) {
 // every colour is a constant after inlining (no per-lane stack for the
 // per-component pointer tables)
 template <typename T, int DIM>
-__device__ void blk_stag_smooth_d(const SLevelDesc<T> &L, int visc, T omega, int nsweeps, int alo, int ahi) {
+__device__ void blk_stag_smooth_d(const SLevelDesc<T> &L, int visc, T omega, int nsweeps) {
   const long half = (long)(L.g.n[0] >> 1) * L.g.n[1] * L.g.n[2];
   const T dxsqinv = (T)(1.0 / (L.g.dx * L.g.dx));
   for (int m = 0; m < nsweeps; m++) {
 #pragma unroll
     for (int color = 1; color <= 2 * DIM; color++) {
       const int a = (color - 1) / 2, par = (color + 1) % 2;
-      if (a < alo || a >= ahi) continue;  // uniform over the workgroup
       for (long t = threadIdx.x; t < half; t += CTPB)
         gs_colour_at<T>(L.g, DIM, visc, a, par, omega, dxsqinv, L.phi, L.K, L.rhs.c[a], t);
       __syncthreads();
@@ -67,102 +66,50 @@ __device__ void blk_stag_smooth_d(const SLevelDesc<T> &L, int visc, T omega, int
 }
 
 template <typename T>
-__device__ void blk_stag_smooth(const SLevelDesc<T> &L, int visc, T omega, int nsweeps, int alo, int ahi) {
-  if (L.g.dim == 3) blk_stag_smooth_d<T, 3>(L, visc, omega, nsweeps, alo, ahi);
-  else blk_stag_smooth_d<T, 2>(L, visc, omega, nsweeps, alo, ahi);
+__device__ void blk_stag_smooth(const SLevelDesc<T> &L, int visc, T omega, int nsweeps) {
+  if (L.g.dim == 3) blk_stag_smooth_d<T, 3>(L, visc, omega, nsweeps);
+  else blk_stag_smooth_d<T, 2>(L, visc, omega, nsweeps);
 }
 
 template <typename T>
-__device__ void blk_prolong(const SLevelDesc<T> &F, const SLevelDesc<T> &C, int alo, int ahi) {
+__device__ void blk_prolong(const SLevelDesc<T> &F, const SLevelDesc<T> &C) {
   const long N = F.g.N;
   if (F.g.dim == 2) {
-    if (alo <= 0 && 0 < ahi)
-      for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 2, 0>(F.g, C.g, F.phi.c[0], C.phi.c[0], t);
-    if (alo <= 1 && 1 < ahi)
-      for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 2, 1>(F.g, C.g, F.phi.c[1], C.phi.c[1], t);
+    for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 2, 0>(F.g, C.g, F.phi.c[0], C.phi.c[0], t);
+    for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 2, 1>(F.g, C.g, F.phi.c[1], C.phi.c[1], t);
   } else {
-    if (alo <= 0 && 0 < ahi)
-      for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 0>(F.g, C.g, F.phi.c[0], C.phi.c[0], t);
-    if (alo <= 1 && 1 < ahi)
-      for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 1>(F.g, C.g, F.phi.c[1], C.phi.c[1], t);
-    if (alo <= 2 && 2 < ahi)
-      for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 2>(F.g, C.g, F.phi.c[2], C.phi.c[2], t);
+    for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 0>(F.g, C.g, F.phi.c[0], C.phi.c[0], t);
+    for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 1>(F.g, C.g, F.phi.c[1], C.phi.c[1], t);
+    for (long t = threadIdx.x; t < N; t += CTPB) prolong_at<T, 3, 2>(F.g, C.g, F.phi.c[2], C.phi.c[2], t);
   }
   __syncthreads();
 }
 
+// The staggered coarse V-cycle passing every field through memory, all
+// components in one workgroup (visc_type -1 / 1 with coarse_split = 0 only: the
+// form that the LDS kernels below are compared with).
 template <typename T>
 __global__ void __launch_bounds__(CTPB) k_stag_coarse_vcycle(SCoarseArgs<T> A) {
   const int m = A.m, dim = A.L[0].g.dim;
-  // the components this workgroup handles
-  const int alo = A.split ? (int)blockIdx.x : 0, ahi = A.split ? alo + 1 : dim;
   for (int n = 0; n < m; n++)
-    for (int d = alo; d < ahi; d++) blk_fill<T>(A.L[n].phi.c[d], A.L[n].g.N, (T)0);
+    for (int d = 0; d < dim; d++) blk_fill<T>(A.L[n].phi.c[d], A.L[n].g.N, (T)0);
   __syncthreads();
   for (int n = 0; n < m - 1; n++) {
     const SLevelDesc<T> &L = A.L[n];
-    blk_stag_smooth<T>(L, A.visc, A.omega, A.nd, alo, ahi);
+    blk_stag_smooth<T>(L, A.visc, A.omega, A.nd);
     const T dxsqinv = (T)(1.0 / (L.g.dx * L.g.dx));
-    for (int a = alo; a < ahi; a++)
+    for (int a = 0; a < dim; a++)
       for (long t = threadIdx.x; t < L.g.N; t += CTPB) residual_at<T>(L.g, dim, A.visc, dxsqinv, L.phi, L.rhs, L.res, L.K, a, t);
     __syncthreads();
     const SLevelDesc<T> &Cn = A.L[n + 1];
-    for (int a = alo; a < ahi; a++)
+    for (int a = 0; a < dim; a++)
       for (long t = threadIdx.x; t < Cn.g.N; t += CTPB) restrict_at<T>(Cn.g, L.g, 0, L.res, Cn.rhs, a, t);
     __syncthreads();
   }
-  blk_stag_smooth<T>(A.L[m - 1], A.visc, A.omega, A.nb, alo, ahi);
+  blk_stag_smooth<T>(A.L[m - 1], A.visc, A.omega, A.nb);
   for (int n = m - 2; n >= 0; n--) {
-    blk_prolong<T>(A.L[n], A.L[n + 1], alo, ahi);
-    blk_stag_smooth<T>(A.L[n], A.visc, A.omega, A.nu, alo, ahi);
-  }
-}
-
-template <typename T>
-struct CLevelDesc {
-  Grid g;
-  T *phi, *rhs, *res;
-  Ptr3<T> a;
-};
-
-template <typename T>
-struct CCoarseArgs {
-  CLevelDesc<T> L[COARSE_MAX_LEVELS];
-  int m, nd, nu, nb;
-};
-
-template <typename T>
-__device__ void blk_cc_rb(const CLevelDesc<T> &L, int nsweeps) {
-  const long half = (long)(L.g.n[0] >> 1) * L.g.n[1] * L.g.n[2];
-  const T inv = (T)(1.0 / (L.g.dx * L.g.dx));
-  for (int s = 0; s < nsweeps; s++)
-    for (int colour = 0; colour < 2; colour++) {
-      for (long t = threadIdx.x; t < half; t += CTPB) cc_rb_at<T>(L.g, colour, inv, L.phi, L.rhs, L.a, t);
-      __syncthreads();
-    }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(CTPB) k_cc_coarse_vcycle(CCoarseArgs<T> A) {
-  const int m = A.m;
-  for (int n = 0; n < m; n++) blk_fill<T>(A.L[n].phi, A.L[n].g.N, (T)0);
-  __syncthreads();
-  for (int n = 0; n < m - 1; n++) {
-    const CLevelDesc<T> &L = A.L[n];
-    blk_cc_rb<T>(L, A.nd);
-    const T inv = (T)(1.0 / (L.g.dx * L.g.dx));
-    for (long t = threadIdx.x; t < L.g.N; t += CTPB) cc_residual_at<T>(L.g, inv, L.phi, L.rhs, L.res, L.a, t);
-    __syncthreads();
-    const CLevelDesc<T> &Cn = A.L[n + 1];
-    for (long t = threadIdx.x; t < Cn.g.N; t += CTPB) cc_restrict_at<T>(Cn.g, L.g, L.res, Cn.rhs, t);
-    __syncthreads();
-  }
-  blk_cc_rb<T>(A.L[m - 1], A.nb);
-  for (int n = m - 2; n >= 0; n--) {
-    const CLevelDesc<T> &F = A.L[n], &Cn = A.L[n + 1];
-    for (long t = threadIdx.x; t < F.g.N; t += CTPB) cc_prolong_add_at<T>(F.g, Cn.g, F.phi, Cn.phi, t);
-    __syncthreads();
-    blk_cc_rb<T>(F, A.nu);
+    blk_prolong<T>(A.L[n], A.L[n + 1]);
+    blk_stag_smooth<T>(A.L[n], A.visc, A.omega, A.nu);
   }
 }
 
@@ -182,7 +129,8 @@ __global__ void __launch_bounds__(CTPB) k_cc_coarse_vcycle(CCoarseArgs<T> A) {
 // instruction issue on the first level (one compute unit works; about 0.5 us
 // a pass of 16^3) and the chain of LDS read, update and barrier below (0.2 us).
 // Each point's arithmetic and the order of passes are those of the form
-// above, so the bits are the same.  A whole coarse part over 16^3 .. 2^3,
+// above, so the bits are the same (div_by has the range).  visc_type 3 in 3D and
+// FP64 spills 31 registers at two pairs a thread, the cell-centred kernel one.  A whole coarse part over 16^3 .. 2^3,
 // before and after: staggered FP64 100 -> 31 us, visc_type 2 (one workgroup)
 // 315 -> 86 us, cell-centred 73 -> 28 us.
 // ---------------------------------------------------------------------------
@@ -273,7 +221,10 @@ struct Nbr<T, DIM, false> {
 // the exact remainder; the first brings q within an ulp, and with r the
 // correctly rounded reciprocal the second is then the correctly rounded
 // quotient (Markstein, IBM J. Res. Dev. 34, 1990), the same bits as x / d in
-// 5 operations instead of about 14.  A quotient that is not finite is x r.
+// 5 operations instead of about 14 as long as the remainders and 1 / d are
+// normal numbers, that is for |x| above about 1e-289 and |d| between 1e-307 and
+// 1e307; below, the last bit may differ, and a quotient of -0 comes out as +0,
+// which changes nothing where it is added.  A quotient that is not finite is x r.
 __device__ __forceinline__ double rcp_of(double d) { return 1.0 / d; }
 __device__ __forceinline__ float rcp_of(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ float div_by(float x, float, float r) { return x * r; }
@@ -769,15 +720,17 @@ __global__ void __launch_bounds__(CTPB) k_cc_coarse_lds(CLdsArgs<T> A) {
 
 // Shapes and LDS offsets of levels lv[0..m-1] with nc components each: phi of
 // every level, the right-hand sides below the first, one residual field of
-// the first level's size.  false: more than the LDS holds, or a level whose
-// indices do not fit the kernels' 16-bit offsets or colouring.
+// the first level's size.  Levels of at most COARSE_MAX_CELLS = 4096 cells and
+// even extents always fit: the largest need is 16^3's, 159104 bytes with three
+// FP64 components.  false: a level past that (also past the kernels' 16-bit
+// offsets, colouring or two pairs a thread).
 template <typename T, typename LV, typename OUT>
 bool lds_plan(int m, const LV *lv, int nc, OUT *L, int &res) {
   long off = 0;
   for (int n = 0; n < m; n++) {
     const Grid &g = lv[n].g;
     LvShape &s = L[n].s;
-    if (g.N > 65535 || g.n[0] % 2 != 0) return false;
+    if (g.N > COARSE_MAX_CELLS || g.n[0] % 2 != 0) return false;
     s.nx = g.n[0];
     s.ny = g.n[1];
     s.nz = g.n[2];
@@ -795,6 +748,7 @@ bool lds_plan(int m, const LV *lv, int nc, OUT *L, int &res) {
   }
   res = (int)off;
   if (m > 1) off += L[0].s.N;
+  static_assert(COARSE_MAX_CELLS <= 4 * CTPB, "two pairs a thread");
   return off * (long)sizeof(T) <= LDS_BYTES;
 }
 
@@ -805,12 +759,14 @@ inline int lds_threads(int half, int nq) {
 }
 
 template <typename T, int DIM, int VISC>
-bool launch_stag_lds(hipStream_t s, int m, const CoarseStagLevel<T> *lv, T omega, int nd, int nu, int nb) {
+void launch_stag_lds(hipStream_t s, int m, const CoarseStagLevel<T> *lv, T omega, int nd, int nu, int nb) {
   constexpr int NC = (VISC == -1 || VISC == 1) ? 1 : DIM;
   SLdsArgs<T> A;
-  if (!lds_plan<T>(m, lv, NC, A.L, A.res)) return false;
+  if (!lds_plan<T>(m, lv, NC, A.L, A.res)) {
+    report_error("launch_stag_coarse_vcycle: the levels do not fit LDS");
+    return;
+  }
   const int half = (int)(lv[0].g.N / 2), nq = half > CTPB ? 2 : 1;
-  if (half > nq * CTPB) return false;
   for (int n = 0; n < m; n++) {
     A.L[n].K = lv[n].K;
     A.L[n].dxsqinv = (T)(1.0 / (lv[n].g.dx * lv[n].g.dx));
@@ -826,29 +782,29 @@ bool launch_stag_lds(hipStream_t s, int m, const CoarseStagLevel<T> *lv, T omega
   if (nq == 1) hipLaunchKernelGGL((k_stag_coarse_lds<T, DIM, VISC, 1>), grid, block, 0, s, A);
   else hipLaunchKernelGGL((k_stag_coarse_lds<T, DIM, VISC, 2>), grid, block, 0, s, A);
   post_launch(s, kStagCoarseName);
-  return true;
 }
 
 template <typename T, int DIM>
-bool launch_stag_lds_visc(hipStream_t s, int m, const CoarseStagLevel<T> *lv, int visc, T omega, int nd, int nu,
+void launch_stag_lds_visc(hipStream_t s, int m, const CoarseStagLevel<T> *lv, int visc, T omega, int nd, int nu,
                           int nb) {
   switch (visc) {
-    case -1: return launch_stag_lds<T, DIM, -1>(s, m, lv, omega, nd, nu, nb);
-    case 1: return launch_stag_lds<T, DIM, 1>(s, m, lv, omega, nd, nu, nb);
-    case 2: return launch_stag_lds<T, DIM, 2>(s, m, lv, omega, nd, nu, nb);
-    case 3: return launch_stag_lds<T, DIM, 3>(s, m, lv, omega, nd, nu, nb);
-    case -2: return launch_stag_lds<T, DIM, -2>(s, m, lv, omega, nd, nu, nb);
-    case -3: return launch_stag_lds<T, DIM, -3>(s, m, lv, omega, nd, nu, nb);
-    default: return false;
+    case -1: launch_stag_lds<T, DIM, -1>(s, m, lv, omega, nd, nu, nb); break;
+    case 1: launch_stag_lds<T, DIM, 1>(s, m, lv, omega, nd, nu, nb); break;
+    case 2: launch_stag_lds<T, DIM, 2>(s, m, lv, omega, nd, nu, nb); break;
+    case 3: launch_stag_lds<T, DIM, 3>(s, m, lv, omega, nd, nu, nb); break;
+    case -2: launch_stag_lds<T, DIM, -2>(s, m, lv, omega, nd, nu, nb); break;
+    default: launch_stag_lds<T, DIM, -3>(s, m, lv, omega, nd, nu, nb); break;
   }
 }
 
 template <typename T, int DIM>
-bool launch_cc_lds(hipStream_t s, int m, const CoarseCCLevel<T> *lv, int nd, int nu, int nb) {
+void launch_cc_lds(hipStream_t s, int m, const CoarseCCLevel<T> *lv, int nd, int nu, int nb) {
   CLdsArgs<T> A;
-  if (!lds_plan<T>(m, lv, 1, A.L, A.res)) return false;
+  if (!lds_plan<T>(m, lv, 1, A.L, A.res)) {
+    report_error("launch_cc_coarse_vcycle: the levels do not fit LDS");
+    return;
+  }
   const int half = (int)(lv[0].g.N / 2), nq = half > CTPB ? 2 : 1;
-  if (half > nq * CTPB) return false;
   for (int n = 0; n < m; n++) {
     A.L[n].a = p3(lv[n].a);
     A.L[n].inv = (T)(1.0 / (lv[n].g.dx * lv[n].g.dx));
@@ -863,7 +819,6 @@ bool launch_cc_lds(hipStream_t s, int m, const CoarseCCLevel<T> *lv, int nd, int
   if (nq == 1) hipLaunchKernelGGL((k_cc_coarse_lds<T, DIM, 1>), dim3(1), block, 0, s, A);
   else hipLaunchKernelGGL((k_cc_coarse_lds<T, DIM, 2>), dim3(1), block, 0, s, A);
   post_launch(s, kCCCoarseName);
-  return true;
 }
 
 }  // namespace
@@ -871,13 +826,12 @@ bool launch_cc_lds(hipStream_t s, int m, const CoarseCCLevel<T> *lv, int nd, int
 template <typename T>
 void launch_stag_coarse_vcycle(hipStream_t s, int m, const CoarseStagLevel<T> *lv, int visc, T omega, int nd,
                                int nu, int nb) {
-  // the LDS form wherever the levels fit it (it was the faster one at every
-  // size measured, 4 to 4096 cells); not where coarse_split = 0 asks for
-  // visc_type -1 / 1 in one workgroup
+  // the LDS form was the faster one at every size measured, 4 to 4096 cells;
+  // coarse_split = 0 asks for visc_type -1 / 1 in one workgroup
   if (tuning().coarse_split || (visc != -1 && visc != 1)) {
-    if (lv[0].g.dim == 3 ? launch_stag_lds_visc<T, 3>(s, m, lv, visc, omega, nd, nu, nb)
-                         : launch_stag_lds_visc<T, 2>(s, m, lv, visc, omega, nd, nu, nb))
-      return;
+    if (lv[0].g.dim == 3) launch_stag_lds_visc<T, 3>(s, m, lv, visc, omega, nd, nu, nb);
+    else launch_stag_lds_visc<T, 2>(s, m, lv, visc, omega, nd, nu, nb);
+    return;
   }
   SCoarseArgs<T> A;
   A.m = m;
@@ -893,30 +847,14 @@ void launch_stag_coarse_vcycle(hipStream_t s, int m, const CoarseStagLevel<T> *l
     A.L[n].res = p3(lv[n].res);
     A.L[n].K = lv[n].K;
   }
-  // visc_type -1 / 1: independent components, one workgroup each
-  const int dim = lv[0].g.dim;
-  A.split = (visc == -1 || visc == 1) && tuning().coarse_split ? 1 : 0;
-  hipLaunchKernelGGL(k_stag_coarse_vcycle<T>, dim3(A.split ? dim : 1), dim3(CTPB), 0, s, A);
-  post_launch(s, kStagCoarseName);
+  hipLaunchKernelGGL(k_stag_coarse_vcycle<T>, dim3(1), dim3(CTPB), 0, s, A);
+  post_launch(s, "k_stag_coarse_vcycle");
 }
 
 template <typename T>
 void launch_cc_coarse_vcycle(hipStream_t s, int m, const CoarseCCLevel<T> *lv, int nd, int nu, int nb) {
-  if (lv[0].g.dim == 3 ? launch_cc_lds<T, 3>(s, m, lv, nd, nu, nb) : launch_cc_lds<T, 2>(s, m, lv, nd, nu, nb)) return;
-  CCoarseArgs<T> A;
-  A.m = m;
-  A.nd = nd;
-  A.nu = nu;
-  A.nb = nb;
-  for (int n = 0; n < m; n++) {
-    A.L[n].g = lv[n].g;
-    A.L[n].phi = lv[n].phi;
-    A.L[n].rhs = lv[n].rhs;
-    A.L[n].res = lv[n].res;
-    A.L[n].a = p3(lv[n].a);
-  }
-  hipLaunchKernelGGL(k_cc_coarse_vcycle<T>, dim3(1), dim3(CTPB), 0, s, A);
-  post_launch(s, kCCCoarseName);
+  if (lv[0].g.dim == 3) launch_cc_lds<T, 3>(s, m, lv, nd, nu, nb);
+  else launch_cc_lds<T, 2>(s, m, lv, nd, nu, nb);
 }
 
 template void launch_stag_coarse_vcycle<double>(hipStream_t, int, const CoarseStagLevel<double> *, int, double,

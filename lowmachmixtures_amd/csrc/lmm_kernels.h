@@ -158,7 +158,7 @@ struct CoarseStagLevel {
 template <typename T>
 struct CoarseCCLevel {
   Grid g;
-  T *phi, *rhs, *res;
+  T *phi, *rhs;
   T *a[3];
 };
 // Levels lv[0..m-1] (finest first): zero phi on all of them, then the

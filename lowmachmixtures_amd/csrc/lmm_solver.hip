@@ -860,7 +860,6 @@ static void cc_vcycles(lmm_ctx *c, std::vector<CLevel<T>> &C, T *phi0, const T *
     L.g = C[n].g;
     L.phi = C[n].phi;
     L.rhs = C[n].rhs;
-    L.res = C[n].res;
     for (int d = 0; d < 3; d++) L.a[d] = C[n].a[d];
     clv.push_back(L);
   }
