@@ -71,13 +71,15 @@ def short(name, width=60):
 
 
 def fetch_factor(fetch):
-    """True read bytes / FETCH_SIZE of k_convert<float, double> (one 8-byte value per work-item)."""
+    """True read bytes / FETCH_SIZE of the conversion kernels (one 8-byte value per
+    work-item): k_convert_list, a level's coefficients to FP32, and k_convert<float, double>."""
     ratios = []
     for name, val, grid in fetch.values():
-        if "k_convert<float, double>" in name and val > 0 and grid >= (1 << 22):
+        if ("k_convert_list" in name or "k_convert<float, double>" in name) and val > 0 and grid >= (1 << 22):
             ratios.append(grid * 8.0 / val)
     if not ratios:
-        return 2.0, []
+        raise ValueError("no conversion dispatch of at least 2^22 work-items to calibrate FETCH_SIZE with "
+                         "(the run needs an FP32 multigrid form)")
     ratios.sort()
     return ratios[len(ratios) // 2], ratios
 
@@ -124,9 +126,9 @@ def summarize(d, n, command, out_trace, out_counters):
         lines.append(f"  rocprofv3 {what} --output-format csv -d <dir> -o run -- {command}")
     lines += ["Reduced by python -m lowmachmixtures_amd.profiling (joined on Dispatch_Id; a launch is level 0 when",
               "its WRITE_SIZE is at least half the arrays a level-0 launch writes).", "",
-              "Calibration with the plain conversion kernel k_convert<float, double> (one 8-byte value per work-item):",
-              f"  true read / FETCH_SIZE = {factor:.3f} (median of {len(ratios)} dispatches"
-              + (f", min {ratios[0]:.3f} max {ratios[-1]:.3f})" if ratios else ")"),
+              "Calibration with the conversion kernels (k_convert_list; one 8-byte value per work-item):",
+              f"  true read / FETCH_SIZE = {factor:.3f} (median of {len(ratios)} dispatches,"
+              f" min {ratios[0]:.3f} max {ratios[-1]:.3f})",
               f"  => HBM read bytes = {factor:.2f} x FETCH_SIZE; WRITE_SIZE is taken as is", "",
               f"{'kernel (level 0)':60s} {'n':>4s} {'avg_us':>8s} {'read MB':>9s} {'write MB':>9s} {'traffic MB':>10s}"
               f" {'alg MB':>8s} {'ratio':>6s} {'alg GB/s':>9s} {'HBM GB/s':>9s}"]
