@@ -103,7 +103,10 @@ typedef struct {
  * LMM_* environment switches present at its creation. */
 typedef struct {
   int fused_sweeps;        /* 1: fused red-black sweeps where a level allows; 0: colour kernels */
-  int fused_min_tiles;     /* a level below this many workgroups per launch uses the colour kernels */
+  int fused_min_tiles;     /* above 64: a level whose sweep has fewer workgroups uses the colour
+                              kernels; 2 to 64 (default 64): the form measured as the faster, which
+                              has no such limit but where it marches; 1: a fused sweep on every
+                              level whose extents allow one */
   int fused_kernel;        /* fused-sweep form: 0 plane marching, 1 block, 2 paired plane marching */
   int fused_target;        /* workgroups the z-slab choice aims for (FP32; FP64 twice) */
   int fused_x3;            /* 1: the three face components in one launch */

@@ -1223,13 +1223,13 @@ static int tiles2d(const Grid &g) { return ((g.n[0] + TX2D - 1) / TX2D) * ((g.n[
 // Every 2D level of even extents is swept in tiles: one launch (visc_type -1,
 // 1) or one a component against two colour launches a component, each as long
 // as a tile's (192 x 160 FP64 visc_type -2, a component: 4.15 against 2 x 3.2 us).
-// min_tiles above its default of 64 workgroups counts them, two components'.
-static bool even2d(const Grid &g, int min_tiles) {
-  return g.dim == 2 && g.n[0] % 2 == 0 && g.n[1] % 2 == 0 && (min_tiles <= 64 || 2 * tiles2d(g) >= min_tiles);
+// min_tiles above its default of 64 workgroups counts a sweep's, ncomp components'.
+static bool even2d(const Grid &g, int min_tiles, int ncomp) {
+  return g.dim == 2 && g.n[0] % 2 == 0 && g.n[1] % 2 == 0 && (min_tiles <= 64 || ncomp * tiles2d(g) >= min_tiles);
 }
 
 bool fused_rb2d_ok(const Grid &g, int visc, int min_tiles) {
-  return (visc == -1 || visc == 1) && even2d(g, min_tiles);
+  return (visc == -1 || visc == 1) && even2d(g, min_tiles, 2);
 }
 
 template <typename T, int VISC>
@@ -1267,7 +1267,7 @@ template void launch_stag_rb2d<float>(hipStream_t, const Grid &, int, float, flo
                                       float *const[3], const StagCoef<float> &, bool);
 
 bool fused_rb2d_comp_ok(const Grid &g, int visc, int min_tiles) {
-  return (visc < -1 || visc > 1) && even2d(g, min_tiles);
+  return (visc < -1 || visc > 1) && even2d(g, min_tiles, 2);
 }
 
 template <typename T, int A, int VISC>
@@ -1315,7 +1315,7 @@ template void launch_stag_rb2d_comp<float>(hipStream_t, const Grid &, int, int, 
                                            const float *, const StagCoef<float> &, const float *);
 
 bool cc_rb2d_ok(const Grid &g, int min_tiles) {
-  return even2d(g, min_tiles);
+  return even2d(g, min_tiles, 1);
 }
 
 template <typename T>

@@ -104,13 +104,13 @@ struct lmm_ctx {
   int n_rngs = 0;
   double *Wcc = nullptr, *Wed = nullptr;
   double *stoch_work = nullptr;  // filtered stochastic fluxes (filtering_width > 0)
-  // Smoother kernels: fused red-black sweeps on levels with at least
-  // fused_min_tiles workgroups in a launch (32^3 and up), colour-by-colour kernels
-  // elsewhere.  Both give the same bits.  LMM_SMOOTHER=colour in the
-  // environment selects the colour kernels everywhere, LMM_SMOOTHER=fused
-  // the fused sweep on every level whose extents allow it;
-  // LMM_FUSED_MIN_TILES and LMM_FUSED_TARGET (workgroups aimed for when the
-  // z-slab thickness is chosen) tune the choice.
+  // Smoother kernels: fused red-black sweeps or colour-by-colour kernels, by
+  // the measured rules of lmm_smooth.hip.  Both give the same bits.
+  // LMM_SMOOTHER=colour in the environment selects the colour kernels
+  // everywhere, LMM_SMOOTHER=fused (fused_min_tiles = 1) a fused sweep on every
+  // level whose extents allow one; LMM_FUSED_MIN_TILES above 64 leaves levels
+  // with fewer workgroups to the colour kernels, LMM_FUSED_TARGET is the number
+  // of workgroups aimed for when the z-slab thickness is chosen.
   bool fused = true;
   int fused_min_tiles = 64;
   // coarse levels (at most COARSE_MAX_CELLS cells) of both multigrids run

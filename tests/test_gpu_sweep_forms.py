@@ -55,3 +55,15 @@ def test_form_by_default(n, visc, prec, stag, cc, monkeypatch):
             assert (forms(ctx, "stag"), forms(ctx, "cc")) == want
             sol.append(dp.solution())
     assert bit_equal(sol[0][0], sol[1][0]) and bit_equal(sol[0][1], sol[1][1])
+
+
+@pytest.mark.parametrize("tiles,stag,cc", [(64, True, True), (65, True, False), (128, True, False), (129, False, False)])
+def test_min_tiles_counts_a_sweeps_workgroups(tiles, stag, cc, monkeypatch):
+    """256 x 128: 64 tiles, 128 workgroups for the two components of a sweep."""
+    monkeypatch.setenv("LMM_FUSED_MIN_TILES", str(tiles))
+    pb = P.small_problem(2, (256, 128), visc_type=-1, seed=52)
+    with S.Context(2, pb.n, pb.dx, stag_mg_minwidth=128, mg_minwidth=128, visc_type=-1, gmres_max_iter=1) as ctx:
+        dp = S.DeviceProblem(ctx, pb, rhs=P.rhs_from_noise_host(pb))
+        ctx.profiling(True)
+        dp.solve()
+        assert (forms(ctx, "stag"), forms(ctx, "cc")) == ({"tile2d"} if stag else set(), {"tile2d"} if cc else set())
