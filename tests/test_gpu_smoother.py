@@ -1,13 +1,13 @@
-"""The fused red-black smoother (visc_type -1 and 1; 3D and 2D) on levels
-whose extents allow it (x a multiple of 64, y of 8), against the oracle and against
-the colour-by-colour kernels.  Both must agree bit for bit: every point is
-computed with the reference's operation order.  Two forms of the fused sweep
-exist (LMM_FUSED_KERNEL=march2, the default, block and march).
-LMM_SMOOTHER=fused makes the small test levels use the fused sweep, which by
-default only launches of at least 64 workgroups (32^3 and up) do; the
-plane-marching forms choose their z-slab thickness for LMM_FUSED_TARGET
-workgroups (768 by default: 2-plane slabs on these small levels, 1 for the
-thickest slab a level allows)."""
+"""The fused red-black smoother (3D and 2D) on levels whose extents the
+plane-marching tiles divide (x a multiple of 64, y of 8; or 32 and 16), against
+the oracle and against the colour-by-colour kernels.  Both must agree bit for
+bit: every point is computed with the reference's operation order.  Three
+marching forms exist (LMM_FUSED_KERNEL=march2, the default, block and march).
+LMM_SWEEP_BRICK=0 keeps these small levels from the bricks that they take by
+default (test_gpu_brick.py), LMM_SMOOTHER=fused from the colour kernels; the
+launch counts of kernel_stats say which form ran.  The plane-marching forms
+choose their z-slab thickness for LMM_FUSED_TARGET workgroups (768 by default:
+2-plane slabs on these small levels, 1 for the thickest slab a level allows)."""
 import numpy as np
 import pytest
 
@@ -19,6 +19,17 @@ from tests.helpers import bit_equal, oracle_args, relerr
 pytestmark = pytest.mark.gpu
 
 N3 = (64, 16, 32)
+FORMS = ["brick4", "brick8", "march", "march_pairs", "march_narrow", "plane", "block", "tile2d"]
+FORM_OF = {"march2": "march", "march": "plane", "block": "block"}  # by LMM_FUSED_KERNEL
+
+
+def _forms(ctx, multigrid):
+    return {f for f in FORMS if ctx.kernel_stats(f"{multigrid}_sweep_{f}")["launches"] > 0}
+
+
+@pytest.fixture
+def marching(monkeypatch):
+    monkeypatch.setenv("LMM_SWEEP_BRICK", "0")
 
 
 def _rand_faces(shape, seed, ncomp=3):
@@ -33,13 +44,13 @@ def _mg_solve(pb, kw, rhs, guess):
         ctx.profiling(True)
         S.stag_mg_solver(ctx, dp.alpha, dp.beta, dp.beta_ed, dp.gamma, 0.9, phi, dp.b_u)
         fused = ctx.kernel_stats("stag_rb_fused")["launches"]
-        return [f.download() for f in phi], fused
+        return [f.download() for f in phi], fused, _forms(ctx, "stag")
 
 
 @pytest.mark.parametrize("kernel,target", [("march2", "1024"), ("march2", "1"), ("block", "1024"), ("march", "1")])
 @pytest.mark.parametrize("visc", [-1, 1])
 @pytest.mark.parametrize("vcycles,sweeps", [(1, (2, 2, 8)), (2, (2, 2, 8)), (1, (1, 3, 3))])
-def test_fused_mg_solver_bit_exact(visc, vcycles, sweeps, kernel, target, monkeypatch):
+def test_fused_mg_solver_bit_exact(visc, vcycles, sweeps, kernel, target, marching, monkeypatch):
     monkeypatch.setenv("LMM_SMOOTHER", "fused")
     monkeypatch.setenv("LMM_FUSED_KERNEL", kernel)
     monkeypatch.setenv("LMM_FUSED_TARGET", target)
@@ -50,26 +61,27 @@ def test_fused_mg_solver_bit_exact(visc, vcycles, sweeps, kernel, target, monkey
     rhs = _rand_faces(pb.shape, 7)
     guess = _rand_faces(pb.shape, 8)
     want = O.stag_mg_solver(g, p, cf, 0.9, rhs, phi=guess)
-    got, fused = _mg_solve(pb, kw, rhs, guess)
+    got, fused, forms = _mg_solve(pb, kw, rhs, guess)
     assert fused > 0, "the fused smoother did not run"
+    assert forms == {FORM_OF[kernel]}
     assert bit_equal(got, want), relerr(got, want)
 
 
 @pytest.mark.parametrize("visc", [-1, 1])
-def test_fused_equals_colour_kernels(visc, monkeypatch):
+def test_fused_equals_colour_kernels(visc, marching, monkeypatch):
     pb = P.small_problem(3, (128, 32, 16), visc_type=visc, seed=67)
     kw = dict(visc_type=visc)
     rhs = _rand_faces(pb.shape, 9)
     guess = _rand_faces(pb.shape, 10)
     monkeypatch.setenv("LMM_SMOOTHER", "colour")
-    ref, fused0 = _mg_solve(pb, kw, rhs, guess)
+    ref, fused0, _ = _mg_solve(pb, kw, rhs, guess)
     monkeypatch.setenv("LMM_SMOOTHER", "fused")
-    got, fused1 = _mg_solve(pb, kw, rhs, guess)
-    assert fused0 == 0 and fused1 > 0
+    got, fused1, forms = _mg_solve(pb, kw, rhs, guess)
+    assert fused0 == 0 and fused1 > 0 and forms == {"march"}
     assert bit_equal(got, ref)
 
 
-def test_fused_fp32_fgmres_equals_colour(monkeypatch):
+def test_fused_fp32_fgmres_equals_colour(marching, monkeypatch):
     pb = P.small_problem(3, (64, 32, 32), visc_type=-1, seed=71, contrast=100.0)
     b_u = P.rhs_from_noise_host(pb)
     out = []
@@ -77,13 +89,15 @@ def test_fused_fp32_fgmres_equals_colour(monkeypatch):
         monkeypatch.setenv("LMM_SMOOTHER", mode)
         with S.Context(3, pb.n, pb.dx, visc_type=-1, precision=S.FP32_MG) as ctx:
             dp = S.DeviceProblem(ctx, pb, rhs=b_u)
+            ctx.profiling(True)
             _, info = dp.solve()
             out.append((info["total_iter"], dp.solution()))
+            assert _forms(ctx, "stag") == (set() if mode == "colour" else {"march_pairs", "march_narrow"})
     assert out[0][0] == out[1][0]
     assert bit_equal(out[0][1][0], out[1][1][0]) and bit_equal(out[0][1][1], out[1][1][1])
 
 
-def test_fused_gmres_parity(monkeypatch):
+def test_fused_gmres_parity(marching, monkeypatch):
     monkeypatch.setenv("LMM_SMOOTHER", "fused")
     pb = P.small_problem(3, N3, visc_type=-1, seed=73, contrast=100.0)
     g, p, cf = oracle_args(pb)
@@ -101,7 +115,7 @@ def test_fused_gmres_parity(monkeypatch):
 @pytest.mark.parametrize("kernel,target", [("march2", "1024"), ("march2", "1"), ("block", "1024"), ("march", "1")])
 @pytest.mark.parametrize("n,vcycles,sweeps", [((64, 16, 32), 1, (2, 2)), ((128, 32, 16), 2, (3, 1)),
                                               ((64, 32, 32), 1, (1, 2))])
-def test_fused_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, kernel, target, monkeypatch):
+def test_fused_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, kernel, target, marching, monkeypatch):
     monkeypatch.setenv("LMM_FUSED_KERNEL", kernel)
     monkeypatch.setenv("LMM_FUSED_TARGET", target)
     rng = np.random.default_rng(91)
@@ -118,8 +132,11 @@ def test_fused_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, kernel
             a = ctx.faces(ainv)
             r = ctx.field(S.CELL, 1, rhs)
             phi = ctx.field(S.CELL)
+            ctx.profiling(True)
             S.macproject(ctx, phi, None, a, r)
             out[mode] = phi.download()
+            narrow = {"march_narrow"} if kernel == "march2" and n == (64, 32, 32) else set()  # its 32 x 16 x 16 level
+            assert _forms(ctx, "cc") == (set() if mode == "colour" else {FORM_OF[kernel]} | narrow)
     assert bit_equal(out["fused"], out["colour"])
     assert bit_equal(out["fused"], want)
 
@@ -127,7 +144,7 @@ def test_fused_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, kernel
 @pytest.mark.parametrize("visc", [-1, 1])
 @pytest.mark.parametrize("n,target", [((64, 16, 32), "1024"), ((128, 32, 16), "1"), ((64, 32, 32), "1"),
                                       ((32, 32, 16), "768")])
-def test_three_components_in_one_launch_equal_separate(visc, n, target, monkeypatch):
+def test_three_components_in_one_launch_equal_separate(visc, n, target, marching, monkeypatch):
     """The default fused sweep runs the three face components in one launch
     (64 x 8 tiles, or 32 x 16 on levels 32 points wide, as the plane-marching
     one-component launches do too); LMM_FUSED_X3=0 launches them one by one.
@@ -138,17 +155,18 @@ def test_three_components_in_one_launch_equal_separate(visc, n, target, monkeypa
     kw = dict(visc_type=visc, stag_mg_max_vcycles=2)
     rhs, guess = _rand_faces(pb.shape, 8), _rand_faces(pb.shape, 9)
     monkeypatch.setenv("LMM_FUSED_X3", "0")
-    ref, n0 = _mg_solve(pb, kw, rhs, guess)
+    ref, n0, f0 = _mg_solve(pb, kw, rhs, guess)
     monkeypatch.setenv("LMM_FUSED_X3", "1")
-    got, n1 = _mg_solve(pb, kw, rhs, guess)
+    got, n1, f1 = _mg_solve(pb, kw, rhs, guess)
     assert n1 > 0
+    assert f0 == f1 == {(64, 32, 32): {"march", "march_narrow"}, (32, 32, 16): {"march_narrow"}}.get(n, {"march"})
     if n[0] % 64 == 0 and n[0] // 2 % 64 == 0:  # no 32-wide fused level
         assert n0 == 3 * n1
     assert bit_equal(got, ref)
 
 
 @pytest.mark.parametrize("visc", [-1, 1])
-def test_narrow_tile_sweep_matches_oracle(visc, monkeypatch):
+def test_narrow_tile_sweep_matches_oracle(visc, marching, monkeypatch):
     """Levels 32 points wide run the three-component sweep on 32 x 16 tiles."""
     monkeypatch.setenv("LMM_SMOOTHER", "fused")
     pb = P.small_problem(3, (32, 32, 16), visc_type=visc, seed=107)
@@ -156,19 +174,21 @@ def test_narrow_tile_sweep_matches_oracle(visc, monkeypatch):
     g, p, cf = oracle_args(pb, **kw)
     rhs, guess = _rand_faces(pb.shape, 10), _rand_faces(pb.shape, 11)
     want = O.stag_mg_solver(g, p, cf, 0.9, rhs, phi=guess)
-    got, fused = _mg_solve(pb, kw, rhs, guess)
-    assert fused > 0
+    got, fused, forms = _mg_solve(pb, kw, rhs, guess)
+    assert fused > 0 and forms == {"march_narrow"}
     assert bit_equal(got, want), relerr(got, want)
 
 
 @pytest.mark.parametrize("n,coarse", [((64, 32, 2), "1"), ((128, 64, 4), "0"), ((128, 64, 4), "1")])
 @pytest.mark.parametrize("prec", ["fp64", "fp32_mg"])
-def test_first_sweep_from_zeros_equals_filled_guess(n, coarse, prec, monkeypatch):
+@pytest.mark.parametrize("brick", ["-1", "0"])
+def test_first_sweep_from_zeros_equals_filled_guess(n, coarse, prec, brick, monkeypatch):
     """A level whose first smoothing in a cycle is a fused sweep starts from
     its zero guess without the guess being written or read.  Covers a single
     level (z = 2 does not coarsen) and a bottom level smoothed in the level
     loop (LMM_COARSE=0), in both multigrids, against the colour kernels,
     which zero the guess in memory."""
+    monkeypatch.setenv("LMM_SWEEP_BRICK", brick)
     monkeypatch.setenv("LMM_COARSE", coarse)
     pb = P.small_problem(3, n, visc_type=-1, seed=109, contrast=30.0)
     b_u = P.rhs_from_noise_host(pb)
@@ -184,7 +204,7 @@ def test_first_sweep_from_zeros_equals_filled_guess(n, coarse, prec, monkeypatch
     assert bit_equal(out["fused"][1][0], out["colour"][1][0]) and bit_equal(out["fused"][1][1], out["colour"][1][1])
 
 
-# 2D: both face components in one launch on 64 x 8 tiles
+# 2D: both face components in one launch on 32 x 16 tiles
 
 
 @pytest.mark.parametrize("visc", [-1, 1])
@@ -199,21 +219,21 @@ def test_fused_2d_mg_solver_bit_exact(n, visc, vcycles, sweeps, monkeypatch):
     rhs = _rand_faces(pb.shape, 12, 2)
     guess = _rand_faces(pb.shape, 13, 2)
     want = O.stag_mg_solver(g, p, cf, 0.9, rhs, phi=guess)
-    got, fused = _mg_solve(pb, kw, rhs, guess)
-    assert fused > 0, "the fused smoother did not run"
+    got, fused, forms = _mg_solve(pb, kw, rhs, guess)
+    assert fused > 0 and forms == {"tile2d"}, "the fused smoother did not run"
     assert bit_equal(got, want), relerr(got, want)
 
 
 @pytest.mark.parametrize("visc", [-1, 1])
 def test_fused_2d_equals_colour_kernels(visc, monkeypatch):
-    """At the default launch threshold (16 workgroups on 2D levels: 64^2 and up)."""
+    """At the default launch threshold, which every 2D level passes."""
     pb = P.small_problem(2, (512, 256), visc_type=visc, seed=127)
     kw = dict(visc_type=visc, stag_mg_max_vcycles=2)
     rhs, guess = _rand_faces(pb.shape, 14, 2), _rand_faces(pb.shape, 15, 2)
     monkeypatch.setenv("LMM_SMOOTHER", "colour")
-    ref, fused0 = _mg_solve(pb, kw, rhs, guess)
+    ref, fused0, _ = _mg_solve(pb, kw, rhs, guess)
     monkeypatch.delenv("LMM_SMOOTHER")
-    got, fused1 = _mg_solve(pb, kw, rhs, guess)
+    got, fused1, _ = _mg_solve(pb, kw, rhs, guess)
     assert fused0 == 0 and fused1 > 0
     assert bit_equal(got, ref)
 
@@ -243,9 +263,8 @@ def test_fused_2d_gmres_equals_colour(prec, visc, monkeypatch):
 @pytest.mark.parametrize("n,vcycles,sweeps,mode", [((128, 64), 1, (2, 2), "fused"), ((256, 128), 2, (3, 1), "fused"),
                                                    ((512, 256), 2, (2, 2), None)])
 def test_fused_2d_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, mode, monkeypatch):
-    """The 2D cell-centred red-black sweep in one launch per sweep (64 x 8
-    tiles): with LMM_SMOOTHER=fused on every eligible level, and at the
-    default threshold (16 workgroups on 2D levels: 8192 cells and up)."""
+    """The 2D cell-centred red-black sweep in one launch per sweep (32 x 16
+    tiles): with LMM_SMOOTHER=fused and at the default threshold."""
     rng = np.random.default_rng(93)
     shape = tuple(reversed(n))
     ainv = [0.5 + rng.random(shape) for _ in range(2)]
@@ -279,7 +298,7 @@ def test_fused_2d_cc_multigrid_matches_oracle_and_colour(n, vcycles, sweeps, mod
 @pytest.mark.parametrize("visc", [2, 3])
 @pytest.mark.parametrize("dim,n,vcycles,sweeps", [(3, (64, 16, 32), 2, (2, 2, 8)), (3, (64, 32, 16), 1, (1, 3, 3)),
                                                   (2, (128, 64), 2, (2, 2, 8)), (2, (128, 128), 1, (1, 3, 3))])
-def test_fused_coupled_visc_mg_solver_bit_exact(dim, n, vcycles, sweeps, visc, monkeypatch):
+def test_fused_coupled_visc_mg_solver_bit_exact(dim, n, vcycles, sweeps, visc, marching, monkeypatch):
     monkeypatch.setenv("LMM_SMOOTHER", "fused")
     pb = P.small_problem(dim, n, visc_type=visc, seed=137)
     kw = dict(visc_type=visc, stag_mg_max_vcycles=vcycles, stag_mg_nsmooths_down=sweeps[0],
@@ -288,8 +307,9 @@ def test_fused_coupled_visc_mg_solver_bit_exact(dim, n, vcycles, sweeps, visc, m
     rhs = _rand_faces(pb.shape, 16, dim)
     guess = _rand_faces(pb.shape, 17, dim)
     want = O.stag_mg_solver(g, p, cf, 0.9, rhs, phi=guess)
-    got, fused = _mg_solve(pb, kw, rhs, guess)
+    got, fused, forms = _mg_solve(pb, kw, rhs, guess)
     assert fused > 0, "the fused smoother did not run"
+    assert ("march" if dim == 3 else "tile2d") in forms and not forms & {"brick4", "brick8"}
     assert bit_equal(got, want), relerr(got, want)
 
 
@@ -317,7 +337,7 @@ def test_fused_coupled_visc_gmres_equals_colour(dim, n, visc, prec, monkeypatch)
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32_mg"])
-def test_autotune_keeps_the_bits(prec):
+def test_autotune_keeps_the_bits(prec, marching):
     """lmm_ctx_autotune picks the z-slab target among its candidates by timing
     the fine-level sweeps; a solve after it equals one before it bit for bit
     (the slab shape never changes the arithmetic), and the target stays in the
@@ -337,3 +357,27 @@ def test_autotune_keeps_the_bits(prec):
         after = dp.solution()
     assert i0["total_iter"] == i1["total_iter"]
     assert bit_equal(before[0], after[0]) and bit_equal(before[1], after[1])
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mg"])
+def test_large_level_marches_by_default(prec, monkeypatch):
+    """128^3, which no switch keeps from the form it takes in use: tiles of 64 x 8
+    (FP64) or 64 x 16 (FP32) points marching through slabs of the default target, the
+    levels below in bricks; against the colour kernels."""
+    pb = P.small_problem(3, (128, 128, 128), visc_type=-1, seed=151, contrast=10.0)
+    b_u = P.rhs_from_noise_host(pb)
+    out = []
+    for mode in ("colour", None):
+        if mode is None:
+            monkeypatch.delenv("LMM_SMOOTHER", raising=False)
+        else:
+            monkeypatch.setenv("LMM_SMOOTHER", mode)
+        with S.Context(3, pb.n, pb.dx, visc_type=-1, precision={"fp64": S.FP64, "fp32_mg": S.FP32_MG}[prec],
+                       gmres_max_iter=3) as ctx:
+            dp = S.DeviceProblem(ctx, pb, rhs=b_u)
+            ctx.profiling(True)
+            dp.solve()
+            out.append(dp.solution())
+            forms = _forms(ctx, "stag")
+            assert forms == (set() if mode else {"march" if prec == "fp64" else "march_pairs", "brick4", "brick8"})
+    assert bit_equal(out[0][0], out[1][0]) and bit_equal(out[0][1], out[1][1])
