@@ -1422,17 +1422,31 @@ static bool brick_ok(const Grid &g, int min_tiles, int ncomp) {
 //   cell-centred  FP64  32^3 5.8/9.0/6.4       64^3 7.1/9.9/8.1    48^3 5.9/-/7.6            128^3 33/36/30
 //                       80^3 9.6/-/12          160^3 59/51/54      8x128x128 5.7/-/11        16x256x256 17/-/30
 //                 FP32  32^3 6.7/-/6.4         64^3 7.4/9.4/7.9    128^3 20/19/22            112^3 15/-/20
-// On the smallest levels every form is bound by its launches.  Bricks make
-// half as many there as the colour passes: one solve takes as long (visc_type
-// 2, -2, -3 32^3 within 5 %), sixteen on the four hardware queues 1 to 6 % less.
+// On small levels every form is bound by its launches, and in a V-cycle bricks
+// gain what the table does not show: half as many launches, and no fill with
+// zeros before the first sweep of the three components and of the
+// cell-centred field.  So the lines are drawn by whole solves (the contexts'
+// runs in turn, medians in ms, bricks / colour passes in the part named):
+//   three components, bricks of 8 rows  FP64  20x128x128 (512 bricks) 30.6 / 34.1, 40x96x96 (576)
+//                     11.0 / 11.4, 12x160x160 (800) 51.2 / 50.1, 16x192x192 (1152) 15.2 / 14.3
+//                     FP32  8x128x128 (512) 6.2 / 7.5, 20x160x160 (800) 29.0 / 31.0, 8x192x192 (1152)
+//                     20.5 / 21.4, 8x256x256 (2048) with the cell-centred field 38.1 / 32.9
+//   one, of 4 rows    visc_type 2 FP64  32^3 (64) 4.22 / 4.19, 64^3 (512) 4.88 / 4.87, 96x48x64 (576)
+//                     7.15 / 7.33, 128x64x64 (1024) 6.60 / 6.39, 48^3 (288, 75 % full) 4.10 / 3.89
+//                     visc_type -2 FP64  64x32x64 (256) 4.74 / 4.60, 64^3 6.12 / 5.96, 96x48x64 8.26 / 7.71
+//                     FP32  64^3 3.85 / 3.78, 96x48x64 5.49 / 5.57, inertial step 64^3 7.10 / 7.29
+//   cell-centred      FP64  80x16x104 (312) 6.02 / 6.20, 36x72x72 (648) 13.5 / 13.7, 80^3 (1200) 5.54 /
+//                     5.50, 48x112x112 (1568) 7.53 / 7.26, 8x256x256 (4096) 65.0 / 60.7
+// Sixteen solves on the four hardware queues take 1 to 6 % less with bricks
+// on levels of at most 128.
 static bool brick_pays(const Grid &g, SweepUse use, int visc, int es, bool marches) {
   if (tuning().rb_brick > 0) return g.N <= tuning().rb_brick;
   const long n4 = bricks(g, 4).n;
   const double fill = (double)g.N / (n4 * (KX * 4 * KZ));
   if (use == SWEEP_THREE)
-    return bricks(g, 8).n <= (es == 8 ? 400 : 700) || (fill >= 0.7 && (!marches || g.N <= 1200000));
-  if (n4 <= 128) return true;
-  if (use == SWEEP_ONE) return visc >= -1 && n4 <= 512 && fill >= 0.85;
+    return bricks(g, 8).n <= (es == 8 ? 600 : 1200) || (fill >= 0.7 && (!marches || g.N <= 1200000));
+  if (use == SWEEP_ONE) return n4 <= 128 || ((visc >= -1 || es == 4) && n4 <= 640 && fill >= 0.85);
+  if (n4 <= 700) return true;
   return fill >= 0.85 && (g.N <= (es == 8 ? 3000000 : 1200000) || (es == 8 && !marches));
 }
 // Whether the one-component sweep of a level too large for bricks marches; the

@@ -22,18 +22,25 @@ CASES = [
     ((32, 32, 32), -1, "fp64", "brick4", "brick4"),
     ((64, 64, 64), -1, "fp64", "brick8", "brick4"),
     ((64, 64, 64), -1, "fp32", "brick8", "brick4"),
-    ((16, 64, 64), 1, "fp64", "brick4", None),       # thin, but few bricks; cell-centred: half of each in the box
-    ((8, 128, 128), -1, "fp64", None, None),         # a quarter of each brick lies in the box
-    ((8, 128, 128), -1, "fp32", "brick8", None),
+    ((16, 64, 64), 1, "fp64", "brick4", "brick4"),   # thin, but few bricks
+    ((8, 128, 128), -1, "fp64", "brick8", None),     # a quarter of each brick lies in the box; 512 of 8 rows
+    ((8, 128, 176), -1, "fp64", None, None),         # 704
+    ((8, 128, 176), -1, "fp32", "brick8", None),
+    ((8, 128, 304), -1, "fp32", None, None),         # 1216
     ((128, 12, 128), -1, "fp32", "brick4", "brick4"),  # 8 rows would hang over by a third
     ((32, 32, 32), -2, "fp64", "brick4", "brick4"),  # launch-bound
     ((32, 32, 32), -3, "fp32", "brick4", "brick4"),
     ((64, 32, 32), 2, "fp64", "brick4", "brick4"),
     ((64, 64, 64), 3, "fp64", "brick4", "brick4"),
     ((64, 64, 64), -2, "fp64", None, "brick4"),      # one component, variable coefficients
-    ((64, 64, 64), -3, "fp32", None, "brick4"),
-    ((48, 48, 48), 2, "fp64", None, None),           # three quarters full
-    ((96, 64, 64), 2, "fp32", None, "brick4"),       # more than 512 bricks a component
+    ((64, 64, 64), -3, "fp32", "brick4", "brick4"),
+    ((96, 64, 64), -3, "fp32", None, "brick4"),      # more than 640 bricks
+    ((48, 48, 48), 2, "fp64", None, "brick4"),       # three quarters full
+    ((36, 72, 72), 1, "fp64", "brick8", "brick4"),   # 648 bricks, half full
+    ((40, 72, 80), 1, "fp64", "brick8", None),       # 720 bricks; 8 rows: 360 for each of three components
+    ((96, 64, 64), 2, "fp32", None, "brick4"),
+    ((80, 64, 52), 2, "fp64", None, "brick4"),       # 624 bricks, 83 % full
+    ((96, 48, 64), 3, "fp64", "brick4", "brick4"),   # 576, full
 ]
 
 
