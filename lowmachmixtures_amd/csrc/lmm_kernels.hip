@@ -1488,7 +1488,7 @@ void launch_sub_means(hipStream_t s, const Grid &g, T *const x[3], int nc, const
 }
 
 // x -= its mean, from the nsrc sums of 256 cells each that k_precon_final
-// left in src; work holds RED_BLOCKS * 4.  Up to RED_BLOCKS sums are read by
+// left in src; work holds RED_BLOCKS doubles.  Up to RED_BLOCKS sums are read by
 // the subtracting pass as they are, more are folded to RED_BLOCKS first.
 template <typename T>
 void launch_sub_cell_mean(hipStream_t s, const Grid &g, T *x, const double *src, int nsrc, double *work) {
