@@ -665,7 +665,7 @@ inline Bricks bricks(const Grid &g, int ky) {
 // 64^3 FP64 15.8 / 14.0, 128 x 96 x 64 FP64 38.4 / 34.6, 256 x 12 x 256 FP64
 // 37.2 / 43.2; cell-centred 64^3 FP64 8.2 / 9.1, 128 x 96 x 64 FP64 15.1 /
 // 13.4, 256 x 12 x 256 FP64 15.1 / 18.0.  The one-component staggered form takes
-// levels of at most 512 bricks (brick_pays) and has 4 rows.
+// levels of at most 640 bricks (brick_pays) and has 4 rows.
 inline int brick_rows(const Grid &g, int ncomp) {
   const int rows = tuning().rb_brick_rows;
   if (rows == 4 || rows == 8) return rows;
@@ -1431,7 +1431,7 @@ static bool brick_ok(const Grid &g, int min_tiles, int ncomp) {
 //                     11.0 / 11.4, 12x160x160 (800) 51.2 / 50.1, 16x192x192 (1152) 15.2 / 14.3
 //                     FP32  8x128x128 (512) 6.2 / 7.5, 20x160x160 (800) 29.0 / 31.0, 8x192x192 (1152)
 //                     20.5 / 21.4, 8x256x256 (2048) with the cell-centred field 38.1 / 32.9
-//   one, of 4 rows    visc_type 2 FP64  32^3 (64) 4.22 / 4.19, 64^3 (512) 4.88 / 4.87, 96x48x64 (576)
+//   one, of 4 rows    visc_type 2 FP64  32^3 (64) 4.22 / 4.19, 64^3 (512) 6.77 / 6.73, 96x48x64 (576)
 //                     7.15 / 7.33, 128x64x64 (1024) 6.60 / 6.39, 48^3 (288, 75 % full) 4.10 / 3.89
 //                     visc_type -2 FP64  64x32x64 (256) 4.74 / 4.60, 64^3 6.12 / 5.96, 96x48x64 8.26 / 7.71
 //                     FP32  64^3 3.85 / 3.78, 96x48x64 5.49 / 5.57, inertial step 64^3 7.10 / 7.29
